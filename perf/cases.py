@@ -72,10 +72,9 @@ def draw(rng):
     return {"op": op, "dtype": dtype, "M": M, "d": d, "ff": ff}
 
 
-def prepare(case, seed):
+def _tensors(case, seed):
     """Activations ~ N(0, 1) (half of that in fp16, whose range is short), weights ~ N(0, 1) / sqrt(fan_in): values of a
     trained layer's size. H of the down projection alone has the spread that a gated product of such values has."""
-    import fused_mlp_module
     M, d, ff, dtype = case["M"], case["d"], case["ff"], DTYPES[case["dtype"]]
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(seed)
@@ -85,20 +84,19 @@ def prepare(case, seed):
         t = torch.empty((rows, cols), dtype=dtype, device=dev)
         return t.normal_(0.0, scale, generator=g)
 
-    op = case["op"]
-    if op == "down":
-        fn = getattr(fused_mlp_module, "swiglu_down_" + case["dtype"])
+    if case["op"] == "down":
         up, gate = normal(M, ff, x_scale), normal(M, ff, x_scale)
-        return {"fn": fn, "args": (up * torch.nn.functional.silu(gate), normal(d, ff, ff ** -0.5))}
+        return up * torch.nn.functional.silu(gate), normal(d, ff, ff ** -0.5)
     args = (normal(M, d, x_scale), normal(2 * ff, d, d ** -0.5))
-    if op == "mlp":
-        fn = getattr(fused_mlp_module, "fused_swiglu_mlp_" + case["dtype"])
-        args += (normal(d, ff, ff ** -0.5),)
-    elif op == "gateup_f32":
-        fn = fused_mlp_module.fused_swiglu_bf16_f32out
-    else:
-        fn = getattr(fused_mlp_module, "fused_swiglu_" + case["dtype"])
-    return {"fn": fn, "args": args}
+    return args + (normal(d, ff, ff ** -0.5),) if case["op"] == "mlp" else args
+
+
+def prepare(case, seed):
+    """The activations and the weights, as a layer of the program holds them, and the entry point it calls."""
+    import fused_mlp_module
+    name = {"mlp": "fused_swiglu_mlp_" + case["dtype"], "gateup": "fused_swiglu_" + case["dtype"],
+            "gateup_f32": "fused_swiglu_bf16_f32out", "down": "swiglu_down_" + case["dtype"]}[case["op"]]
+    return {"fn": getattr(fused_mlp_module, name), "args": _tensors(case, seed)}
 
 
 def run(state):
@@ -125,3 +123,14 @@ def tolerance(case):
     if case["op"] == "mlp":
         return {"rel": 1e-2, "max": 4e-2} if case["dtype"] == "bf16" else {"rel": 1.2e-3, "max": 5e-3}
     return {"rel": 7e-3, "max": 1.6e-2} if case["dtype"] == "bf16" else {"rel": 8e-4, "max": 2e-3}
+
+
+def exact(case, seed):
+    """The formulas in float64: rows 2j of W1W3 are the up operand, rows 2j + 1 the gate."""
+    args = [t.double() for t in _tensors(case, seed)]
+    if case["op"] == "down":
+        return args[0] @ args[1].t()
+    pre = args[0] @ args[1].t()
+    up, gate = pre[:, 0::2], pre[:, 1::2]
+    h = up * (gate / (1.0 + torch.exp(-gate)))
+    return h @ args[2].t() if case["op"] == "mlp" else h
