@@ -240,14 +240,15 @@ tiled_dma_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const i
   // back-to-back forwards 110 -> 106 us.
   // DMA of K tile `kt` into `stage`: wave-uniform LDS base per instruction, loop-invariant per-lane offset in a
   // VGPR, the K offset in an SGPR. Rows beyond the matrix are out of range for the buffer descriptor and arrive
-  // as zeros. A prefetch past the last tile re-reads the last tile (never consumed). Only when K is not a
-  // multiple of 64 (KTAIL) do lanes whose chunk lies at or beyond K redirect their offset out of range.
+  // as zeros. A prefetch past the last tile is out of range as a whole: no memory traffic (with three stages and
+  // a dozen K tiles a re-read of the last tile would be a sixth of it all), never consumed. When K is not a multiple of
+  // 64 (KTAIL) lanes whose chunk lies at or beyond K redirect their offset out of range as well.
   auto dma = [&](unsigned char* stage, int kt) {
-    int ktr = (kt < nkt ? kt : nkt - 1) + rot;
+    int ktr = kt + rot;
     if (ktr >= nkt) ktr -= nkt;
     const int ktc = kt0 + ktr;
-    const int kb = ktc * (BK * 2);
-    const bool in = !KTAIL || (ktc * BK + lc * 8) < a.k;
+    const int kb = kt < nkt ? ktc * (BK * 2) : 0;
+    const bool in = kt < nkt && (!KTAIL || (ktc * BK + lc * 8) < a.k);
 #pragma unroll
     for (int i = 0; i < LP; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(prs, (lds_void*)(stage + i * RSTEP * ROWB + wave * 1024), 16,
@@ -320,11 +321,10 @@ tiled_dma_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const i
     }
   };
 
-  // NS stages: two for the compute-bound uses; three when every weight byte comes from HBM exactly once (a single
-  // tile of activation rows, weights streamed non-temporally): the copy of tile kt + 2 is issued while tile kt is
-  // multiplied, which doubles the bytes in flight per workgroup. Measured at 4096 x 28672, gate/up: M = 65: 67.6 ->
-  // 43.9 us, M = 128: 67.0 -> 49.0 us (a fourth stage: level). The split-K down projection keeps two stages (three
-  // cost it an LDS-limited workgroup per CU: 36.7 -> 40.4 us).
+  // NS stages: two where two workgroups share a compute unit; three or four where a workgroup has it to itself (see
+  // launch_dma_kernel): the copy of tile kt + NS - 1 is issued while tile kt is multiplied, which multiplies the
+  // bytes in flight per workgroup. Measured at 4096 x 28672, gate/up, two -> three: M = 65: 67.6 -> 43.9 us, M = 128:
+  // 67.0 -> 49.0 us (a fourth stage: level).
   if constexpr (NS == 2) {
     if (nkt > 0) dma(lds0, 0);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -456,24 +456,35 @@ int raster_group(bool gated, int tiles_q) { return gated ? 4 : (tiles_q >= 32 ? 
 
 namespace {
 
-// the 128-row instances stream their weights non-temporally when at most two tiles of activation rows share them
+// The 128-row instances stream their weights non-temporally when at most two tiles of activation rows share them.
+// Ring length: a launch of at most 256 workgroups has a compute unit to itself per workgroup, so nothing else hides
+// the latency of its copies and the LDS is free: three stages (four of the small 128 x 64 ones), copies two (three) K
+// tiles ahead. Two stages -> three, us: gate/up fp16 3000 x 16016 at 200 rows (252 workgroups) 68 -> 57, whole forward
+// 92.1 -> 82.9; forward 512 rows of 1024 x 2816 29.8 -> 24.2; gate/up 250 rows of 1024 x 5632 17.7 -> 12.9; a fourth and
+// fifth stage of 32 KB: level. 128 x 64, three -> four stages: gate/up 64 rows of 4096 x 22016 34.3 -> 32.2.
+// More workgroups than compute units keep two stages and two workgroups per compute unit (8192 x 57344 at 65 rows,
+// 448 workgroups: 168 us with three stages, 158 with two), except the wide tiles, whose stages leave no room for a second
+// workgroup anyway.
 template <class E, bool GATED, bool KTAIL, int WP, int WQ, int FP, int FQ>
 void launch_dma_kernel(const dim3 grid, hipStream_t stream, const GemmArgs& a, int tiles_p, int tiles_q, int group) {
-  // a single tile of activation rows: three stages (see NS). They leave room for one workgroup per compute unit,
-  // so 128 x 128 launches of more than 256 workgroups keep two stages and two workgroups (8192 x 57344 at 65 rows,
-  // 448 workgroups: 168 -> 158 us)
-  if (tiles_q == 1 && (WQ * FQ >= 6 || (long long)grid.x * grid.y <= 256)) {
-    hipLaunchKernelGGL((tiled_dma_kernel<E, GATED, KTAIL, WP, WQ, FP, FQ, true, 3>), grid, dim3(WP * WQ * 64), 0, stream,
-                       a, tiles_p, tiles_q, group);
-    return;
-  }
+  constexpr int DEEP = WQ * FQ == 2 ? 4 : 3;
+  const dim3 block(WP * WQ * 64);
+  const bool deep = (long long)grid.x * grid.y <= 256 || (WQ * FQ >= 6 && tiles_q == 1);
   if (tiles_q <= 2) {
-    hipLaunchKernelGGL((tiled_dma_kernel<E, GATED, KTAIL, WP, WQ, FP, FQ, true>), grid, dim3(WP * WQ * 64), 0, stream,
-                       a, tiles_p, tiles_q, group);
-    return;
+    if (deep) {
+      hipLaunchKernelGGL((tiled_dma_kernel<E, GATED, KTAIL, WP, WQ, FP, FQ, true, DEEP>), grid, block, 0, stream, a,
+                         tiles_p, tiles_q, group);
+    } else {
+      hipLaunchKernelGGL((tiled_dma_kernel<E, GATED, KTAIL, WP, WQ, FP, FQ, true>), grid, block, 0, stream, a, tiles_p,
+                         tiles_q, group);
+    }
+  } else if (deep) {
+    hipLaunchKernelGGL((tiled_dma_kernel<E, GATED, KTAIL, WP, WQ, FP, FQ, false, DEEP>), grid, block, 0, stream, a, tiles_p,
+                       tiles_q, group);
+  } else {
+    hipLaunchKernelGGL((tiled_dma_kernel<E, GATED, KTAIL, WP, WQ, FP, FQ>), grid, block, 0, stream, a, tiles_p, tiles_q,
+                       group);
   }
-  hipLaunchKernelGGL((tiled_dma_kernel<E, GATED, KTAIL, WP, WQ, FP, FQ>), grid, dim3(WP * WQ * 64), 0, stream, a, tiles_p,
-                     tiles_q, group);
 }
 
 template <class E, bool GATED, int WP, int WQ, int FP, int FQ>

@@ -627,6 +627,24 @@ def test_pieces_zero_the_ticket_counters_of_the_down_projection_too(capi):
         assert torch.equal(capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws), Y)
 
 
+@pytest.mark.parametrize("M", [40, 200, 300])
+@pytest.mark.parametrize("K", [8, 64, 72, 128, 192, 200, 256, 320, 328])
+def test_stage_ring_with_few_k_tiles(capi, M, K):
+    """The three- and four-stage rings of the 128-row tiles (launches of at most 256 workgroups: one, two and three tiles
+    of activation rows) with fewer K tiles than stages, as many, one more, and a K tail: copies issued past the last
+    tile bring nothing in."""
+    inp = fsw_weights.make_inputs(M, K, 8 * K, torch.bfloat16, seed=41 * K + M)
+    g = to_dev(inp)
+    try:
+        capi.set_variant(0, 4 if M <= 64 else 0)
+        H = capi.gateup(g["X"], g["W13"])
+    finally:
+        capi.set_variant(0, -1)
+    assert_one_rounding(H, oracle.ref_gateup(inp["X"], inp["W13"], torch.float64), torch.bfloat16, "H %s" % ((M, K),))
+    Y = capi.down(H, g["W2"])
+    assert_one_rounding(Y, oracle.ref_down(H.cpu(), inp["W2"], torch.float64), torch.bfloat16, "Y %s" % ((M, K),))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 16, 64, 65, 300, 1024])
 def test_float32_output_is_the_unrounded_gated_value(capi, M, dtype):
