@@ -312,8 +312,13 @@ int fsw_gateup(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int64_
 }
 
 // The reference's other build (C_TYPE float, constants.cuh:9-14; "C can work with either bf16 or fp32",
-// swiglu.cu:470-471): H is float and receives the gated fp32 value without a rounding. Two kernels serve it: the
-// weight-streaming kernel up to 64 rows, the 256 x 256 kernel on row-major operands above.
+// swiglu.cu:470-471): H is float and receives the gated fp32 value without a rounding. From 2^21 gated weight pairs on
+// (a layer of 1024 x 2816 has 2.9 million) it runs the kernel that the 16-bit output would run, whose tiles fit
+// the rows and the compute units (the persistent decode kernel has no float store: skinny_kernel there); smaller layers
+// run the weight-streaming kernel up to 64 rows and the 256 x 256 kernel above, so that rounding their result gives the
+// 16-bit output of those kernels bit for bit. Measured against those two kernels, us: 4096 x 11008:
+// 40 rows 38.4 -> 31.6, 65 rows 64.6 -> 41.0, 130 rows 66.0 -> 50.1, 200 rows 66.6 -> 55.7; 1024 x 2816: 16 rows level,
+// 65 rows 21.0 -> 10.1, 300 rows 23.5 -> 10.9, 1000 rows 25.3 -> 18.5; 8192 x 28672: 40 rows 189 -> 150.
 int fsw_gateup_f32out(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* W13,
                       int64_t ldw, float* H, int64_t ldh, void* stream) {
   const int rc = fsw_validate_gateup(dtype, M, N, K, X, ldx, W13, ldw, H, ldh);
@@ -333,8 +338,11 @@ int fsw_gateup_f32out(int dtype, int64_t M, int64_t N, int64_t K, const void* X,
   a.nq = (int)M;
   a.k = (int)K;
   a.out_f32 = 1;
-  if (M <= 64) return finish(fsw::launch_skinny(dtype, true, a, nullptr, (hipStream_t)stream));
-  return finish(fsw::launch_pair16(dtype, true, a, (hipStream_t)stream));
+  int v = M <= 64 ? VARIANT_SKINNY : V_256x256;
+  if ((N / 2) * K >= (int64_t)1 << 21) v = resolve_variant(0, M, N, K);
+  a.tile_p = stream_tile_rows(v, M, N);
+  if (v == VARIANT_SKINNY) return finish(fsw::launch_skinny(dtype, true, a, nullptr, (hipStream_t)stream));
+  return finish(fsw::launch_tiled(v, dtype, true, a, (hipStream_t)stream));
 }
 
 // Inside fsw_mlp the down projection of up to 32 activation rows runs the split-K streaming kernel when (i) the

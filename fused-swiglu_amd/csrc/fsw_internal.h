@@ -28,7 +28,7 @@ struct GemmArgs {
   // skinny_kernel honour it): the ticket counters of the split-K streaming down projection that follows in fsw_mlp
   unsigned* zero_words = nullptr;
   int n_zero_words = 0;
-  // gated kernels on row-major operands (skinny_kernel, the 256 x 256 kernel with layout 0): O is float [nq, np/2]
+  // gated kernels on row-major operands (skinny_kernel, tiled_dma_kernel, the 256 x 256 kernel with layout 0): O is float [nq, np/2]
   // and receives the gated fp32 value unrounded (the reference's build with C_TYPE float, constants.cuh:9)
   int out_f32 = 0;
   // tiled_dma_kernel with one tile of activation rows: weight rows a workgroup owns when that is fewer than the

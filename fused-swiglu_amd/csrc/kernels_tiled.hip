@@ -23,13 +23,14 @@ namespace fsw {
 // Epilogue shared by the tiled kernels. A lane owns activation row m = l32 of each Q fragment and, per group
 // of 4 accumulator registers, 4 consecutive output features: feature = 8 * (i / 4) + 4 * hi + (i % 4) within
 // the fragment. Gating (fp32 multiply and SiLU, swiglu.cu:380-381) happens here, then ONE rounding and an
-// 8-byte store.
+// 8-byte store (GemmArgs::out_f32: no rounding and a 16-byte store).
 template <class E, bool GATED, int WP, int WQ, int FP, int FQ>
 __device__ __forceinline__ void store_tile(f32x16 (&acc)[FP][FQ], const GemmArgs& a, int p0, int q0, int wp, int wq,
                                            int l32, int hi, int p_end) {
   unsigned short* O = (unsigned short*)a.O;
   const int nout = GATED ? p_end / 2 : p_end;  // p_end: first weight row this workgroup does not own
   const bool vec_ok = ((a.ldo & 3) == 0) && ((((uintptr_t)a.O) & 7) == 0);
+  const bool vec32_ok = ((a.ldo & 3) == 0) && ((((uintptr_t)a.O) & 15) == 0);
   constexpr int FO = GATED ? FP / 2 : FP;
 #pragma unroll
   for (int g = 0; g < FQ; ++g) {
@@ -51,7 +52,16 @@ __device__ __forceinline__ void store_tile(f32x16 (&acc)[FP][FQ], const GemmArgs
           }
         }
         const int n = nb + i4 * 8;
-        if (vec_ok && n + 3 < nout) {
+        if (GATED && a.out_f32) {
+          float* o32 = (float*)a.O + (long long)m * a.ldo + n;
+          if (vec32_ok && n + 3 < nout) {
+            *(f32x4*)o32 = f32x4{v[0], v[1], v[2], v[3]};
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < nout) o32[e] = v[e];
+          }
+        } else if (vec_ok && n + 3 < nout) {
           u32x2 pk = {E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
           *(u32x2*)(orow + n) = pk;
         } else {

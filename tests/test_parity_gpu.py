@@ -674,6 +674,24 @@ def test_float32_output_is_the_unrounded_gated_value(capi, M, dtype):
     assert torch.equal(wide[:, :ff], capi.gateup_f32out(g["X"], g["W13"])) and torch.isnan(wide[:, ff:]).all()
 
 
+@pytest.mark.parametrize("M,d,ff", [(17, 1024, 2056), (49, 1024, 2056), (49, 264, 8200), (64, 264, 8200), (65, 1024, 2056),
+                                    (128, 264, 8200), (130, 264, 8200), (193, 264, 8200), (256, 264, 8204), (257, 1024, 2052)])
+def test_float32_output_of_larger_layers(capi, M, d, ff):
+    """From 2^21 gated weight pairs on the float32 output comes from the kernel the 16-bit output uses (128 x 64, pieces,
+    128 x 128, 128 x 192, 128 x 256 on 8 waves): rounding it gives that output bit for bit. ff = 8204 and 2052 end in a
+    partial group of 8 features; the second output has an odd row stride (scalar stores)."""
+    assert d * ff >= 1 << 21
+    inp = fsw_weights.make_inputs(M, d, ff, torch.bfloat16, seed=M + ff, x_scale=0.5)
+    g = to_dev(inp)
+    H32 = capi.gateup_f32out(g["X"], g["W13"])
+    ref = oracle.ref_gateup(inp["X"], inp["W13"], torch.float64)
+    assert not ((H32.cpu().double() - ref).abs() > 1e-5 * (1.0 + ref.abs())).any()
+    assert torch.equal(capi.gateup(g["X"], g["W13"]), H32.to(torch.bfloat16))
+    wide = torch.full((M, ff + 5), float("nan"), dtype=torch.float32, device=DEV)
+    capi.gateup_f32out(g["X"], g["W13"], out=wide[:, :ff])
+    assert torch.equal(wide[:, :ff], H32) and torch.isnan(wide[:, ff:]).all()
+
+
 def test_float32_output_through_the_operators(ext):
     """fused_swiglu_bf16_f32out, and swiglu_fwd_bf16 with a float C (the reference's operator compiled with C_TYPE
     float): the ldC / 2 rule holds in elements of C's type (swiglu.cu:414); wrong C types still raise."""
