@@ -22,6 +22,8 @@ constexpr int VARIANT_DECODE_STREAM = 102;   // M <= 16: the streaming kernel of
 constexpr int VARIANT_DECODE_FUSED = 101;    // fsw_mlp only: single-launch decode forward (family 0)
 constexpr int VARIANT_DECODE_FUSED_FAIL = 103;  // 101 with a device-wide barrier that cannot complete (failure-path test)
 constexpr int VARIANT_STREAM_SPLIT = 104;    // family 1, fsw_mlp only: split-K streaming down projection for M <= 32
+// the 256 x 256 kernel with narrower tiles: VARIANT_NARROW + 5, 6, 7 = 160, 192, 224 activation rows per tile
+constexpr int VARIANT_NARROW = 110;
 constexpr int64_t MAX_DIM = 1LL << 30;       // every size is cast to int inside the kernels
 constexpr int64_t MAX_LD = 1LL << 21;        // keeps tile-relative byte offsets below 2^31
 
@@ -56,7 +58,8 @@ constexpr int V_128x128 = 0, V_128x192 = 2, V_8W_128x256 = 3, V_128x64 = 4, V_25
 
 // Variant choice for the tiled kernels: the widest tile whose activation-row extent is not mostly padding,
 // stepping down to 128x128 when a 256-wide grid would leave most of the 256 CUs idle.
-int pick_tiled(int family, int64_t m, int64_t np) {
+// `narrow_need`: a narrower large tile is taken only if its estimated time is below this share of 256 x 256's
+int pick_tiled(int family, int64_t m, int64_t np, double narrow_need = 0.95) {
   const int64_t tiles256 = ((np + 255) / 256) * ((m + 255) / 256);
   // 256 x 256 tiles down to half-filled compute units. Below that the down product splits K (see
   // tiled_split_plan); between 129 and 191 tiles one large tile per compute unit beats 128 x 128 tiles in
@@ -78,6 +81,9 @@ int pick_tiled(int family, int64_t m, int64_t np) {
     // up to 64 rows the gate/up tile is 128 x 64 (4096 x 28672, M = 48: 39.4 -> 37.2 us)
     return (family == 0 && m <= 64) ? V_128x64 : V_128x128;
   }
+  // (the down projection of a multiple of 256 rows keeps the kernel it always had there)
+  const int rows = family == 1 && m % 256 == 0 ? 256 : fsw::pair16_tile_rows(family == 0, np, m, narrow_need);
+  if (rows != 256) return VARIANT_NARROW + rows / 32;
   if (family == 0 && tiles256 > 256 && tiles256 <= 512) {
     // A few large tiles more than compute units: the second round is nearly empty, while 128 x 128 tiles (two per
     // compute unit, ~1.3-1.7 x the time per output element) come in rounds a quarter as long. Per round of 256
@@ -159,6 +165,14 @@ int finish(hipError_t e) {
   return FSW_OK;
 }
 
+bool narrow_variant(int v) { return v >= VARIANT_NARROW + 5 && v <= VARIANT_NARROW + 7; }
+
+hipError_t launch_tiled_variant(int v, int dtype, bool gated, fsw::GemmArgs& a, hipStream_t stream) {
+  if (!narrow_variant(v)) return fsw::launch_tiled(v, dtype, gated, a, stream);
+  a.tile_q = 32 * (v - VARIANT_NARROW);
+  return fsw::launch_tiled(V_256x256, dtype, gated, a, stream);
+}
+
 }  // namespace
 
 extern "C" {
@@ -203,7 +217,7 @@ int fsw_set_variant(int family, int variant) {
   if (variant >= 0 && variant != VARIANT_SKINNY && variant != VARIANT_DECODE_STREAM &&
       !(family == 0 && (variant == VARIANT_DECODE_FUSED || variant == VARIANT_DECODE_FUSED_FAIL)) &&
       !(family == 1 && variant == VARIANT_STREAM_SPLIT) &&
-      variant >= fsw::tiled_variant_count())
+      !narrow_variant(variant) && variant >= fsw::tiled_variant_count())
     return FSW_E_VARIANT;
   g_forced_variant[family] = variant < 0 ? -1 : variant;
   return FSW_OK;
@@ -227,8 +241,15 @@ const char* fsw_variant_name(int family, int dtype, int64_t M, int64_t N_or_D, i
       if (plan.tile == 128) return "splitk_dma_128x128";
       if (plan.tile == 129) return "splitk_dma_128x256";
       if (plan.tile == 130) return "splitk_dma_128x192";
+      if (plan.tile == 160) return "splitk_pair16_256x160";
+      if (plan.tile == 192) return "splitk_pair16_256x192";
+      if (plan.tile == 224) return "splitk_pair16_256x224";
       return "splitk_pair16_256x256";
     }
+  }
+  if (narrow_variant(v)) {
+    static const char* const names[3] = {"pair16_256x160", "pair16_256x192", "pair16_256x224"};
+    return names[v - VARIANT_NARROW - 5];
   }
   return fsw::tiled_variant(v).name;
 }
@@ -303,7 +324,7 @@ static int gateup_impl(int dtype, int64_t M, int64_t N, int64_t K, const void* X
     }
     return finish(fsw::launch_skinny(dtype, true, a, nullptr, (hipStream_t)stream));
   }
-  return finish(fsw::launch_tiled(v, dtype, true, a, (hipStream_t)stream));
+  return finish(launch_tiled_variant(v, dtype, true, a, (hipStream_t)stream));
 }
 
 int fsw_gateup(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* W13, int64_t ldw,
@@ -342,7 +363,7 @@ int fsw_gateup_f32out(int dtype, int64_t M, int64_t N, int64_t K, const void* X,
   if ((N / 2) * K >= (int64_t)1 << 21) v = resolve_variant(0, M, N, K);
   a.tile_p = stream_tile_rows(v, M, N);
   if (v == VARIANT_SKINNY) return finish(fsw::launch_skinny(dtype, true, a, nullptr, (hipStream_t)stream));
-  return finish(fsw::launch_tiled(v, dtype, true, a, (hipStream_t)stream));
+  return finish(launch_tiled_variant(v, dtype, true, a, (hipStream_t)stream));
 }
 
 // Inside fsw_mlp the down projection of up to 32 activation rows runs the split-K streaming kernel when (i) the
@@ -418,7 +439,7 @@ int fsw_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H, int64_t
     a.partial = (float*)workspace;
     return finish(fsw::launch_tiled_splitk(dtype, plan.tile, a, (hipStream_t)stream));
   }
-  return finish(fsw::launch_tiled(v, dtype, false, a, (hipStream_t)stream));
+  return finish(launch_tiled_variant(v, dtype, false, a, (hipStream_t)stream));
 }
 
 // Large-tile regime of fsw_mlp: both projections run 256 x 256 tiles, and H never exists row-major: the gate/up
@@ -427,7 +448,9 @@ int fsw_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H, int64_t
 static bool blocked_regime(int64_t M, int64_t D, int64_t FF) {
   if (M <= 64 || D <= 0 || FF <= 0 || g_forced_variant[0] >= 0 || g_forced_variant[1] >= 0) return false;
   if (M > MAX_DIM || D > MAX_DIM || FF > MAX_DIM / 2) return false;
-  return pick_tiled(0, M, 2 * FF) == V_256x256 && pick_tiled(1, M, D) == V_256x256 &&
+  // a down projection on narrower tiles reads row-major H; it has to gain more than H blocked does (3000 rows of 4096 x
+  // 11008: 7 % of the down kernel, a third of the forward, is not enough; 2500 rows: 11 %)
+  return pick_tiled(0, M, 2 * FF) == V_256x256 && pick_tiled(1, M, D, 0.9) == V_256x256 &&
          fsw::tiled_split_plan((int)D, (int)M, (int)FF).splits == 1;  // a split-K down projection reads row-major H
 }
 

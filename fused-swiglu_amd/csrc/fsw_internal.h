@@ -36,6 +36,8 @@ struct GemmArgs {
   // of range for its copies (zeros, no traffic) and are not stored: lets a weight stream be cut into exactly as
   // many pieces as there are compute units. A multiple of 8 (whole 8-byte stores of the gated output).
   int tile_p = 0;
+  // launch_pair16 with layout 0 and launch_pair16_splitk: activation rows per tile, 256 or one of 224, 192, 160
+  int tile_q = 256;
 };
 inline long long blocked_bytes(long long rows, long long k) {
   return ((rows + 255) / 256) * ((k + 31) / 32) * (256 * 64);
@@ -65,10 +67,14 @@ hipError_t launch_block_rows(const void* src, long long ld, int rows, int k, voi
 // tile (128 or 256 square) and how many K partitions, so that about two workgroups per CU are in flight.
 // splits == 1 means the ordinary launch path.
 struct SplitPlan {
-  int tile;    // 128 or 256 (square), 129 = 128 output features x 256 activation rows, 130 = 128 x 192
+  int tile;    // 128 (square), 129 = 128 output features x 256 activation rows, 130 = 128 x 192, else 256 x tile
+               // (256, 224, 192 or 160 activation rows)
   int splits;  // K partitions
 };
 SplitPlan tiled_split_plan(int np, int nq, int k);
+// activation rows per tile (256, 224, 192, 160) of the 256-weight-row kernel on row-major operands; a narrow one is
+// returned only if its estimated time is below `need` times that of 256
+int pair16_tile_rows(bool gated, long long np, long long nq, double need);
 hipError_t launch_tiled_splitk(int dtype, int tile, const GemmArgs& a, hipStream_t stream);  // a.splits, a.partial set
 
 // Weight-streaming kernels for M <= 16 activation rows (kernels_skinny.hip).

@@ -44,11 +44,16 @@ typedef __attribute__((address_space(3))) void lds_void;
 // SPLIT (row-major operands, plain product): blockIdx.y selects one of a.splits contiguous runs of 64-element K
 // pairs; the workgroup multiplies that run only and stores its fp32 accumulators to a.partial[blockIdx.y][nq][np].
 // OF32 (gated, row-major operands and output): H is float and receives the gated value unrounded.
+// NQ (row-major operands): 16-row activation blocks per wave, i.e. a tile of 256 weight rows x 32 NQ activation rows.
+// Everything about the schedule stays (a pair has 16 NQ MFMAs per wave instead of 128, NQ activation copies instead
+// of 8); the K order of every output is the same for all NQ, so results are bit-identical. For row counts that
+// 256-row tiles would fill badly, see pair16_tile_rows().
 template <class E, bool GATED, bool KTAIL, bool OBLK, bool PBLK = false, bool QROW = false, bool SPLIT = false,
-          bool OF32 = false>
+          bool OF32 = false, int NQ = 8>
 __global__ void __launch_bounds__(256)
 tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, const int group) {
   static_assert(!SPLIT || (QROW && !GATED && !OBLK && !PBLK), "split-K: row-major operands, plain product");
+  static_assert(NQ == 8 || (QROW && !OBLK && !PBLK && NQ >= 4 && NQ < 8), "narrow tiles: row-major operands and output");
   static_assert(!OF32 || (GATED && QROW && !OBLK && !PBLK), "fp32 output: the gated kernel on row-major operands");
   GemmArgs a = a_in;
   if constexpr (SPLIT) {  // the run of this workgroup as a product of its own: shifted operands, shorter K
@@ -60,9 +65,9 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
     a.Q = (const unsigned short*)a_in.Q + k0;
   }
   constexpr int WP = 2, WQ = 2;
-  constexpr int NB = 8;  // 16-row blocks per wave and operand
-  constexpr int BP = 256, BQ = 256;
-  constexpr int PSLOT = BP * 128, QSTAGE = BQ * 64;
+  constexpr int NB = 8;  // 16-row weight blocks per wave (NQ activation blocks)
+  constexpr int BP = 256, BQ = 32 * NQ;
+  constexpr int PSLOT = BP * 128, QSLOT = BQ * 128, QSTAGE = BQ * 64;
   constexpr int LPH = 4;  // weight copy instructions per wave per HALF pair (8 rows x 128 B each)
   constexpr int LQ = 4;   // activation copy instructions per wave per K tile (16 rows x 64 B each)
   static_assert(!OBLK || GATED, "only H is ever written blocked");
@@ -73,8 +78,8 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
   __shared__ __align__(1024) unsigned char ps1[PSLOT];
   __shared__ __align__(1024) unsigned char ps2[PSLOT];
   // activations: four 16 KB stages, or (QROW) two 32 KB pair slots qs0, qs1; one array per stage or slot
-  __shared__ __align__(1024) unsigned char qs0[QROW ? PSLOT : QSTAGE];
-  __shared__ __align__(1024) unsigned char qs1[QROW ? PSLOT : QSTAGE];
+  __shared__ __align__(1024) unsigned char qs0[QROW ? QSLOT : QSTAGE];
+  __shared__ __align__(1024) unsigned char qs1[QROW ? QSLOT : QSTAGE];
   unsigned char* qs2 = nullptr;
   unsigned char* qs3 = nullptr;
   if constexpr (!QROW) {  // 160 KB are all there is: the two stages exist only where they are used
@@ -140,7 +145,7 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
   const unsigned rd_p = PBLK ? (unsigned)((GATED ? wp * 64 : wp * 128) + r16) * 64u +
                                    (unsigned)((c4 ^ ((r16 >> 2) & 3)) * 16)
                              : (unsigned)((GATED ? wp * 64 : wp * 128) + r16) * 128u;
-  const unsigned rd_q = QROW ? (unsigned)(wq * 128 + r16) * 128u
+  const unsigned rd_q = QROW ? (unsigned)(wq * 16 * NQ + r16) * 128u
                              : (unsigned)(wq * 128 + r16) * 64u + (unsigned)((c4 ^ ((r16 >> 2) & 3)) * 16);
   unsigned xp[2];  // [half of the pair]
 #pragma unroll
@@ -151,17 +156,18 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
     return (unsigned)(f * 16) * RB;
   };
 
-  f32x4 acc[NB][NB];
+  f32x4 acc[NB][NQ];
 #pragma unroll
   for (int f = 0; f < NB; ++f)
 #pragma unroll
-    for (int g = 0; g < NB; ++g) acc[f][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < NQ; ++g) acc[f][g] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // two register sets of the 16 fragments of a K tile: [0..7] weight blocks, [8..15] activation blocks
-  u32x4 fr[2][2 * NB];
+  // two register sets of the fragments of a K tile: [0..7] weight blocks, [8..] activation blocks
+  u32x4 fr[2][NB + NQ];
   // ONE workgroup barrier per K PAIR (two K tiles, 128 MFMAs per wave), in the MIDDLE of the pair. Pair iteration I
   // multiplies tile a = 2I (fragments in register set 0) and tile b = 2I + 1 (set 1) in four quarters of 32 MFMAs;
-  // every quarter carries 8 fragment reads and 4 copies, so that LDS and the copy queue see an even load:
+  // every quarter carries 8 fragment reads and 4 copies, so that LDS and the copy queue see an even load (numbers for
+  // NQ = 8; in general a quarter is 4 NQ MFMAs, Q1 and Q3 read NQ fragments, Q3 + Q4 issue NQ copies):
   //   Q1  a, weight blocks 0..3   + the activation fragments of b      + weight copies 0..3 of pair I + 2
   //   Q2  a, weight blocks 4..7   + the weight fragments of b (first half of the quarter) + weight copies 4..7
   //   barrier: pair I + 1 has landed (all but the 8 weight copies just issued); every wave has read all of pair I
@@ -176,10 +182,10 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
   auto read_one = [&](int set, int idx, const unsigned char* pslot, int half, const unsigned char* qstage) {
     if (idx == 0) {
       fr[set][0] = *(const u32x4*)(pslot + rd_p + p_block_off(0) + (PBLK ? 0u : xp[half]));
-    } else if (idx <= NB) {
+    } else if (idx <= NQ) {
       fr[set][NB + idx - 1] = *(const u32x4*)(qstage + rd_q + (idx - 1) * 16 * (QROW ? 128 : 64) + (QROW ? xp[half] : 0u));
     } else {
-      fr[set][idx - NB] = *(const u32x4*)(pslot + rd_p + p_block_off(idx - NB) + (PBLK ? 0u : xp[half]));
+      fr[set][idx - NQ] = *(const u32x4*)(pslot + rd_p + p_block_off(idx - NQ) + (PBLK ? 0u : xp[half]));
     }
   };
   // MFMA i of a K tile: weight block f = i / 8, activation block g walking forth on even f and back on odd f, so
@@ -187,7 +193,7 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
   // fragment). Operand register reads cost power like everything else here: against restarting g at 0 the whole
   // forward at 8192 x 4096 x 14336 measures 0.5 % faster (1.8628 vs 1.8728 ms), bit-identical.
   auto mma_one = [&](int set, int i) {
-    const int f = i / NB, g = (f & 1) ? NB - 1 - i % NB : i % NB;
+    const int f = i / NQ, g = (f & 1) ? NQ - 1 - i % NQ : i % NQ;
     E::mfma16_acc(acc[f][g], fr[set][f], fr[set][NB + g]);
   };
   // activation copy j (0 .. 7) of pair `pair`: tile 2 pair + j / 4; tiles past the end arrive as zeros
@@ -230,15 +236,20 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
     unsigned char* const qfa = QROW ? qs[I & 1] : qs[(2 * I) & 3];
     unsigned char* const qb = QROW ? qs[I & 1] : qs[(2 * I + 1) & 3];
     unsigned char* const qna = QROW ? qs[(I + 1) & 1] : qs[(2 * I + 2) & 3];
+    // `n` events spread evenly over `steps` steps: those of step c are spread(c, n, steps) .. spread(c + 1, n, steps) - 1
+    auto spread = [](int c, int n, int steps) constexpr -> int { return c * n / steps; };
+    constexpr int QN = 4 * NQ;      // MFMAs of a quarter
+    constexpr int QC3 = NQ / 2;     // activation copies in Q3, the others in Q4
+    constexpr int R2 = NQ - 4;      // MFMAs per step in the second half of Q2
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
+    for (int c = 0; c < NQ; ++c) {
       mma_one(0, 4 * c + 0);
       read_one(1, 1 + c, pb, 1, qb);
       mma_one(0, 4 * c + 1);
       __builtin_amdgcn_sched_barrier(0);
       mma_one(0, 4 * c + 2);
-      if (c & 1) {
-        p_pair_copy(pfill, pr + 2, c >> 1);
+      if (spread(c + 1, 4, NQ) > spread(c, 4, NQ)) {
+        p_pair_copy(pfill, pr + 2, spread(c, 4, NQ));
         __builtin_amdgcn_sched_barrier(0);
       }
       mma_one(0, 4 * c + 3);
@@ -246,31 +257,31 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
     }
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      mma_one(0, 4 * NB + 2 * c);
-      read_one(1, c == 0 ? 0 : NB + c, pb, 1, qb);
-      mma_one(0, 4 * NB + 2 * c + 1);
+      mma_one(0, QN + 2 * c);
+      read_one(1, c == 0 ? 0 : NQ + c, pb, 1, qb);
+      mma_one(0, QN + 2 * c + 1);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      mma_one(0, 4 * NB + 16 + 4 * c);
-      mma_one(0, 4 * NB + 16 + 4 * c + 1);
+#pragma unroll
+      for (int i = 0; i < R2 / 2; ++i) mma_one(0, QN + 16 + R2 * c + i);
       p_pair_copy(pfill, pr + 2, 4 + c);
       __builtin_amdgcn_sched_barrier(0);
-      mma_one(0, 4 * NB + 16 + 4 * c + 2);
-      mma_one(0, 4 * NB + 16 + 4 * c + 3);
+#pragma unroll
+      for (int i = R2 / 2; i < R2; ++i) mma_one(0, QN + 16 + R2 * c + i);
       __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("s_waitcnt %0\n\ts_barrier" ::"n"(WAIT_IMM) : "memory");
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
+    for (int c = 0; c < NQ; ++c) {
       mma_one(1, 4 * c + 0);
       read_one(0, 1 + c, pna, 0, qna);
       mma_one(1, 4 * c + 1);
       __builtin_amdgcn_sched_barrier(0);
       mma_one(1, 4 * c + 2);
-      if (c & 1) {
-        q_pair_copy(qfa, qb, pr + 2, c >> 1);
+      if (spread(c + 1, QC3, NQ) > spread(c, QC3, NQ)) {
+        q_pair_copy(qfa, qb, pr + 2, spread(c, QC3, NQ));
         __builtin_amdgcn_sched_barrier(0);
       }
       mma_one(1, 4 * c + 3);
@@ -278,33 +289,36 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
     }
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      mma_one(1, 4 * NB + 4 * c);
-      read_one(0, c == 0 ? 0 : NB + c, pna, 0, qna);
-      mma_one(1, 4 * NB + 4 * c + 1);
+      const int m0 = QN + spread(c, QN, 8), m1 = QN + spread(c + 1, QN, 8);
+      mma_one(1, m0);
+      read_one(0, c == 0 ? 0 : NQ + c, pna, 0, qna);
+      mma_one(1, m0 + 1);
       __builtin_amdgcn_sched_barrier(0);
-      mma_one(1, 4 * NB + 4 * c + 2);
-      if (c & 1) {
-        q_pair_copy(qfa, qb, pr + 2, 4 + (c >> 1));
+#pragma unroll
+      for (int i = m0 + 2; i < m1 - 1; ++i) mma_one(1, i);
+      if (spread(c + 1, NQ - QC3, 8) > spread(c, NQ - QC3, 8)) {
+        q_pair_copy(qfa, qb, pr + 2, QC3 + spread(c, NQ - QC3, 8));
         __builtin_amdgcn_sched_barrier(0);
       }
-      mma_one(1, 4 * NB + 4 * c + 3);
+      if (m1 - m0 > 2) mma_one(1, m1 - 1);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
   if (nkt > 0) {
-    // pairs 0 and 1 of both operands; pair 0 has landed when the 16 copies of pair 1 are still in flight
+    // pairs 0 and 1 of both operands; pair 0 has landed when the copies of pair 1 are still in flight
+    constexpr int NC = QROW ? NQ : 8;  // activation copies of a pair
 #pragma unroll
     for (int j = 0; j < 8; ++j) p_pair_copy(ps0, 0, j);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) q_pair_copy(qs0, qs1, 0, j);
+    for (int j = 0; j < NC; ++j) q_pair_copy(qs0, qs1, 0, j);
 #pragma unroll
     for (int j = 0; j < 8; ++j) p_pair_copy(ps1, 1, j);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) q_pair_copy(QROW ? qs1 : qs2, qs3, 1, j);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * VM) : "memory");
+    for (int j = 0; j < NC; ++j) q_pair_copy(QROW ? qs1 : qs2, qs3, 1, j);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(VM + NC) : "memory");
 #pragma unroll
-    for (int i = 0; i < 2 * NB; ++i) read_one(0, i, ps0, 0, qs0);
+    for (int i = 0; i < NB + NQ; ++i) read_one(0, i, ps0, 0, qs0);
   }
   int pr = 0;
   for (; pr + 5 < npair; pr += 6) {
@@ -356,7 +370,7 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
     const int nblocks = (a.np / 2 + 31) >> 5;
     unsigned char* O = (unsigned char*)a.O;
 #pragma unroll
-    for (int g = 0; g < NB; ++g) {
+    for (int g = 0; g < NQ; ++g) {
       const int row = wq * 128 + g * 16 + r16e;
 #pragma unroll
       for (int f = 0; f < NB / 2; f += 2) {
@@ -377,8 +391,8 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
     float* const part = a.partial + (long long)blockIdx.y * a.nq * a.np;
     const bool vec_ok = (a.np & 3) == 0;
 #pragma unroll
-    for (int g = 0; g < NB; ++g) {
-      const int m = q0 + wq * 128 + g * 16 + r16e;
+    for (int g = 0; g < NQ; ++g) {
+      const int m = q0 + wq * 16 * NQ + g * 16 + r16e;
       if (m >= a.nq) continue;
       float* prow = part + (long long)m * a.np;
 #pragma unroll
@@ -399,8 +413,8 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
     const bool vec_ok = ((a.ldo & 3) == 0) && ((((uintptr_t)a.O) & 15) == 0);
     const int nbase = p0 / 2 + wp * 64;
 #pragma unroll
-    for (int g = 0; g < NB; ++g) {
-      const int m = q0 + wq * 128 + g * 16 + r16e;
+    for (int g = 0; g < NQ; ++g) {
+      const int m = q0 + wq * 16 * NQ + g * 16 + r16e;
       if (m >= a.nq) continue;
       float* orow = O + (long long)m * a.ldo;
 #pragma unroll
@@ -426,8 +440,8 @@ tiled_pair16_kernel(const GemmArgs a_in, const int tiles_p, const int tiles_q, c
     const bool vec16_ok = ((a.ldo & 7) == 0) && ((((uintptr_t)a.O) & 15) == 0);
     const int nbase = GATED ? p0 / 2 + wp * 64 : p0 + wp * 128;
 #pragma unroll
-    for (int g = 0; g < NB; ++g) {
-      const int m = q0 + wq * 128 + g * 16 + r16e;
+    for (int g = 0; g < NQ; ++g) {
+      const int m = q0 + wq * 16 * NQ + g * 16 + r16e;
       unsigned short* orow = O + (long long)m * a.ldo;
 #pragma unroll
       for (int f = 0; f < FO; f += 2) {
@@ -479,35 +493,35 @@ hipError_t launch_pair16_blocked_x(const GemmArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// both operands row-major (OBLK: H written blocked; OF32: H float)
-template <class E, bool GATED, bool OBLK = false, bool OF32 = false>
+// both operands row-major (OBLK: H written blocked; OF32: H float; NQ: 32 NQ activation rows per tile)
+template <class E, bool GATED, bool OBLK = false, bool OF32 = false, int NQ = 8>
 hipError_t launch_pair16_rowmajor(const GemmArgs& a, hipStream_t stream) {
   const int tiles_p = (a.np + 255) / 256;
-  const int tiles_q = (a.nq + 255) / 256;
+  const int tiles_q = (a.nq + 32 * NQ - 1) / (32 * NQ);
   if (tiles_p <= 0 || tiles_q <= 0) return hipSuccess;
   const dim3 grid((unsigned)(tiles_p * tiles_q)), block(256);
   if (a.k % 64 == 0) {
-    hipLaunchKernelGGL((tiled_pair16_kernel<E, GATED, false, OBLK, false, true, false, OF32>), grid, block, 0, stream, a,
+    hipLaunchKernelGGL((tiled_pair16_kernel<E, GATED, false, OBLK, false, true, false, OF32, NQ>), grid, block, 0, stream, a,
                        tiles_p, tiles_q, raster_group(GATED, tiles_q));
   } else {
-    hipLaunchKernelGGL((tiled_pair16_kernel<E, GATED, true, OBLK, false, true, false, OF32>), grid, block, 0, stream, a,
+    hipLaunchKernelGGL((tiled_pair16_kernel<E, GATED, true, OBLK, false, true, false, OF32, NQ>), grid, block, 0, stream, a,
                        tiles_p, tiles_q, raster_group(GATED, tiles_q));
   }
   return hipGetLastError();
 }
 
 // both operands row-major, plain product, K split over blockIdx.y: fp32 partial tiles to a.partial
-template <class E>
+template <class E, int NQ>
 hipError_t launch_pair16_split(const GemmArgs& a, hipStream_t stream) {
   const int tiles_p = (a.np + 255) / 256;
-  const int tiles_q = (a.nq + 255) / 256;
+  const int tiles_q = (a.nq + 32 * NQ - 1) / (32 * NQ);
   if (tiles_p <= 0 || tiles_q <= 0 || a.splits <= 0) return hipSuccess;
   const dim3 grid((unsigned)(tiles_p * tiles_q), (unsigned)a.splits), block(256);
   if (a.k % 64 == 0) {
-    hipLaunchKernelGGL((tiled_pair16_kernel<E, false, false, false, false, true, true>), grid, block, 0, stream, a,
+    hipLaunchKernelGGL((tiled_pair16_kernel<E, false, false, false, false, true, true, false, NQ>), grid, block, 0, stream, a,
                        tiles_p, tiles_q, raster_group(false, tiles_q));
   } else {
-    hipLaunchKernelGGL((tiled_pair16_kernel<E, false, true, false, false, true, true>), grid, block, 0, stream, a,
+    hipLaunchKernelGGL((tiled_pair16_kernel<E, false, true, false, false, true, true, false, NQ>), grid, block, 0, stream, a,
                        tiles_p, tiles_q, raster_group(false, tiles_q));
   }
   return hipGetLastError();
@@ -530,8 +544,21 @@ hipError_t launch_pair16_blocked_xw(const GemmArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// row-major operands and output, tiles of 32 NQ activation rows
+template <class E, int NQ>
+hipError_t launch_pair16_narrow(bool gated, const GemmArgs& a, hipStream_t stream) {
+  if (gated && a.out_f32) return launch_pair16_rowmajor<E, true, false, true, NQ>(a, stream);
+  return gated ? launch_pair16_rowmajor<E, true, false, false, NQ>(a, stream)
+               : launch_pair16_rowmajor<E, false, false, false, NQ>(a, stream);
+}
+
 template <class E>
 hipError_t launch_pair16_typed(bool gated, const GemmArgs& a, hipStream_t stream) {
+  if (a.layout == 0 && !(a.out_f32 && !gated)) {
+    if (a.tile_q == 224) return launch_pair16_narrow<E, 7>(gated, a, stream);
+    if (a.tile_q == 192) return launch_pair16_narrow<E, 6>(gated, a, stream);
+    if (a.tile_q == 160) return launch_pair16_narrow<E, 5>(gated, a, stream);
+  }
   if (gated && a.layout == 1) return launch_pair16_blocked_x<E, true, false>(a, stream);
   if (gated && a.layout == 3) return launch_pair16_blocked_x<E, true, true>(a, stream);
   if (!gated && a.layout == 1) return launch_pair16_blocked_x<E, false, false>(a, stream);
@@ -555,7 +582,10 @@ hipError_t launch_pair16(int dtype, bool gated, const GemmArgs& a, hipStream_t s
 
 // Row-major plain product with K split over a.splits workgroups per tile; fp32 partials to a.partial (not reduced).
 hipError_t launch_pair16_splitk(int dtype, const GemmArgs& a, hipStream_t stream) {
-  return dtype == 0 ? launch_pair16_split<Bf16>(a, stream) : launch_pair16_split<Fp16>(a, stream);
+  if (a.tile_q == 224) return dtype == 0 ? launch_pair16_split<Bf16, 7>(a, stream) : launch_pair16_split<Fp16, 7>(a, stream);
+  if (a.tile_q == 192) return dtype == 0 ? launch_pair16_split<Bf16, 6>(a, stream) : launch_pair16_split<Fp16, 6>(a, stream);
+  if (a.tile_q == 160) return dtype == 0 ? launch_pair16_split<Bf16, 5>(a, stream) : launch_pair16_split<Fp16, 5>(a, stream);
+  return dtype == 0 ? launch_pair16_split<Bf16, 8>(a, stream) : launch_pair16_split<Fp16, 8>(a, stream);
 }
 
 }  // namespace fsw

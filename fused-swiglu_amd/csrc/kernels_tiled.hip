@@ -526,6 +526,47 @@ hipError_t launch_variant(int variant, const GemmArgs& a, hipStream_t stream) {
 }
 
 }  // namespace
+
+// Rounds of one-workgroup-per-compute-unit launches, as time. A partly filled round takes 0.75 .. 0.8 of a full one up to
+// 160 workgroups (its compute units run at a higher clock) and grows from there to 1 (down 11008 -> 4096 in 256 x 256 tiles:
+// 64 workgroups 162.7 us, 128 167.7, 160 173, 192 191, 224 208; in 256 x 160 tiles 64 112.7, 160 121.6, 208 139, 240 148.5,
+// 256 152.7, 432 282).
+static double pair16_rounds(long long wgs) {
+  const double r = (double)(wgs % 256);
+  const double part = r == 0.0 ? 0.0 : (r <= 160.0 ? 0.75 + 0.05 * r / 160.0 : 0.8 + 0.2 * (r - 160.0) / 96.0);
+  return (double)(wgs / 256) + part;
+}
+
+// Time of a 256 x rows tile as a share of a 256 x 256 one (full rounds of the down product above: 216, 200.5, 177, 152.7
+// us; gate/up 4096 x 28672, 224 tiles: 79.2, 70.5, 62.9, 57.9): per FLOP the narrow tile costs up to 14 % more.
+struct NarrowTile {
+  int rows;
+  double cost;
+};
+static const NarrowTile kNarrow[] = {{256, 1.0}, {224, 0.91}, {192, 0.81}, {160, 0.715}};
+
+// Activation rows per tile of the 256-weight-row kernel: 256, or 224, 192, 160 where these fit the rows and the compute
+// units better, by the two measurements above. Only up to 512 large tiles (two rounds; gate/up, with seven times
+// as many, four): beyond, the padding of the last tile and the last round weigh little against the dearer tiles and against
+// blocked H, which these tiles do not read. A narrow tile must be ahead by 1 - `need`.
+// 256 -> best, us: gate/up 4096 x 28672: 300 rows 78 -> 57 (160), 333 rows 79 -> 63 (192), 448 rows 85 -> 77 (224),
+// 640 rows 150 -> 112 (160), 1000 rows stay (168, narrow 193 or more); 8192 x 57344, 520 rows 472 -> 412 (192); down
+// 11008 -> 4096: 2500 rows 173 -> 153 (160), 3000 rows 191 -> 177 (192), 4300 rows 379 -> 282 (160).
+int pair16_tile_rows(bool gated, long long np, long long nq, double need) {
+  const long long tp = (np + 255) / 256;
+  if (tp * ((nq + 255) / 256) > (gated ? 1024 : 512)) return 256;
+  int rows = 256;
+  double best = pair16_rounds(tp * ((nq + 255) / 256)) * need;
+  for (const NarrowTile& t : kNarrow) {
+    const double cost = t.cost * pair16_rounds(tp * ((nq + t.rows - 1) / t.rows));
+    if (t.rows < 256 && cost < best) {
+      best = cost;
+      rows = t.rows;
+    }
+  }
+  return rows;
+}
+
 SplitPlan tiled_split_plan(int np, int nq, int k) {
   const long long t128 = (long long)((np + 127) / 128) * ((nq + 127) / 128);
   const long long t256 = (long long)((np + 255) / 256) * ((nq + 255) / 256);
@@ -550,40 +591,48 @@ SplitPlan tiled_split_plan(int np, int nq, int k) {
     // 14336: 160 tiles x 3 splits 86 us, x 4 splits 110 us), and every split adds a partial tile to write and read
     // back. Estimated time per candidate, in us on 256 compute units: MFMA work of the busiest compute unit at
     // ~5.1 TFLOP/s (a lone 128 x 128 workgroup runs at half of that, the small tile costs ~15 % more per flop, the
-    // large one on 16x16x32 MFMAs ~15 % less) plus the fp32 partials at ~5 TB/s. Measured against it (4096 x 14336):
+    // large one on 16x16x32 MFMAs ~23 % less, see pair16_rounds() for its partly filled rounds) plus the fp32 partials at ~5 TB/s. Measured against it (4096 x 14336):
     // 257 rows 128/5 59 us, 640 rows 128/3 85 us, 1024 rows 256/4 106 us, 2048 rows 256/2 185 us, each within 5 % of
     // the fastest of 12 tile/split pairs tried.
     // From 129 large tiles up the unsplit alternative is the 16x16x32 kernel on blocked H (~8 % faster than on
     // row-major H, which the split kernel reads): there only large-tile splits are candidates, over several rounds
     // if need be, they must win by 15 %, and their partials stay under 256 MB.
+    // Below 129 large tiles the large tile comes in four heights (kNarrow); it is a candidate where 55 % of its rows are
+    // used, a narrow one where 85 % are and 256-row tiles would not be full. Down 11008 -> 4096, us, without -> with narrow
+    // tiles: 300 rows 56.0 -> 43.2 (160 x 6 splits), 333 rows 55.8 -> 45.8 (192 x 6), 640 rows 66.6 -> 57.3 (160 x 4), 1300
+    // rows 111.8 -> 98.9 (192 x 2); 28672 -> 8192, 520 rows 288 -> 249 (192 x 2).
     const int nkt = (k + 63) / 64;
     const bool large = t256 >= 129;
     double best = 0.0, unsplit = 0.0;
     p.tile = 128;
     p.splits = 1;
-    for (int c = large ? 1 : 0; c < 2; ++c) {
-      const int tile = c == 0 ? 128 : 256;
-      const long long nt = c == 0 ? t128 : t256;
-      const long long slots = c == 0 ? 512 : 256;
+    for (int c = large ? 0 : -1; c < 4; ++c) {  // -1: 128 x 128, 0 .. 3: kNarrow
+      const bool small = c < 0;
+      const int tile_q = small ? 128 : kNarrow[c].rows;
+      const long long nt = small ? t128 : (long long)((np + 255) / 256) * ((nq + tile_q - 1) / tile_q);
+      const long long padded = (long long)((nq + tile_q - 1) / tile_q) * tile_q;
+      if (c == 0 && !large && 20LL * nq < 11 * padded) continue;
+      if (c > 0 && (large || nq % 256 == 0 || 20LL * nq < 17 * padded)) continue;
+      const long long slots = small ? 512 : 256;
       long long smax = large ? 16 : slots / nt;
-      const long long deep = c == 0 ? k / 512 : k / 1024;  // at least 8 (16) K tiles of 64 per partition
+      const long long deep = small ? k / 512 : k / 1024;  // at least 8 (16) K tiles of 64 per partition
       if (smax > deep) smax = deep;
       if (smax > 16) smax = 16;
       if (smax < 1) smax = 1;
       for (int sp = 1; sp <= (int)smax; ++sp) {
         if (sp > 1 && 4.0 * sp * (double)nq * (double)np > 256e6) break;
+        if (sp == 1 && !large && tile_q != 128 && tile_q != 256) continue;  // unsplit: 128 x 128 below
         const double kper = 64.0 * ((nkt + sp - 1) / sp);
-        // a partly filled round of large tiles runs at a higher clock: 0.6 .. 0.95 of a full one (4096 x 14336:
-        // 16 tiles 0.57, 144 tiles 0.80, 176 tiles 0.83 of the 310 us a round of 256 takes)
         const long long wgs = nt * sp;
-        const double rounds = c == 0 ? (double)((wgs + slots - 1) / slots)
-                                     : (double)(wgs / slots) + (wgs % slots ? 0.6 + 0.35 * (wgs % slots) / slots : 0.0);
-        const double mfma = 2.0 * kper * tile * tile * (c == 0 ? 2.0 * 1.15 : 0.85) * rounds / 5.1e6;
+        const double rounds = small ? (double)((wgs + slots - 1) / slots) : pair16_rounds(wgs);
+        const double tile_cost = small ? 2.0 * kper * 128 * 128 * 2.0 * 1.15 : 2.0 * kper * 256 * 256 * 0.77 * kNarrow[c].cost;
+        const double mfma = tile_cost * rounds / 5.1e6;
         const double partials = sp > 1 ? 8.0 * sp * (double)nq * (double)np / 5.0e6 : 0.0;
-        if (sp == 1 && c == 1) unsplit = mfma;
-        if (best == 0.0 || mfma + partials < best) {
-          best = mfma + partials;
-          p.tile = tile;
+        if (sp == 1 && !small && (unsplit == 0.0 || mfma < unsplit)) unsplit = mfma;
+        const double cost = (c > 0 ? 1.05 : 1.0) * (mfma + partials);  // the estimates are no closer than 5 %
+        if (best == 0.0 || cost < best) {
+          best = cost;
+          p.tile = tile_q;
           p.splits = sp;
         }
       }
@@ -659,8 +708,10 @@ hipError_t launch_tiled_splitk(int dtype, int tile, const GemmArgs& a, hipStream
   if (tile == 129) {  // 128 output features x 256 activation rows, 8 waves
     return dtype == 0 ? launch_splitk_one<Bf16, 2, 4, 2, 2>(a, stream) : launch_splitk_one<Fp16, 2, 4, 2, 2>(a, stream);
   }
-  // 256 x 256 on the 16x16x32 kernel, then the reduction
-  const hipError_t e = launch_pair16_splitk(dtype, a, stream);
+  // 256 x tile on the 16x16x32 kernel, then the reduction
+  GemmArgs b = a;
+  b.tile_q = tile;
+  const hipError_t e = launch_pair16_splitk(dtype, b, stream);
   if (e != hipSuccess || a.splits <= 1) return e;
   return dtype == 0 ? launch_splitk_reduce<Bf16>(a, stream) : launch_splitk_reduce<Fp16>(a, stream);
 }

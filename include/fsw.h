@@ -196,6 +196,7 @@ FSW_API int fsw_version(void);
  * (69.7 vs 61.0 us at M = 16, d = 4096, ff = 14336) and is kept for study only; 103 is 101 with a barrier that cannot
  * complete, a hook of the failure-path test that is refused (FSW_E_VARIANT) unless the environment holds
  * FSW_TEST_HOOKS=1;
+ * variants 115, 116, 117 = the 256-row kernel with 160, 192, 224 activation rows per tile (row-major operands);
  * family 1 variant 104 makes fsw_mlp run the down projection of M <= 32 rows on the split-K streaming kernel
  * (32-row tiles, two K ranges whose partial tiles meet through ticket counters that the gate/up kernel zeroes)
  * whatever the shape; the dispatcher picks it for 17 .. 32 rows of large weight matrices.

@@ -646,6 +646,68 @@ def test_stage_ring_with_few_k_tiles(capi, M, K):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [160, 192, 224])
+@pytest.mark.parametrize("K", [8, 64, 72, 200, 392, 456, 832])
+def test_narrow_tiles_give_the_bits_of_256_row_tiles(capi, rows, dtype, K):
+    """Tiles of 256 weight rows x 160, 192, 224 activation rows (variants 115 .. 117) around their row and K-pair edges: the
+    K order of an output does not depend on the tile, so both projections equal the 256 x 256 kernel bit for bit, in the
+    row-major and (large layers) the float32 output; outputs inside a wider NaN buffer."""
+    v = 110 + rows // 32
+    for M in (1, rows - 1, rows, rows + 1, 2 * rows + 17):
+        ff = 8 * (33 + M % 5)
+        inp = fsw_weights.make_inputs(M, K, ff, dtype, seed=rows + K + M, x_scale=0.5)
+        g = to_dev(inp)
+        out = {}
+        try:
+            for which in (5, v):
+                capi.set_variant(0, which)
+                capi.set_variant(1, which)
+                wh = torch.full((M, ff + 8), float("nan"), dtype=dtype, device=DEV)
+                wy = torch.full((M, K + 8), float("nan"), dtype=dtype, device=DEV)
+                H = capi.gateup(g["X"], g["W13"], out=wh[:, :ff])
+                capi.down(H.contiguous(), g["W2"], out=wy[:, :K])
+                assert torch.isnan(wh[:, ff:]).all() and torch.isnan(wy[:, K:]).all()
+                out[which] = (wh[:, :ff], wy[:, :K])
+            assert capi.variant_name(0, 0, M, 2 * ff, K) == "pair16_256x%d" % rows or M <= 64
+        finally:
+            capi.set_variant(0, -1)
+            capi.set_variant(1, -1)
+        assert torch.equal(out[5][0], out[v][0]) and torch.equal(out[5][1], out[v][1]), (M, K, ff)
+    assert_one_rounding(H, oracle.ref_gateup(inp["X"], inp["W13"], torch.float64), dtype, "narrow H")
+    if K == 832:  # 832 x 2528 is past the size from which the float32 output honours the kernel choice
+        inp = fsw_weights.make_inputs(rows + 40, K, 2528, dtype, seed=rows, x_scale=0.5)
+        g = to_dev(inp)
+        try:
+            capi.set_variant(0, v)
+            H32, H16 = capi.gateup_f32out(g["X"], g["W13"]), capi.gateup(g["X"], g["W13"])
+        finally:
+            capi.set_variant(0, -1)
+        ref = oracle.ref_gateup(inp["X"], inp["W13"], torch.float64)
+        assert not ((H32.cpu().double() - ref).abs() > 1e-5 * (1.0 + ref.abs())).any()
+        assert torch.equal(H16, H32.to(dtype))
+
+
+NARROW_SPLITS = [(435, 4096, 8192, 160), (300, 4096, 8200, 160), (520, 4096, 3072, 192), (520, 2048, 8200, 192),
+                 (400, 4096, 8192, 224), (400, 4096, 8200, 224)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,D,FF,rows", NARROW_SPLITS)
+def test_split_k_on_narrow_tiles(capi, M, D, FF, rows, dtype):
+    """The split-K down projection on tiles of 160, 192 and 224 activation rows, K a multiple of 64 and not, last tile full
+    and not: against the oracle on a one-rounding bound, output inside a wider NaN buffer."""
+    assert capi.variant_name(1, 0, M, D, FF) == "splitk_pair16_256x%d" % rows
+    gen = torch.Generator().manual_seed(M + FF)
+    H = (torch.randn(M, FF, generator=gen) * 0.5).to(dtype)
+    W2 = (torch.randn(D, FF, generator=gen) / FF ** 0.5).to(dtype)
+    wide = torch.full((M, D + 8), float("nan"), dtype=dtype, device=DEV)
+    capi.down(H.to(DEV), W2.to(DEV), out=wide[:, :D])
+    assert torch.isnan(wide[:, D:]).all()
+    ref = (H.to(DEV).double() @ W2.to(DEV).double().T).cpu()
+    assert_one_rounding(wide[:, :D], ref, dtype, "split %s" % ((M, D, FF),))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 16, 64, 65, 300, 1024])
 def test_float32_output_is_the_unrounded_gated_value(capi, M, dtype):
     """fsw_gateup_f32out (the reference's build with C_TYPE float, constants.cuh:9-14, swiglu.cu:470-471): H in
