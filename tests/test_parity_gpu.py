@@ -687,6 +687,21 @@ def test_narrow_tiles_give_the_bits_of_256_row_tiles(capi, rows, dtype, K):
         assert torch.equal(H16, H32.to(dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,D,FF", [(49, 512, 4096), (63, 1000, 2056), (64, 512, 4104), (64, 136, 1032), (33, 4096, 8200)])
+def test_split_k_of_at_most_64_rows(capi, M, D, FF, dtype):
+    """The split-K down projection on 128 x 64 tiles (four stages): full and ragged rows and features, K with and without
+    a tail, parts of a few K tiles. Output inside a wider NaN buffer."""
+    assert capi.variant_name(1, 0, M, D, FF) == "splitk_dma_128x128"
+    gen = torch.Generator().manual_seed(M + FF)
+    H = (torch.randn(M, FF, generator=gen) * 0.5).to(dtype)
+    W2 = (torch.randn(D, FF, generator=gen) / FF ** 0.5).to(dtype)
+    wide = torch.full((M, D + 8), float("nan"), dtype=dtype, device=DEV)
+    capi.down(H.to(DEV), W2.to(DEV), out=wide[:, :D])
+    assert torch.isnan(wide[:, D:]).all()
+    assert_one_rounding(wide[:, :D], H.double() @ W2.double().T, dtype, "split %s" % ((M, D, FF),))
+
+
 NARROW_SPLITS = [(435, 4096, 8192, 160), (300, 4096, 8200, 160), (520, 4096, 3072, 192), (520, 2048, 8200, 192),
                  (400, 4096, 8192, 224), (400, 4096, 8200, 224)]
 
