@@ -76,7 +76,7 @@ int pick_tiled(int family, int64_t m, int64_t np, double narrow_need = 0.95) {
     // Up to 192 rows the tile is 128 x 192: the single-tile kernels are bound by their MFMA and LDS work as much as
     // by the weight stream (4096 x 28672, M = 160: 65 -> 54 us; 5120 x 27648: 89 -> 68 us).
     // 193 .. 256 rows: 128 x 256 on 8 waves, two per SIMD (4096 x 28672: 72 -> 64 us, 5120 x 27648: 94 -> 79-87 us
-    // against the 4-wave instance, variant 15).
+    // against the 4-wave instance, variant 1).
     if (family == 0 && m > 128 && m <= 256 && (np + 127) / 128 >= 128) return m <= 192 ? V_128x192 : V_8W_128x256;
     // up to 64 rows the gate/up tile is 128 x 64 (4096 x 28672, M = 48: 39.4 -> 37.2 us)
     return (family == 0 && m <= 64) ? V_128x64 : V_128x128;
@@ -388,20 +388,30 @@ static size_t stream_scratch_bytes(const fsw::StreamPlan& p) {
   return (p.partial_bytes + (size_t)p.ticket_words * 4 + 255) & ~(size_t)255;
 }
 
-size_t fsw_down_workspace_bytes(int dtype, int64_t M, int64_t D, int64_t FF) {
-  (void)dtype;
+// Bytes of the split-K down projection's partial sums, 0 if it runs unsplit. `limit`: most bytes they may take; a plan that
+// wants more splits K less often (fsw_mlp_static, whose scratch is fixed, keeps the shapes that any plan fits).
+static size_t down_split(int64_t M, int64_t D, int64_t FF, size_t limit, fsw::SplitPlan* plan) {
   if (M <= 0 || M > MAX_DIM || D <= 0 || D > MAX_DIM || FF <= 0 || FF > MAX_DIM || streams_weights(1, M, D, FF)) return 0;
   if (g_forced_variant[1] >= 0) return 0;  // a forced kernel runs unsplit
-  const fsw::SplitPlan plan = fsw::tiled_split_plan((int)D, (int)M, (int)FF);
-  return plan.splits > 1 ? (size_t)plan.splits * (size_t)M * (size_t)D * sizeof(float) : 0;
+  *plan = fsw::tiled_split_plan((int)D, (int)M, (int)FF);
+  const size_t part = (size_t)M * (size_t)D * sizeof(float);
+  if (plan->splits > 1 && limit / part < (size_t)plan->splits) plan->splits = (int)(limit / part);
+  return plan->splits > 1 ? plan->splits * part : 0;
 }
 
-int fsw_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H, int64_t ldh, const void* W2, int64_t ldw2,
-             void* Y, int64_t ldy, void* workspace, size_t workspace_bytes, void* stream) {
+size_t fsw_down_workspace_bytes(int dtype, int64_t M, int64_t D, int64_t FF) {
+  (void)dtype;
+  fsw::SplitPlan plan;
+  return down_split(M, D, FF, SIZE_MAX, &plan);
+}
+
+static int down_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* H, int64_t ldh, const void* W2, int64_t ldw2,
+                     void* Y, int64_t ldy, void* workspace, size_t workspace_bytes, size_t limit, void* stream) {
   const int rc = fsw_validate_down(dtype, M, D, FF, H, ldh, W2, ldw2, Y, ldy);
   if (rc != FSW_OK) return rc;
   if (M == 0 || D == 0) return FSW_OK;
-  const size_t need = fsw_down_workspace_bytes(dtype, M, D, FF);
+  fsw::SplitPlan plan;
+  const size_t need = down_split(M, D, FF, limit, &plan);
   if (need > 0 && (!workspace || workspace_bytes < need)) return FSW_E_WORKSPACE;
   const int drc = check_device();
   if (drc != FSW_OK) return drc;
@@ -432,9 +442,8 @@ int fsw_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H, int64_t
     }
     return finish(fsw::launch_skinny(dtype, false, a, workspace, (hipStream_t)stream));
   }
-  if (need > 0 && g_forced_variant[1] < 0) {  // few output tiles, deep K: split K across workgroups
+  if (need > 0) {  // few output tiles, deep K: split K across workgroups
     if (!aligned16(workspace)) return FSW_E_ALIGN;
-    const fsw::SplitPlan plan = fsw::tiled_split_plan((int)D, (int)M, (int)FF);
     a.splits = plan.splits;
     a.partial = (float*)workspace;
     return finish(fsw::launch_tiled_splitk(dtype, plan.tile, a, (hipStream_t)stream));
@@ -442,16 +451,33 @@ int fsw_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H, int64_t
   return finish(launch_tiled_variant(v, dtype, false, a, (hipStream_t)stream));
 }
 
+int fsw_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H, int64_t ldh, const void* W2, int64_t ldw2,
+             void* Y, int64_t ldy, void* workspace, size_t workspace_bytes, void* stream) {
+  return down_impl(dtype, M, D, FF, H, ldh, W2, ldw2, Y, ldy, workspace, workspace_bytes, SIZE_MAX, stream);
+}
+
+static size_t h_bytes(int64_t M, int64_t FF) {
+  const size_t raw = (size_t)M * (size_t)FF * 2;
+  return (raw + 255) & ~(size_t)255;
+}
+
+// what row-major H leaves of `scratch` bytes (SIZE_MAX: no limit) for the down projection's partial sums
+static size_t beside_h(int64_t M, int64_t FF, size_t scratch) {
+  const size_t h = h_bytes(M, FF);
+  return scratch == SIZE_MAX ? SIZE_MAX : scratch > h ? (scratch - h) & ~(size_t)255 : 0;
+}
+
 // Large-tile regime of fsw_mlp: both projections run 256 x 256 tiles, and H never exists row-major: the gate/up
 // epilogue writes it panel-blocked (whole 1 KB runs) and the down projection reads it blocked. Against row-major H
 // the whole forward measures 0.8 % (8192 x 4096 x 14336) to 1.3 % (4096 x 4096 x 11008) faster; X is read row-major.
-static bool blocked_regime(int64_t M, int64_t D, int64_t FF) {
+static bool blocked_regime(int64_t M, int64_t D, int64_t FF, size_t scratch) {
   if (M <= 64 || D <= 0 || FF <= 0 || g_forced_variant[0] >= 0 || g_forced_variant[1] >= 0) return false;
   if (M > MAX_DIM || D > MAX_DIM || FF > MAX_DIM / 2) return false;
   // a down projection on narrower tiles reads row-major H; it has to gain more than H blocked does (3000 rows of 4096 x
   // 11008: 7 % of the down kernel, a third of the forward, is not enough; 2500 rows: 11 %)
+  fsw::SplitPlan plan;  // a split-K down projection reads row-major H
   return pick_tiled(0, M, 2 * FF) == V_256x256 && pick_tiled(1, M, D, 0.9) == V_256x256 &&
-         fsw::tiled_split_plan((int)D, (int)M, (int)FF).splits == 1;  // a split-K down projection reads row-major H
+         (size_t)fsw::blocked_bytes(M, FF) <= scratch && down_split(M, D, FF, beside_h(M, FF, scratch), &plan) == 0;
 }
 
 size_t fsw_blocked_bytes(int64_t rows, int64_t k) {
@@ -585,29 +611,31 @@ int fsw_gateup_ws(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int
   return fsw_gateup(dtype, M, N, K, X, ldx, W13, ldw, H, ldh, stream);
 }
 
-static size_t h_bytes(int64_t M, int64_t FF) {
-  const size_t raw = (size_t)M * (size_t)FF * 2;
-  return (raw + 255) & ~(size_t)255;
-}
-
-size_t fsw_mlp_workspace_bytes(int dtype, int64_t M, int64_t D, int64_t FF) {
+// `scratch`: the bytes there are, which the plan keeps to if H alone fits (SIZE_MAX: no limit)
+static size_t mlp_workspace(int64_t M, int64_t D, int64_t FF, size_t scratch) {
   if (M <= 0 || D <= 0 || FF <= 0) return 0;
-  if (blocked_regime(M, D, FF)) return (size_t)fsw::blocked_bytes(M, FF);  // H, panel-blocked
+  if (blocked_regime(M, D, FF, scratch)) return (size_t)fsw::blocked_bytes(M, FF);  // H, panel-blocked
   const fsw::StreamPlan sp = mlp_stream_plan(M, D, FF);
   if (sp.splits > 1) return h_bytes(M, FF) + stream_scratch_bytes(sp);  // [H row-major][partials][ticket counters]
   // otherwise [H row-major][split-K scratch of the down projection]
-  return h_bytes(M, FF) + ((fsw_down_workspace_bytes(dtype, M, D, FF) + 255) & ~(size_t)255);
+  fsw::SplitPlan plan;
+  return h_bytes(M, FF) + ((down_split(M, D, FF, beside_h(M, FF, scratch), &plan) + 255) & ~(size_t)255);
+}
+
+size_t fsw_mlp_workspace_bytes(int dtype, int64_t M, int64_t D, int64_t FF) {
+  (void)dtype;
+  return mlp_workspace(M, D, FF, SIZE_MAX);
 }
 
 // single_launch_ok: whether the opt-in single-launch decode forward may be used (it creates events on first use,
-// which the entry point that must not allocate cannot afford)
+// which the entry point that must not allocate cannot afford); scratch: see mlp_workspace
 static int mlp_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* X, int64_t ldx, const void* W13,
                     int64_t ldw13, const void* W2, int64_t ldw2, void* Y, int64_t ldy, void* workspace,
-                    size_t workspace_bytes, void* stream, bool single_launch_ok) {
+                    size_t workspace_bytes, void* stream, bool single_launch_ok, size_t scratch) {
   if (dtype != FSW_BF16 && dtype != FSW_FP16) return FSW_E_DTYPE;
   if (M < 0 || D < 0 || FF < 0 || M > MAX_DIM || D > MAX_DIM || FF > MAX_DIM / 2) return FSW_E_SHAPE;
   if (M == 0 || D == 0) return FSW_OK;  // Y is empty: nothing to read or write
-  const size_t need = fsw_mlp_workspace_bytes(dtype, M, D, FF);
+  const size_t need = mlp_workspace(M, D, FF, scratch);
   if (need > 0 && (!workspace || workspace_bytes < need)) return FSW_E_WORKSPACE;
   if (need > 0 && !aligned16(workspace)) return FSW_E_ALIGN;
   // FF == 0 needs no H: any non-NULL pointer satisfies the validators and is never dereferenced
@@ -645,7 +673,7 @@ static int mlp_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* X, 
       if (lrc != FSW_OK || launched) return lrc;
     }
   }
-  if (blocked_regime(M, D, FF)) {  // workspace = H, panel-blocked
+  if (blocked_regime(M, D, FF, scratch)) {  // workspace = H, panel-blocked
     rc = fsw_gateup_hblocked(dtype, M, 2 * FF, D, X, ldx, W13, ldw13, 0, workspace, stream);
     if (rc != FSW_OK) return rc;
     return fsw_down_blocked(dtype, M, D, FF, workspace, W2, ldw2, 0, Y, ldy, stream);
@@ -668,16 +696,17 @@ static int mlp_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* X, 
     a.k = (int)FF;
     return finish(fsw::launch_stream_split(dtype, a, sp, ws2, (hipStream_t)stream));
   }
-  const size_t down_ws = (fsw_down_workspace_bytes(dtype, M, D, FF) + 255) & ~(size_t)255;
+  const size_t down_ws = workspace_bytes > h_bytes(M, FF) ? workspace_bytes - h_bytes(M, FF) : 0;
   rc = fsw_gateup(dtype, M, 2 * FF, D, X, ldx, W13, ldw13, Hbuf, FF, stream);
   if (rc != FSW_OK) return rc;
-  return fsw_down(dtype, M, D, FF, Hbuf, FF, W2, ldw2, Y, ldy, ws2, down_ws, stream);
+  return down_impl(dtype, M, D, FF, Hbuf, FF, W2, ldw2, Y, ldy, ws2, down_ws, beside_h(M, FF, scratch), stream);
 }
 
 int fsw_mlp(int dtype, int64_t M, int64_t D, int64_t FF, const void* X, int64_t ldx, const void* W13, int64_t ldw13,
             const void* W2, int64_t ldw2, void* Y, int64_t ldy, void* workspace, size_t workspace_bytes,
             void* stream) {
-  return mlp_impl(dtype, M, D, FF, X, ldx, W13, ldw13, W2, ldw2, Y, ldy, workspace, workspace_bytes, stream, true);
+  return mlp_impl(dtype, M, D, FF, X, ldx, W13, ldw13, W2, ldw2, Y, ldy, workspace, workspace_bytes, stream, true,
+                  SIZE_MAX);
 }
 
 // ---- the entry point that allocates nothing ------------------------------------------------------------------
@@ -717,13 +746,14 @@ int fsw_mlp_static(int dtype, int64_t M, int64_t D, int64_t FF, const void* X, i
   if (dtype != FSW_BF16 && dtype != FSW_FP16) return FSW_E_DTYPE;
   if (M < 0 || D < 0 || FF < 0 || M > MAX_DIM || D > MAX_DIM || FF > MAX_DIM / 2) return FSW_E_SHAPE;
   if (M == 0 || D == 0) return FSW_OK;
-  if (fsw_mlp_workspace_bytes(dtype, M, D, FF) > FSW_STATIC_SCRATCH_BYTES) return FSW_E_STATIC_LIMIT;
+  if (mlp_workspace(M, D, FF, FSW_STATIC_SCRATCH_BYTES) > FSW_STATIC_SCRATCH_BYTES) return FSW_E_STATIC_LIMIT;
   const int drc = check_device();
   if (drc != FSW_OK) return drc;
   void* ws = nullptr;
   const int rc = static_scratch_ptr(&ws);
   if (rc != FSW_OK) return rc;
-  return mlp_impl(dtype, M, D, FF, X, ldx, W13, ldw13, W2, ldw2, Y, ldy, ws, FSW_STATIC_SCRATCH_BYTES, stream, false);
+  return mlp_impl(dtype, M, D, FF, X, ldx, W13, ldw13, W2, ldw2, Y, ldy, ws, FSW_STATIC_SCRATCH_BYTES, stream, false,
+                  FSW_STATIC_SCRATCH_BYTES);
 }
 
 }  // extern "C"

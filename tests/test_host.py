@@ -326,3 +326,20 @@ def test_meta_kernels_trace_shapes_without_a_gpu(ext):
         a = torch.empty(5, 16, dtype=torch.bfloat16, device="cuda")
         b = torch.empty(12, 16, dtype=torch.bfloat16, device="cuda")
         assert torch.ops.ASMLLM.fused_swiglu_bf16(a, b).shape == (5, 6)
+
+
+@pytest.mark.parametrize("M,d,ff", [(996, 2048, 11008), (5938, 1024, 3272), (849, 1024, 19136), (771, 8480, 22872),
+                                    (2833, 4096, 11008), (1785, 4096, 4712), (373, 5376, 26528), (2340, 4096, 14336)])
+def test_static_forward_takes_every_shape_whose_h_fits(capi, M, d, ff):
+    """Narrow tiles made the down projection split K more often, and fsw_mlp_static refused shapes that it had taken: its
+    plan keeps to the array. The NULL operands (with a GPU) or the missing GPU are what these calls report."""
+    L = capi.lib()
+    assert 2 * M * ff <= L.fsw_mlp_static_max_bytes()
+    rc = L.fsw_mlp_static(0, M, d, ff, None, d, None, d, None, ff, None, d, None)
+    assert rc in (capi.E_DEVICE, capi.E_NULL)
+
+
+def test_static_forward_refuses_what_cannot_fit(capi):
+    L = capi.lib()
+    assert L.fsw_mlp_static(0, 2341, 4096, 14336, None, 4096, None, 4096, None, 14336, None, 4096,
+                            None) == capi.E_STATIC_LIMIT

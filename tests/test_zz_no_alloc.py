@@ -62,6 +62,29 @@ def test_static_scratch_forward_matches_fsw_mlp_call_after_call(capi):
         assert torch.equal(Y, want), "second pass differs at %s" % (shape,)
 
 
+# plan of the down projection with all the scratch it wants -> within the array: fewer splits, no split, H row-major
+@pytest.mark.parametrize("M,d,ff", [(996, 2048, 11008), (5938, 1024, 3272), (849, 1024, 19136), (1785, 4096, 4712),
+                                    (2833, 4096, 11008)])
+def test_static_scratch_forward_with_a_smaller_plan(capi, M, d, ff):
+    """Shapes whose H fits the array and whose split-K plan does not: within one rounding of fsw_mlp's result (H is
+    the same, the fp32 sums are taken in another order), repeated calls equal, output inside a wider NaN buffer."""
+    L = capi.lib()
+    assert L.fsw_mlp_workspace_bytes(0, M, d, ff) > L.fsw_mlp_static_max_bytes() >= 2 * M * ff
+    gen = torch.Generator(device=DEV).manual_seed(M)
+    X = torch.randn(M, d, generator=gen, device=DEV).to(torch.bfloat16)
+    W13 = (torch.randn(2 * ff, d, generator=gen, device=DEV) / d ** 0.5).to(torch.bfloat16)
+    W2 = (torch.randn(d, ff, generator=gen, device=DEV) / ff ** 0.5).to(torch.bfloat16)
+    want = capi.mlp(X, W13, W2).double()
+    wide = torch.full((M, d + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    Y = wide[:, :d]
+    capi.mlp_static(X, W13, W2, out=Y)
+    first = Y.clone()
+    # two roundings to bf16 (2^-8 each, half a unit either side) of sums that differ by fp32 rounding
+    assert not ((first.double() - want).abs() > 2.0 ** -7 * want.abs() + 1e-5).any()
+    capi.mlp_static(X, W13, W2, out=Y)
+    assert torch.equal(first, Y) and torch.isnan(wide[:, d:]).all()
+
+
 def test_static_scratch_limit_and_errors(capi):
     L = capi.lib()
     limit = L.fsw_mlp_static_max_bytes()
