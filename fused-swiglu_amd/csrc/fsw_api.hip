@@ -59,7 +59,7 @@ constexpr int V_128x128 = 0, V_128x192 = 2, V_8W_128x256 = 3, V_128x64 = 4, V_25
 // Variant choice for the tiled kernels: the widest tile whose activation-row extent is not mostly padding,
 // stepping down to 128x128 when a 256-wide grid would leave most of the 256 CUs idle.
 // `narrow_need`: a narrower large tile is taken only if its estimated time is below this share of 256 x 256's
-int pick_tiled(int family, int64_t m, int64_t np, double narrow_need = 0.95) {
+int pick_tiled(int family, int64_t m, int64_t np, int64_t k, double narrow_need = 0.95) {
   const int64_t tiles256 = ((np + 255) / 256) * ((m + 255) / 256);
   // 256 x 256 tiles down to half-filled compute units. Below that the down product splits K (see
   // tiled_split_plan); between 129 and 191 tiles one large tile per compute unit beats 128 x 128 tiles in
@@ -77,7 +77,21 @@ int pick_tiled(int family, int64_t m, int64_t np, double narrow_need = 0.95) {
     // by the weight stream (4096 x 28672, M = 160: 65 -> 54 us; 5120 x 27648: 89 -> 68 us).
     // 193 .. 256 rows: 128 x 256 on 8 waves, two per SIMD (4096 x 28672: 72 -> 64 us, 5120 x 27648: 94 -> 79-87 us
     // against the 4-wave instance, variant 1).
-    if (family == 0 && m > 128 && m <= 256 && (np + 127) / 128 >= 128) return m <= 192 ? V_128x192 : V_8W_128x256;
+    // All that only where two 128-row tiles are more workgroups than compute units: up to 256 workgroups 128 x 128 tiles
+    // have three stages each and a compute unit to themselves (4096 x 16384: M = 129 47.6 -> 41.8 us, M = 256 54.9 -> 45.9;
+    // 2048 x 16384: M = 200 29.3 -> 23.2).
+    // The same limit above 256 rows: 257 .. 512 workgroups of 128 x 128 share compute units two by two and keep two stages,
+    // so the wider tile whose launch fills one round (224 .. 256 workgroups) is taken (4096 x 16384: M = 257 66.6 -> 50.6 us
+    // and M = 384 72.7 -> 58.7 on 128 x 192, M = 450 75.3 -> 61.5 and M = 512 79.0 -> 64.6 on 128 x 256; 2048 x 16384: M =
+    // 384 37.9 -> 31.3). Not with fewer workgroups (2048 x 11264, M = 512, 176 wide ones: 29.5 -> 31.7) and not with a
+    // short K (1024 x 16384, M = 384: 17.1 -> 18.5).
+    const int64_t tp = (np + 127) / 128;
+    if (family == 0 && m > 128 && tp * ((m + 127) / 128) > 256) {
+      if (m <= 256 && tp >= 128) return m <= 192 ? V_128x192 : V_8W_128x256;
+      const int64_t w192 = tp * ((m + 191) / 192), w256 = tp * ((m + 255) / 256);
+      if (k >= 2048 && w192 >= 224 && w192 <= 256) return V_128x192;
+      if (k >= 2048 && w256 >= 224 && w256 <= 256) return V_8W_128x256;
+    }
     // up to 64 rows the gate/up tile is 128 x 64 (4096 x 28672, M = 48: 39.4 -> 37.2 us)
     return (family == 0 && m <= 64) ? V_128x64 : V_128x128;
   }
@@ -127,7 +141,7 @@ int resolve_variant(int family, int64_t m, int64_t np, int64_t k) {
   const int forced = g_forced_variant[family];
   if (forced == VARIANT_DECODE_FUSED || forced == VARIANT_DECODE_FUSED_FAIL || forced == VARIANT_DECODE_STREAM ||
       forced == VARIANT_STREAM_SPLIT)
-    return m <= 64 ? VARIANT_SKINNY : pick_tiled(family, m, np);
+    return m <= 64 ? VARIANT_SKINNY : pick_tiled(family, m, np, k);
   if (forced >= 0 && !(forced == VARIANT_SKINNY && m > 64)) return forced;
   if (m <= decode_rows(family, np, k)) {  // decode and small batches: weight streaming, HBM bound
     // The gate/up product streams its weights faster through the three-stage 128 x 64 tiled kernel (direct-to-LDS
@@ -138,7 +152,7 @@ int resolve_variant(int family, int64_t m, int64_t np, int64_t k) {
     if (family == 0 && m >= 12 && k > 0 && tiles >= 200 && tiles <= 256) return V_128x64;
     return VARIANT_SKINNY;
   }
-  return pick_tiled(family, m, np);
+  return pick_tiled(family, m, np, k);
 }
 
 // the weight-streaming kernels need no scratch and no blocked operands
@@ -476,7 +490,7 @@ static bool blocked_regime(int64_t M, int64_t D, int64_t FF, size_t scratch) {
   // a down projection on narrower tiles reads row-major H; it has to gain more than H blocked does (3000 rows of 4096 x
   // 11008: 7 % of the down kernel, a third of the forward, is not enough; 2500 rows: 11 %)
   fsw::SplitPlan plan;  // a split-K down projection reads row-major H
-  return pick_tiled(0, M, 2 * FF) == V_256x256 && pick_tiled(1, M, D, 0.9) == V_256x256 &&
+  return pick_tiled(0, M, 2 * FF, D) == V_256x256 && pick_tiled(1, M, D, FF, 0.9) == V_256x256 &&
          (size_t)fsw::blocked_bytes(M, FF) <= scratch && down_split(M, D, FF, beside_h(M, FF, scratch), &plan) == 0;
 }
 

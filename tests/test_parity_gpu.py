@@ -645,6 +645,24 @@ def test_stage_ring_with_few_k_tiles(capi, M, K):
     assert_one_rounding(Y, oracle.ref_down(H.cpu(), inp["W2"], torch.float64), torch.bfloat16, "Y %s" % ((M, K),))
 
 
+@pytest.mark.parametrize("M,K,ff,name", [(129, 264, 8192, "dma_128x128"), (256, 264, 8192, "dma_128x128"),
+                                         (200, 264, 8200, "dma8w_128x256"), (257, 2048, 8192, "dma_128x192"),
+                                         (384, 2056, 8188, "dma_128x192"), (385, 2056, 8192, "dma8w_128x256"),
+                                         (511, 2048, 7172, "dma8w_128x256"), (576, 2048, 5120, "dma_128x192")])
+def test_gateup_tiles_that_fill_one_round(capi, M, K, ff, name):
+    """129 rows and more on the tile whose launch has at most 256 workgroups: both sides of its rows, two and three tiles of
+    activation rows on the wide kernels, ragged features, K tails; output inside a wider NaN buffer."""
+    assert capi.variant_name(0, 0, M, 2 * ff, K) == name
+    inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + ff, x_scale=0.5)
+    X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
+    wide = torch.full((M, ff + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    capi.gateup(X, W, out=wide[:, :ff])
+    assert torch.isnan(wide[:, ff:]).all()
+    pre = X.double() @ W.double().T
+    ref = (pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2])).cpu()
+    assert_one_rounding(wide[:, :ff], ref, torch.bfloat16, "H %s" % ((M, K, ff),))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows", [160, 192, 224])
 @pytest.mark.parametrize("K", [8, 64, 72, 200, 392, 456, 832])
