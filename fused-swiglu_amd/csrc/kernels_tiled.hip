@@ -13,6 +13,8 @@
 // LDS rows [0, BP/2) receive the even ("up") rows of the weight tile and rows [BP/2, BP) the odd ("gate")
 // rows. A wave then runs two accumulator sets over the same activation fragments, and up/gate of one (m, j)
 // land in the same lane and register index: the gating is plain per-lane fp32 math, no cross-lane traffic.
+#include <math.h>
+
 #include <type_traits>
 
 #include "fsw_internal.h"
@@ -571,6 +573,73 @@ int pair16_tile_rows(bool gated, long long np, long long nq, double need) {
   return rows;
 }
 
+// Down projection of more than 256 rows with fewer than 129 large tiles: estimated time, us, of K split into `sp` parts
+// (1: no split) on 128 x 128 tiles (tile_q 128) or 256 x tile_q ones of relative cost `tile_cost`. Every term was fitted to
+// 2400 timings: the better plans of 346 problems (layers of common width and random ones; d 500 .. 8192, ff 1.5 .. 5 d,
+// 257 .. 6000 rows, bf16 and fp16, weights rotated so that they come from memory): 5 % rms, and the plan it picks is 0.7 % slower
+// than the fastest one on average, 12 % at worst.
+//   * a workgroup's K tiles of 64: 1.19 us on 256 x 256 plus 1.9 us to fill and drain the pipeline (what shallow parts pay
+//     for: 1996 rows of 2088 -> 736 in two parts of 17 tiles 34.4 us on 256 x 160, 22.2 on 128 x 128), 0.6 us on 128 x 128
+//     alone on a compute unit (three stages), 1.6 .. 1.83 times that where 257 .. 512 workgroups share them two by two;
+//   * a round costs the same whether 100 or 256 compute units are in it, but 256 workgroups of eight parts and more take
+//     a fifth longer (4096 x 11008, 426 rows on 256 x 224: seven parts 53.7 us, eight 65.7);
+//   * K no multiple of 64: rows share cache lines, all tiles take 1.22 times as long;
+//   * the weights once from memory at 4.5 TB/s: combined with the above so that the larger one counts;
+//   * parts: fp32 sums written and read back at 5 TB/s, and the summing kernel's launch and one dependent load per part.
+static double split_time(int np, int nq, int k, int tile_q, double tile_cost, int sp) {
+  const long long rows_p = tile_q == 128 ? 128 : 256;
+  const long long wgs = ((np + rows_p - 1) / rows_p) * ((nq + tile_q - 1) / tile_q) * sp;
+  const int kt = ((k + 63) / 64 + sp - 1) / sp;
+  double t;
+  if (tile_q == 128) {
+    t = 0.6 * kt * (wgs <= 256 ? 1.0 : 1.6 + 0.23 * (double)(wgs - 257) / 255.0);
+  } else {
+    t = tile_cost * (1.9 + 1.19 * kt) * (wgs == 256 && sp >= 8 ? 1.2 : 1.0);
+  }
+  if (k % 64 != 0) t *= 1.22;
+  const double w = 2.0 * (double)np * (double)k / 4.5e6;  // us
+  t = sqrt(sqrt(t * t * t * t + w * w * w * w));
+  if (sp > 1) t += 1.6 + 0.34 * sp + 8.0 * sp * (double)nq * (double)np / 5.0e6;
+  return t;
+}
+
+// The fastest plan by split_time() among those that are resident at once (two 128 x 128 workgroups or one large one per
+// compute unit: a second, partly filled round costs a whole one), whose parts are 8 (16) K tiles deep at least and whose
+// partial sums stay under 256 MB. Tiles half filled with rows and row counts that are multiples of 256 need no rule of their own.
+// Down projection, us, with 128 x 128 and 256 x 256 tiles only / with an estimate that knew neither the fill of short parts nor
+// the three-stage ring and left half-filled tiles out / with this one: 28672 -> 8192, 264 rows 170 / 239 / 144; 8192 -> 2048,
+// 371 rows 30.7 / 35.0 / 27.3; 2088 -> 736, 1996 rows 26.0 / 34.5 / 22.5; 3408 -> 1352, 910 rows 28.4 / 34.0 / 27.8; 11104 -> 5904,
+// 479 rows 76.5 / 86.8 / 76.5; 11008 -> 4096, 333 rows 61.7 / 51.9 / 48.4, 1536 rows 133 / 133 / 120; 14336 -> 4096, 1024 rows
+// level at 102. On 302 random problems none of these were fitted to: 0.896 of the first on average (95 % of them below 0.99, worst
+// 1.06), 0.931 of the second (worst 1.02).
+static SplitPlan mid_split_plan(int np, int nq, int k) {
+  static const struct {
+    int rows;
+    double cost;  // of a K tile against 256 x 256
+  } kTiles[] = {{128, 0.0}, {256, 1.0}, {224, 0.926}, {192, 0.863}, {160, 0.797}};
+  SplitPlan p = {128, 1};
+  double best = split_time(np, nq, k, 128, 0.0, 1);
+  for (const auto& t : kTiles) {
+    const bool small = t.rows == 128;
+    const long long rows_p = small ? 128 : 256;
+    const long long nt = ((np + rows_p - 1) / rows_p) * ((nq + t.rows - 1) / t.rows);
+    long long smax = (small ? 512 : 256) / nt;
+    const long long deep = small ? k / 512 : k / 1024;
+    if (smax > deep) smax = deep;
+    if (smax > 16) smax = 16;
+    for (int sp = 2; sp <= (int)smax; ++sp) {
+      if (4.0 * sp * (double)nq * (double)np > 256e6) break;
+      const double cost = split_time(np, nq, k, t.rows, t.cost, sp);
+      if (cost < best) {
+        best = cost;
+        p.tile = t.rows;
+        p.splits = sp;
+      }
+    }
+  }
+  return p;
+}
+
 SplitPlan tiled_split_plan(int np, int nq, int k) {
   const long long t128 = (long long)((np + 127) / 128) * ((nq + 127) / 128);
   const long long t256 = (long long)((np + 255) / 256) * ((nq + 255) / 256);
@@ -579,6 +648,32 @@ SplitPlan tiled_split_plan(int np, int nq, int k) {
   // More rows: splitting can still pay by evening out rounds (288 tiles are two rounds of K, 288 x 3 are four
   // rounds of K / 3), up to 512 tiles.
   if (t128 <= 0 || t256 > (nq > 256 ? 512 : 128)) return p;
+  if (nq > 256 && t256 < 129) return mid_split_plan(np, nq, k);
+  if (nq > 256) {
+    // From 129 large tiles up: the unsplit alternative is the 16x16x32 kernel on blocked H (~8 % faster than on row-major
+    // H, which the split kernel reads), so a split, over several rounds if need be, must win by 15 %; its partials stay under
+    // 256 MB. Estimated time in us on 256 compute units: MFMA work of the busiest one at 5.1 / 0.77 TFLOP/s (see
+    // pair16_rounds() for partly filled rounds) plus the fp32 partials at ~5 TB/s.
+    // Unsplit tiles of fewer rows need no place in the comparison: of 35 problems that split here (256 x 256, us) 34 are
+    // slower on the best of them (28672 -> 8192: 2079 rows 839 -> 888 on 256 x 160, 2419 rows 907 -> 916; 31856 -> 5408, 3060
+    // rows 1078 -> 1165; the forward of 2079 rows of 8192 x 28672 2257 -> 2300), one is faster (31400 -> 6648, 1170 rows 638 -> 581).
+    const int nkt = (k + 63) / 64;
+    double best = 0.0, unsplit = 0.0;
+    p.splits = 1;
+    for (int sp = 1; sp <= 16 && (sp == 1 || sp <= k / 1024); ++sp) {
+      if (sp > 1 && 4.0 * sp * (double)nq * (double)np > 256e6) break;
+      const double kper = 64.0 * ((nkt + sp - 1) / sp);
+      const double mfma = 2.0 * kper * 256 * 256 * 0.77 * pair16_rounds(t256 * sp) / 5.1e6;
+      const double cost = mfma + (sp > 1 ? 8.0 * sp * (double)nq * (double)np / 5.0e6 : 0.0);
+      if (sp == 1) unsplit = mfma;
+      if (best == 0.0 || cost < best) {
+        best = cost;
+        p.splits = sp;
+      }
+    }
+    if (p.splits > 1 && best > 0.85 * unsplit) p.splits = 1;
+    return p;
+  }
   int by_k;
   long long tiles;
   if (t128 < 256) {
@@ -588,62 +683,6 @@ SplitPlan tiled_split_plan(int np, int nq, int k) {
   } else {
     tiles = t256;
     by_k = k / 1024;
-  }
-  if (nq > 256) {
-    // Several tiles of activation rows: all workgroups should be resident at once (two 128 x 128 workgroups or one
-    // 256 x 256 workgroup per compute unit: a second, partly filled round costs a whole one; 640 rows of 4096 x
-    // 14336: 160 tiles x 3 splits 86 us, x 4 splits 110 us), and every split adds a partial tile to write and read
-    // back. Estimated time per candidate, in us on 256 compute units: MFMA work of the busiest compute unit at
-    // ~5.1 TFLOP/s (a lone 128 x 128 workgroup runs at half of that, the small tile costs ~15 % more per flop, the
-    // large one on 16x16x32 MFMAs ~23 % less, see pair16_rounds() for its partly filled rounds) plus the fp32 partials at ~5 TB/s. Measured against it (4096 x 14336):
-    // 257 rows 128/5 59 us, 640 rows 128/3 85 us, 1024 rows 256/4 106 us, 2048 rows 256/2 185 us, each within 5 % of
-    // the fastest of 12 tile/split pairs tried.
-    // From 129 large tiles up the unsplit alternative is the 16x16x32 kernel on blocked H (~8 % faster than on
-    // row-major H, which the split kernel reads): there only large-tile splits are candidates, over several rounds
-    // if need be, they must win by 15 %, and their partials stay under 256 MB.
-    // Below 129 large tiles the large tile comes in four heights (kNarrow); it is a candidate where 55 % of its rows are
-    // used, a narrow one where 85 % are and 256-row tiles would not be full. Down 11008 -> 4096, us, without -> with narrow
-    // tiles: 300 rows 56.0 -> 43.2 (160 x 6 splits), 333 rows 55.8 -> 45.8 (192 x 6), 640 rows 66.6 -> 57.3 (160 x 4), 1300
-    // rows 111.8 -> 98.9 (192 x 2); 28672 -> 8192, 520 rows 288 -> 249 (192 x 2).
-    const int nkt = (k + 63) / 64;
-    const bool large = t256 >= 129;
-    double best = 0.0, unsplit = 0.0;
-    p.tile = 128;
-    p.splits = 1;
-    for (int c = large ? 0 : -1; c < 4; ++c) {  // -1: 128 x 128, 0 .. 3: kNarrow
-      const bool small = c < 0;
-      const int tile_q = small ? 128 : kNarrow[c].rows;
-      const long long nt = small ? t128 : (long long)((np + 255) / 256) * ((nq + tile_q - 1) / tile_q);
-      const long long padded = (long long)((nq + tile_q - 1) / tile_q) * tile_q;
-      if (c == 0 && !large && 20LL * nq < 11 * padded) continue;
-      if (c > 0 && (large || nq % 256 == 0 || 20LL * nq < 17 * padded)) continue;
-      const long long slots = small ? 512 : 256;
-      long long smax = large ? 16 : slots / nt;
-      const long long deep = small ? k / 512 : k / 1024;  // at least 8 (16) K tiles of 64 per partition
-      if (smax > deep) smax = deep;
-      if (smax > 16) smax = 16;
-      if (smax < 1) smax = 1;
-      for (int sp = 1; sp <= (int)smax; ++sp) {
-        if (sp > 1 && 4.0 * sp * (double)nq * (double)np > 256e6) break;
-        if (sp == 1 && !large && tile_q != 128 && tile_q != 256) continue;  // unsplit: 128 x 128 below
-        const double kper = 64.0 * ((nkt + sp - 1) / sp);
-        const long long wgs = nt * sp;
-        const double rounds = small ? (double)((wgs + slots - 1) / slots) : pair16_rounds(wgs);
-        const double tile_cost = small ? 2.0 * kper * 128 * 128 * 2.0 * 1.15 : 2.0 * kper * 256 * 256 * 0.77 * kNarrow[c].cost;
-        const double mfma = tile_cost * rounds / 5.1e6;
-        const double partials = sp > 1 ? 8.0 * sp * (double)nq * (double)np / 5.0e6 : 0.0;
-        if (sp == 1 && !small && (unsplit == 0.0 || mfma < unsplit)) unsplit = mfma;
-        const double cost = (c > 0 ? 1.05 : 1.0) * (mfma + partials);  // the estimates are no closer than 5 %
-        if (best == 0.0 || cost < best) {
-          best = cost;
-          p.tile = tile_q;
-          p.splits = sp;
-        }
-      }
-    }
-    if (large && p.splits > 1 && best > 0.85 * unsplit) p.splits = 1;
-    if (p.splits == 1) p.tile = large ? 256 : 128;  // unsplit mid-size problems keep the smaller tile
-    return p;
   }
   // One tile of activation rows: three-stage workgroups, one per compute unit, beat two two-stage ones (less
   // partial-sum traffic as well); 129..256 rows take one 128 x 256 tile per workgroup for the same reason.

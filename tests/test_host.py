@@ -174,7 +174,7 @@ def test_variant_choice_by_regime(capi):
     assert name(0, 256, 28672, 4096) == "dma8w_128x256"
     assert name(1, 128, 4096, 14336) == "splitk_dma_128x128" and ws(0, 128, 4096, 14336) == 8 * 128 * 4096 * 4
     # above 256 rows: as many splits as keep all workgroups resident at once, on the tile the time estimate favours
-    assert name(1, 257, 4096, 14336) == "splitk_dma_128x128" and ws(0, 257, 4096, 14336) == 5 * 257 * 4096 * 4
+    assert name(1, 257, 4096, 14336) == "splitk_pair16_256x160" and ws(0, 257, 4096, 14336) == 7 * 257 * 4096 * 4
     assert name(1, 1024, 4096, 14336) == "splitk_pair16_256x256" and ws(0, 1024, 4096, 14336) == 4 * 1024 * 4096 * 4
     assert name(1, 2048, 4096, 14336) == "splitk_pair16_256x256" and ws(0, 2048, 4096, 14336) == 2 * 2048 * 4096 * 4
     assert name(1, 2304, 4096, 14336) == "pair16_256x256"    # 144 large tiles in one round: no split
@@ -187,6 +187,20 @@ def test_variant_choice_by_regime(capi):
     assert L.fsw_mlp_workspace_bytes(0, 8192, 4096, 14336) == L.fsw_blocked_bytes(8192, 14336) == 8192 * 14336 * 2
     assert L.fsw_mlp_workspace_bytes(0, 3000, 4096, 14336) == L.fsw_blocked_bytes(3000, 14336)
     assert capi.lib().fsw_mlp_workspace_bytes(0, 256, 4096, 14336) == 256 * 14336 * 2 + ws(0, 256, 4096, 14336)
+
+
+@pytest.mark.parametrize("M,D,FF,want,splits", [
+    (264, 8192, 28672, "splitk_pair16_256x160", 4),     # one half-filled row of large tiles, many weights
+    (371, 2048, 8192, "splitk_dma_128x128", 5),         # parts of 16 K tiles: small tiles alone on a compute unit
+    (910, 1352, 3408, "splitk_dma_128x128", 2), (1996, 736, 2088, "splitk_dma_128x128", 2),
+    (479, 5904, 11104, "splitk_pair16_256x256", 5),
+    (896, 4096, 4096, "dma_128x128", 0),                # an unsplit launch beats two parts
+    (768, 8192, 28672, "splitk_pair16_256x192", 2), (1536, 4096, 11008, "splitk_pair16_256x192", 2)])
+def test_split_plan_counts_the_fill_of_short_parts(capi, M, D, FF, want, splits):
+    """Down projections that lost 8 .. 41 % to plans of narrow tiles with too few K tiles per part, of half-filled rows of
+    tiles left out, or (the last two) of narrow tiles left out because the row count was a multiple of 256."""
+    assert capi.variant_name(1, 0, M, D, FF) == want
+    assert capi.lib().fsw_down_workspace_bytes(0, M, D, FF) == splits * M * D * 4
 
 
 def test_variant_override_is_per_thread(capi):

@@ -720,8 +720,8 @@ def test_split_k_of_at_most_64_rows(capi, M, D, FF, dtype):
     assert_one_rounding(wide[:, :D], H.double() @ W2.double().T, dtype, "split %s" % ((M, D, FF),))
 
 
-NARROW_SPLITS = [(435, 4096, 8192, 160), (300, 4096, 8200, 160), (520, 4096, 3072, 192), (520, 2048, 8200, 192),
-                 (400, 4096, 8192, 224), (400, 4096, 8200, 224)]
+NARROW_SPLITS = [(435, 4096, 8192, 160), (300, 4096, 8200, 160), (768, 4096, 6144, 192), (516, 4096, 8200, 192),
+                 (887, 4096, 6144, 224), (672, 4096, 8200, 224)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
