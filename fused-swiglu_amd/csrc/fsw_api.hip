@@ -95,8 +95,7 @@ int pick_tiled(int family, int64_t m, int64_t np, int64_t k, double narrow_need 
     // up to 64 rows the gate/up tile is 128 x 64 (4096 x 28672, M = 48: 39.4 -> 37.2 us)
     return (family == 0 && m <= 64) ? V_128x64 : V_128x128;
   }
-  // (the down projection of a multiple of 256 rows keeps the kernel it always had there)
-  const int rows = family == 1 && m % 256 == 0 ? 256 : fsw::pair16_tile_rows(family == 0, np, m, narrow_need);
+  const int rows = fsw::pair16_tile_rows(family == 0, np, m, narrow_need);
   if (rows != 256) return VARIANT_NARROW + rows / 32;
   if (family == 0 && tiles256 > 256 && tiles256 <= 512) {
     // A few large tiles more than compute units: the second round is nearly empty, while 128 x 128 tiles (two per

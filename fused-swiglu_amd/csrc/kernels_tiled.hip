@@ -558,6 +558,8 @@ static const NarrowTile kNarrow[] = {{256, 1.0}, {224, 0.91}, {192, 0.81}, {160,
 // 256 -> best, us: gate/up 4096 x 28672: 300 rows 78 -> 57 (160), 333 rows 79 -> 63 (192), 448 rows 85 -> 77 (224),
 // 640 rows 150 -> 112 (160), 1000 rows stay (168, narrow 193 or more); 8192 x 57344, 520 rows 472 -> 412 (192); down
 // 11008 -> 4096: 2500 rows 173 -> 153 (160), 3000 rows 191 -> 177 (192), 4300 rows 379 -> 282 (160).
+// Rounds decide, not only padding, so row counts that 256 divides gain as well: 11008 -> 4096: 2304 rows 210 -> 169 (160), 2560
+// rows 212 -> 180 (160), 3072 rows 217 -> 199 (192), 4352 rows 408 -> 322 (160); 8192 x 28672, forward of 1280 rows 1371 -> 1332.
 int pair16_tile_rows(bool gated, long long np, long long nq, double need) {
   const long long tp = (np + 255) / 256;
   if (tp * ((nq + 255) / 256) > (gated ? 1024 : 512)) return 256;

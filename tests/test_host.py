@@ -177,7 +177,7 @@ def test_variant_choice_by_regime(capi):
     assert name(1, 257, 4096, 14336) == "splitk_pair16_256x160" and ws(0, 257, 4096, 14336) == 7 * 257 * 4096 * 4
     assert name(1, 1024, 4096, 14336) == "splitk_pair16_256x256" and ws(0, 1024, 4096, 14336) == 4 * 1024 * 4096 * 4
     assert name(1, 2048, 4096, 14336) == "splitk_pair16_256x256" and ws(0, 2048, 4096, 14336) == 2 * 2048 * 4096 * 4
-    assert name(1, 2304, 4096, 14336) == "pair16_256x256"    # 144 large tiles in one round: no split
+    assert name(1, 2304, 4096, 14336) == "pair16_256x160"    # 240 tiles of 160 rows in one round: no split
     # 288 large tiles of a very deep K: three splits (four rounds of K / 3 instead of two of K), H stays row-major
     assert name(1, 2049, 8192, 28672) == "splitk_pair16_256x256" and ws(0, 2049, 8192, 28672) == 3 * 2049 * 8192 * 4
     # large-tile regime: fsw_down reads row-major H in whole cache lines and needs no scratch; fsw_gateup never does;
@@ -201,6 +201,21 @@ def test_split_plan_counts_the_fill_of_short_parts(capi, M, D, FF, want, splits)
     tiles left out, or (the last two) of narrow tiles left out because the row count was a multiple of 256."""
     assert capi.variant_name(1, 0, M, D, FF) == want
     assert capi.lib().fsw_down_workspace_bytes(0, M, D, FF) == splits * M * D * 4
+
+
+@pytest.mark.parametrize("M,D,FF,want,blocked", [
+    (2304, 4096, 11008, "pair16_256x160", False), (4352, 4096, 11008, "pair16_256x160", False),
+    (1280, 8192, 28672, "pair16_256x160", False),
+    (3072, 4096, 11008, "pair16_256x192", True),  # 8 % of the down kernel: less than blocked H is asked for
+    (4096, 4096, 11008, "pair16_256x256", True), (8192, 4096, 14336, "pair16_256x256", True)])
+def test_multiples_of_256_rows_take_the_tile_of_their_neighbours(capi, M, D, FF, want, blocked):
+    """Partly filled rounds do not depend on padding: M - 1 and M rows run the same down projection, and the forward keeps H
+    row-major where the narrow tile gains enough, blocked otherwise."""
+    assert capi.variant_name(1, 0, M, D, FF) == want == capi.variant_name(1, 0, M - 1, D, FF)
+    L = capi.lib()
+    for m in (M - 1, M):
+        assert L.fsw_mlp_workspace_bytes(0, m, D, FF) == (L.fsw_blocked_bytes(m, FF) if blocked else
+                                                          (m * FF * 2 + 255) // 256 * 256)
 
 
 def test_variant_override_is_per_thread(capi):

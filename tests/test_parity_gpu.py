@@ -998,7 +998,8 @@ def test_mlp_large_tile_regime_uses_blocked_path(capi):
     assert torch.equal(Y4, capi.down(capi.gateup(g["X"], g["W13"]), g["W2"]))
 
 
-@pytest.mark.parametrize("shape", [(16, 512, 1024), (96, 512, 1024), (600, 1024, 520), (2304, 4096, 2048)])
+@pytest.mark.parametrize("shape", [(16, 512, 1024), (96, 512, 1024), (600, 1024, 520), (2304, 4096, 2048),
+                                   (8192, 2048, 1024)])
 def test_forward_replays_from_a_hip_graph(capi, shape):
     """fsw_mlp enqueues kernels only (no allocation, no synchronisation, no memset), so a caller can capture it into a
     HIP graph. Every replay — with eager work and synchronisations of the program in between, and with new contents
@@ -1024,6 +1025,29 @@ def test_forward_replays_from_a_hip_graph(capi, shape):
         torch.cuda.synchronize()
         assert torch.equal(Y, eager), "replay %d differs from the eager forward" % rep
     oracle.assert_parity(Y, oracle.ref_mlp(X.cpu(), inp["W13"], inp["W2"], torch.float64), "graph replay")
+
+
+@pytest.mark.parametrize("M,d,ff,gate,down", [(2300, 4096, 3584, "pair16_256x256", "pair16_256x160"),
+                                              (2700, 4096, 3592, "pair16_256x160", "pair16_256x192"),
+                                              (2304, 4096, 2048, "pair16_256x160", "pair16_256x160")])
+def test_forward_with_a_narrow_down_projection(capi, M, d, ff, gate, down):
+    """What the dispatcher picks by itself for the forward: a down projection on narrow tiles reads row-major H, so the gate/up
+    kernel writes it so and the scratch is H alone. Against float64, Y inside a wider NaN buffer."""
+    assert capi.variant_name(0, 0, M, 2 * ff, d) == gate and capi.variant_name(2, 0, M, d, ff) == down
+    assert capi.lib().fsw_mlp_workspace_bytes(0, M, d, ff) == (2 * M * ff + 255) // 256 * 256
+    gen = torch.Generator(device=DEV).manual_seed(M + ff)
+    X = torch.randn(M, d, generator=gen, device=DEV).to(torch.bfloat16)
+    W13 = (torch.randn(2 * ff, d, generator=gen, device=DEV) / d ** 0.5).to(torch.bfloat16)
+    W2 = (torch.randn(d, ff, generator=gen, device=DEV) / ff ** 0.5).to(torch.bfloat16)
+    wide = torch.full((M, d + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    Y = capi.mlp(X, W13, W2, out=wide[:, :d])
+    assert torch.isnan(wide[:, d:]).all()
+    H = capi.gateup(X, W13)
+    assert torch.equal(Y, capi.down(H, W2))
+    pre = X.double() @ W13.double().T
+    ref_h = pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2])
+    assert_one_rounding(H, ref_h.cpu(), torch.bfloat16, "H %s" % ((M, d, ff),))
+    assert_one_rounding(Y, (H.double() @ W2.double().T).cpu(), torch.bfloat16, "Y %s" % ((M, d, ff),))
 
 
 def test_large_tiles_on_row_major_activations(capi):
