@@ -251,7 +251,7 @@ const char* fsw_variant_name(int family, int dtype, int64_t M, int64_t N_or_D, i
       K_or_FF <= MAX_DIM) {
     const fsw::SplitPlan plan = fsw::tiled_split_plan((int)N_or_D, (int)M, (int)K_or_FF);
     if (plan.splits > 1) {
-      if (plan.tile == 128) return "splitk_dma_128x128";
+      if (plan.tile == 128) return M <= 64 ? "splitk_dma_128x64" : "splitk_dma_128x128";  // see launch_tiled_splitk
       if (plan.tile == 129) return "splitk_dma_128x256";
       if (plan.tile == 130) return "splitk_dma_128x192";
       if (plan.tile == 160) return "splitk_pair16_256x160";

@@ -143,7 +143,7 @@ def test_variant_choice_by_regime(capi):
     assert name(0, 8, 28672, 4096) == "skinny" and name(1, 1, 4096, 14336) == "skinny"
     # the weight-streaming kernels take fewer rows the larger the weights: up to 48 / 32 / 16 rows
     assert name(0, 32, 22016, 4096) == "skinny" and name(1, 32, 4096, 14336) == "skinny"
-    assert name(0, 33, 28672, 4096) == "dma_128x64" and name(1, 33, 4096, 14336) == "splitk_dma_128x128"
+    assert name(0, 33, 28672, 4096) == "dma_128x64" and name(1, 33, 4096, 14336) == "splitk_dma_128x64"
     assert name(0, 48, 2 * 8192, 2048) == "skinny" and name(0, 49, 2 * 8192, 2048) == "dma_128x64"
     # gate/up with 200 .. 256 tiles of 128 weight rows and a dozen rows or more: the 128 x 64 tiled kernel streams faster
     assert name(0, 16, 28672, 4096) == "dma_128x64" and name(0, 11, 28672, 4096) == "skinny"
@@ -187,6 +187,11 @@ def test_variant_choice_by_regime(capi):
     assert L.fsw_mlp_workspace_bytes(0, 8192, 4096, 14336) == L.fsw_blocked_bytes(8192, 14336) == 8192 * 14336 * 2
     assert L.fsw_mlp_workspace_bytes(0, 3000, 4096, 14336) == L.fsw_blocked_bytes(3000, 14336)
     assert capi.lib().fsw_mlp_workspace_bytes(0, 256, 4096, 14336) == 256 * 14336 * 2 + ws(0, 256, 4096, 14336)
+
+
+@pytest.mark.parametrize("M,want", [(33, "splitk_dma_128x64"), (64, "splitk_dma_128x64"), (65, "splitk_dma_128x128")])
+def test_split_plan_names_the_tile_that_runs(capi, M, want):
+    assert capi.variant_name(1, 0, M, 4096, 14336) == capi.variant_name(2, 0, M, 4096, 14336) == want
 
 
 @pytest.mark.parametrize("M,D,FF,want,splits", [

@@ -710,7 +710,7 @@ def test_narrow_tiles_give_the_bits_of_256_row_tiles(capi, rows, dtype, K):
 def test_split_k_of_at_most_64_rows(capi, M, D, FF, dtype):
     """The split-K down projection on 128 x 64 tiles (four stages): full and ragged rows and features, K with and without
     a tail, parts of a few K tiles. Output inside a wider NaN buffer."""
-    assert capi.variant_name(1, 0, M, D, FF) == "splitk_dma_128x128"
+    assert capi.variant_name(1, 0, M, D, FF) == "splitk_dma_128x64"
     gen = torch.Generator().manual_seed(M + FF)
     H = (torch.randn(M, FF, generator=gen) * 0.5).to(dtype)
     W2 = (torch.randn(D, FF, generator=gen) / FF ** 0.5).to(dtype)
