@@ -237,11 +237,13 @@ int fsw_set_variant(int family, int variant) {
 }
 
 static fsw::StreamPlan mlp_stream_plan(int64_t M, int64_t D, int64_t FF);
+static bool blocked_regime(int64_t M, int64_t D, int64_t FF, size_t scratch);
 
 const char* fsw_variant_name(int family, int dtype, int64_t M, int64_t N_or_D, int64_t K_or_FF) {
   (void)dtype;
   if (family == 2) {  // the down projection as fsw_mlp runs it
     if (mlp_stream_plan(M, N_or_D, K_or_FF).splits > 1) return "stream_split";
+    if (blocked_regime(M, N_or_D, K_or_FF, SIZE_MAX)) return fsw::tiled_variant(V_256x256).name;
     family = 1;
   }
   if (family < 0 || family > 1) return "invalid";

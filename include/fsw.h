@@ -219,7 +219,8 @@ FSW_API int fsw_decode_barrier_failures(void);
 
 /* Name of the kernel variant the dispatcher picks for this shape (static storage); "splitk_<kernel>" when the
  * down projection splits K (family 1; K_or_FF decides). family 2: the down projection as fsw_mlp runs it (differs
- * from family 1, which is fsw_down on its own, for 17 .. 32 rows: "stream_split"). */
+ * from family 1, which is fsw_down on its own, for 17 .. 32 rows: "stream_split", and where H stays panel-blocked:
+ * "pair16_256x256" also for row counts that fsw_down runs on narrower tiles). */
 FSW_API const char* fsw_variant_name(int family, int dtype, int64_t M, int64_t N_or_D, int64_t K_or_FF);
 
 #ifdef __cplusplus

@@ -217,6 +217,7 @@ def test_multiples_of_256_rows_take_the_tile_of_their_neighbours(capi, M, D, FF,
     """Partly filled rounds do not depend on padding: M - 1 and M rows run the same down projection, and the forward keeps H
     row-major where the narrow tile gains enough, blocked otherwise."""
     assert capi.variant_name(1, 0, M, D, FF) == want == capi.variant_name(1, 0, M - 1, D, FF)
+    assert capi.variant_name(2, 0, M, D, FF) == ("pair16_256x256" if blocked else want)  # as the forward runs it
     L = capi.lib()
     for m in (M - 1, M):
         assert L.fsw_mlp_workspace_bytes(0, m, D, FF) == (L.fsw_blocked_bytes(m, FF) if blocked else
