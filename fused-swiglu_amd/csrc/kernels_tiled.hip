@@ -469,10 +469,12 @@ int raster_group(bool gated, int tiles_q) { return gated ? 4 : (tiles_q >= 32 ? 
 namespace {
 
 // The 128-row instances stream their weights non-temporally when at most two tiles of activation rows share them and weight
-// rows are whole 128-byte lines (ldp a multiple of 64). Otherwise a line at the edge of a 128-byte piece of a row serves two
-// consecutive K tiles and has to stay in the cache between them: non-temporal -> default policy, us: gate/up 3000 x 16016 at
-// 130 rows 51.7 -> 31.5, 4104 x 28000 at 100 rows 66.1 -> 41.7, 5000 x 32016 at 64 rows 82.2 -> 71.6; down 8008 -> 3000 at 64
-// rows 23.3 -> 17.2, 28680 -> 8192 at 100 rows 153 -> 129; forward 3000 x 8008 fp16 at 200 rows 83.3 -> 61.4.
+// rows are whole 128-byte lines (ldp a multiple of 64, the matrix on a line). Otherwise a line at the edge of a 128-byte piece of a
+// row serves two consecutive K tiles and has to stay in the cache between them: non-temporal -> default policy, us, weights that
+// repeat from call to call: gate/up 3000 x 16016 at 130 rows 51.7 -> 31.5, 4104 x 28000 at 100 rows 66.1 -> 41.7, 5000 x 32016 at
+// 64 rows 82.2 -> 71.6; down 8008 -> 3000 at 64 rows 23.3 -> 17.2, 28680 -> 8192 at 100 rows 153 -> 129. Weights that come from
+// memory, the matrix 16 bytes past a line: gate/up 5120 x 27648 at 40 rows 69.8 -> 63.8, 4096 x 28672 at 64 rows 56.3 -> 52.4 and
+// at 200 rows 80.4 -> 76.4; down 14336 -> 4096 at 64 rows 38.4 -> 33.4.
 // Ring length: a launch of at most 256 workgroups has a compute unit to itself per workgroup, so nothing else hides
 // the latency of its copies and the LDS is free: three stages (four of the small 128 x 64 ones), copies two (three) K
 // tiles ahead. Two stages -> three, us: gate/up fp16 3000 x 16016 at 200 rows (252 workgroups) 68 -> 57, whole forward
@@ -486,7 +488,7 @@ void launch_dma_kernel(const dim3 grid, hipStream_t stream, const GemmArgs& a, i
   constexpr int DEEP = WQ * FQ == 2 ? 4 : 3;
   const dim3 block(WP * WQ * 64);
   const bool deep = (long long)grid.x * grid.y <= 256 || (WQ * FQ >= 6 && tiles_q == 1);
-  if (tiles_q <= 2 && a.ldp % 64 == 0) {
+  if (tiles_q <= 2 && a.ldp % 64 == 0 && ((uintptr_t)a.P & 127) == 0) {
     if (deep) {
       hipLaunchKernelGGL((tiled_dma_kernel<E, GATED, KTAIL, WP, WQ, FP, FQ, true, DEEP>), grid, block, 0, stream, a,
                          tiles_p, tiles_q, group);

@@ -720,6 +720,29 @@ def test_split_k_of_at_most_64_rows(capi, M, D, FF, dtype):
     assert_one_rounding(wide[:, :D], H.double() @ W2.double().T, dtype, "split %s" % ((M, D, FF),))
 
 
+@pytest.mark.parametrize("M", [40, 64, 100, 130, 200, 300])
+@pytest.mark.parametrize("off,pad", [(8, 0), (56, 64), (0, 8)])
+def test_weights_that_are_no_whole_cache_lines(capi, M, off, pad):
+    """K a multiple of 64, but the weight matrix starts 16 or 112 bytes past a line or its rows are 16 bytes longer than whole
+    lines (NaN behind them): the copies take the default cache policy without a K tail. Both projections."""
+    d, ff = 320, 4160
+    inp = fsw_weights.make_inputs(M, d, ff, torch.bfloat16, seed=M + off + pad, x_scale=0.5)
+    H0 = (torch.randn(M, ff, generator=torch.Generator().manual_seed(M)) * 0.5).to(torch.bfloat16)
+
+    def placed(W):
+        rows, cols = W.shape
+        flat = torch.full((rows * (cols + pad) + 64,), float("nan"), dtype=W.dtype, device=DEV)
+        assert flat.data_ptr() % 128 == 0
+        view = flat[off:off + rows * (cols + pad)].view(rows, cols + pad)[:, :cols]
+        view.copy_(W)
+        return view
+
+    H = capi.gateup(inp["X"].to(DEV), placed(inp["W13"]))
+    assert_one_rounding(H, oracle.ref_gateup(inp["X"], inp["W13"], torch.float64), torch.bfloat16, "H %s" % ((M, off, pad),))
+    Y = capi.down(H0.to(DEV), placed(inp["W2"]))
+    assert_one_rounding(Y, H0.double() @ inp["W2"].double().T, torch.bfloat16, "Y %s" % ((M, off, pad),))
+
+
 NARROW_SPLITS = [(435, 4096, 8192, 160), (300, 4096, 8200, 160), (768, 4096, 6144, 192), (516, 4096, 8200, 192),
                  (887, 4096, 6144, 224), (672, 4096, 8200, 224)]
 
