@@ -76,7 +76,7 @@ int pick_tiled(int family, int64_t m, int64_t np, int64_t k, double narrow_need 
     // Up to 192 rows the tile is 128 x 192: the single-tile kernels are bound by their MFMA and LDS work as much as
     // by the weight stream (4096 x 28672, M = 160: 65 -> 54 us; 5120 x 27648: 89 -> 68 us).
     // 193 .. 256 rows: 128 x 256 on 8 waves, two per SIMD (4096 x 28672: 72 -> 64 us, 5120 x 27648: 94 -> 79-87 us
-    // against the 4-wave instance, variant 1).
+    // against 4 waves).
     // All that only where two 128-row tiles are more workgroups than compute units: up to 256 workgroups 128 x 128 tiles
     // have three stages each and a compute unit to themselves (4096 x 16384: M = 129 47.6 -> 41.8 us, M = 256 54.9 -> 45.9;
     // 2048 x 16384: M = 200 29.3 -> 23.2).
@@ -87,7 +87,7 @@ int pick_tiled(int family, int64_t m, int64_t np, int64_t k, double narrow_need 
     // short K (1024 x 16384, M = 384: 17.1 -> 18.5).
     const int64_t tp = (np + 127) / 128;
     if (family == 0 && m > 128 && tp * ((m + 127) / 128) > 256) {
-      if (m <= 256 && tp >= 128) return m <= 192 ? V_128x192 : V_8W_128x256;
+      if (m <= 256) return m <= 192 ? V_128x192 : V_8W_128x256;
       const int64_t w192 = tp * ((m + 191) / 192), w256 = tp * ((m + 255) / 256);
       if (k >= 2048 && w192 >= 224 && w192 <= 256) return V_128x192;
       if (k >= 2048 && w256 >= 224 && w256 <= 256) return V_8W_128x256;
@@ -143,7 +143,7 @@ int resolve_variant(int family, int64_t m, int64_t np, int64_t k) {
     return m <= 64 ? VARIANT_SKINNY : pick_tiled(family, m, np, k);
   if (forced >= 0 && !(forced == VARIANT_SKINNY && m > 64)) return forced;
   if (m <= decode_rows(family, np, k)) {  // decode and small batches: weight streaming, HBM bound
-    // The gate/up product streams its weights faster through the three-stage 128 x 64 tiled kernel (direct-to-LDS
+    // The gate/up product streams its weights faster through the four-stage 128 x 64 tiled kernel (direct-to-LDS
     // copies) than through the weight-streaming kernel when its tiles of 128 weight rows fill one round of compute
     // units and there are a dozen rows or more (gate/up, us: 4096 x 28672: M = 16 37.9 -> 35.6, 32 43.3 -> 36.0, M = 1
     // level; 5120 x 27648: M = 16 49.3 -> 47.3, M = 4 45.3 -> 47.2; 172 tiles of 4096 x 22016: 28.8 -> 33.7, no).

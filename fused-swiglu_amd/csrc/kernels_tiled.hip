@@ -167,13 +167,12 @@ tiled_dma_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const i
   constexpr int STAGE = (BP + BQ) * ROWB;
   static_assert(BP % RSTEP == 0 && BQ % RSTEP == 0 && RSTEP % 16 == 0, "copy mapping");
   static_assert(!GATED || (FP % 2 == 0), "gated kernel pairs fragments");
-  static_assert(NS >= 2 && NS <= 5 && NS * STAGE <= 160 * 1024, "LDS budget of a gfx950 CU");
+  static_assert(NS >= 2 && NS <= 4 && NS * STAGE <= 160 * 1024, "LDS budget of a gfx950 CU");
 
   __shared__ __align__(1024) unsigned char lds0[STAGE];
   __shared__ __align__(1024) unsigned char lds1[STAGE];
   __shared__ alignas(NS > 2 ? 1024 : 16) unsigned char lds2[NS > 2 ? STAGE : 16];
   __shared__ alignas(NS > 3 ? 1024 : 16) unsigned char lds3[NS > 3 ? STAGE : 16];
-  __shared__ alignas(NS > 4 ? 1024 : 16) unsigned char lds4[NS > 4 ? STAGE : 16];
 
   const int t = threadIdx.x;
   const int lane = t & 63;
@@ -348,7 +347,7 @@ tiled_dma_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const i
     }
     if (kt < nkt) iteration(lds0, lds1, kt);
   } else {
-    unsigned char* const ring[5] = {lds0, lds1, lds2, lds3, lds4};
+    unsigned char* const ring[4] = {lds0, lds1, lds2, lds3};
     constexpr int VM = (NS - 2) * NL;
     static_assert(VM <= 63, "vmcnt is a 6-bit counter");
     constexpr int WAIT_IMM = (VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (0 << 8);
@@ -449,9 +448,9 @@ namespace {
 
 const TiledVariant kVariants[] = {
     {"dma_128x128", 128, 128, 256},    // two- or three-stage direct-to-LDS copies, 4 waves of 64 x 64
-    {"dma_128x256", 128, 256, 256},    // 129 .. 256 activation rows in ONE tile: every weight byte is read once
-    {"dma_128x192", 128, 192, 256},    // the same for 129 .. 192 rows
-    {"dma8w_128x256", 128, 256, 512},  // 128 x 256 on 8 waves (two per SIMD), wave tile 64 x 64
+    {"dma8w_128x256", 128, 256, 512},  // id 3 under an older number (a form on 4 waves had it: 72 against 64 us)
+    {"dma_128x192", 128, 192, 256},    // 129 .. 192 activation rows in ONE tile: every weight byte is read once
+    {"dma8w_128x256", 128, 256, 512},  // the same for 193 .. 256 rows, on 8 waves (two per SIMD), wave tile 64 x 64
     {"dma_128x64", 128, 64, 256},      // up to 64 activation rows in one tile
     {"pair16_256x256", 256, 256, 256}, // v_mfma_f32_16x16x32 prefill kernel (kernels_pair16.hip), row-major operands
 };
@@ -481,13 +480,12 @@ namespace {
 // 92.1 -> 82.9; forward 512 rows of 1024 x 2816 29.8 -> 24.2; gate/up 250 rows of 1024 x 5632 17.7 -> 12.9; a fourth and
 // fifth stage of 32 KB: level. 128 x 64, three -> four stages: gate/up 64 rows of 4096 x 22016 34.3 -> 32.2.
 // More workgroups than compute units keep two stages and two workgroups per compute unit (8192 x 57344 at 65 rows,
-// 448 workgroups: 168 us with three stages, 158 with two), except the wide tiles, whose stages leave no room for a second
-// workgroup anyway.
+// 448 workgroups: 168 us with three stages, 158 with two).
 template <class E, bool GATED, bool KTAIL, int WP, int WQ, int FP, int FQ>
 void launch_dma_kernel(const dim3 grid, hipStream_t stream, const GemmArgs& a, int tiles_p, int tiles_q, int group) {
   constexpr int DEEP = WQ * FQ == 2 ? 4 : 3;
   const dim3 block(WP * WQ * 64);
-  const bool deep = (long long)grid.x * grid.y <= 256 || (WQ * FQ >= 6 && tiles_q == 1);
+  const bool deep = (long long)grid.x * grid.y <= 256;
   if (tiles_q <= 2 && a.ldp % 64 == 0 && ((uintptr_t)a.P & 127) == 0) {
     if (deep) {
       hipLaunchKernelGGL((tiled_dma_kernel<E, GATED, KTAIL, WP, WQ, FP, FQ, true, DEEP>), grid, block, 0, stream, a,
@@ -525,8 +523,8 @@ template <class E, bool GATED>
 hipError_t launch_variant(int variant, const GemmArgs& a, hipStream_t stream) {
   switch (variant) {
     case 0: return launch_dma<E, GATED, 2, 2, 2, 2>(a, stream);
-    case 1: return launch_dma<E, GATED, 2, 2, 2, 4>(a, stream);
     case 2: return launch_dma<E, GATED, 2, 2, 2, 3>(a, stream);
+    case 1:
     case 3: return launch_dma<E, GATED, 2, 4, 2, 2>(a, stream);
     case 4: return launch_dma<E, GATED, 2, 2, 2, 1>(a, stream);
     default: return hipErrorInvalidValue;

@@ -188,7 +188,7 @@ FSW_API int fsw_version(void);
  * Kernel-selection override for tests and tuning, PER CALLING THREAD (thread-local): it changes the kernel choice
  * of later calls made by the same thread only, so a thread's fsw_*_workspace_bytes() queries and the launches
  * that follow them always agree. family: 0 = gate/up, 1 = down; variant < 0 restores the automatic choice by
- * shape; 0 .. 5 force one tiled kernel (dma_128x128, dma_128x256, dma_128x192, dma8w_128x256, dma_128x64,
+ * shape; 0 .. 5 force one tiled kernel (dma_128x128, dma8w_128x256, dma_128x192, dma8w_128x256 again, dma_128x64,
  * pair16_256x256; a forced kernel runs unsplit and needs no scratch); 100 is the weight-streaming kernel (honoured
  * for M <= 64; the dispatcher itself picks it up to 16 .. 48 rows, the larger the weights the fewer); 102 is the
  * persistent streaming kernel (honoured for M <= 16; automatic only for d * ff >= 2^27); family 0 variant 101

@@ -9,7 +9,7 @@ from oracle import oracle
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-# gate/up kernels by fsw_set_variant id: automatic, the six tiled instances, the weight-streaming kernel and the
+# gate/up kernels by fsw_set_variant id: automatic, the tiled kernels (1 is 3), the weight-streaming kernel and the
 # persistent streaming kernel (the last two take at most 64 and 16 rows)
 GATEUP_VARIANTS = [-1, 0, 1, 2, 3, 4, 5, 100, 102]
 
