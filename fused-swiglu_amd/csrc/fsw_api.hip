@@ -83,8 +83,10 @@ int pick_tiled(int family, int64_t m, int64_t np, int64_t k, double narrow_need 
     // The same limit above 256 rows: 257 .. 512 workgroups of 128 x 128 share compute units two by two and keep two stages,
     // so the wider tile whose launch fills one round (224 .. 256 workgroups) is taken (4096 x 16384: M = 257 66.6 -> 50.6 us
     // and M = 384 72.7 -> 58.7 on 128 x 192, M = 450 75.3 -> 61.5 and M = 512 79.0 -> 64.6 on 128 x 256; 2048 x 16384: M =
-    // 384 37.9 -> 31.3). Not with fewer workgroups (2048 x 11264, M = 512, 176 wide ones: 29.5 -> 31.7) and not with a
-    // short K (1024 x 16384, M = 384: 17.1 -> 18.5).
+    // 384 37.9 -> 31.3), whatever the number of rows (narrower layers: 8192 x 8192, M = 600 121.8 -> 94.0; 2048 x 10240, M = 700
+    // 39.1 -> 33.8; 4096 x 8192, M = 900 69.9 -> 60.3; 2048 x 4096, M = 1179 34.0 -> 28.0, M = 2030 40.4 -> 34.9). Not with fewer
+    // workgroups (2048 x 11264, M = 512, 176 wide ones: 29.5 -> 31.7) and not with a short K (1024 x 16384, M = 384:
+    // 17.1 -> 18.5).
     const int64_t tp = (np + 127) / 128;
     if (family == 0 && m > 128 && tp * ((m + 127) / 128) > 256) {
       if (m <= 256) return m <= 192 ? V_128x192 : V_8W_128x256;

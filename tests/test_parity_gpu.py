@@ -648,10 +648,11 @@ def test_stage_ring_with_few_k_tiles(capi, M, K):
 @pytest.mark.parametrize("M,K,ff,name", [(129, 264, 8192, "dma_128x128"), (256, 264, 8192, "dma_128x128"),
                                          (200, 264, 8200, "dma8w_128x256"), (257, 2048, 8192, "dma_128x192"),
                                          (384, 2056, 8188, "dma_128x192"), (385, 2056, 8192, "dma8w_128x256"),
-                                         (511, 2048, 7172, "dma8w_128x256"), (576, 2048, 5120, "dma_128x192")])
+                                         (511, 2048, 7172, "dma8w_128x256"), (576, 2048, 5120, "dma_128x192"),
+                                         (1179, 2048, 2048, "dma_128x192"), (2030, 2056, 2044, "dma8w_128x256")])
 def test_gateup_tiles_that_fill_one_round(capi, M, K, ff, name):
-    """129 rows and more on the tile whose launch has at most 256 workgroups: both sides of its rows, two and three tiles of
-    activation rows on the wide kernels, ragged features, K tails; output inside a wider NaN buffer."""
+    """129 rows and more on the tile whose launch has at most 256 workgroups: both sides of its rows, two, three and more tiles
+    of activation rows on the wide kernels, ragged features, K tails; output inside a wider NaN buffer."""
     assert capi.variant_name(0, 0, M, 2 * ff, K) == name
     inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + ff, x_scale=0.5)
     X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
