@@ -352,11 +352,14 @@ int fsw_gateup(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int64_
 // The reference's other build (C_TYPE float, constants.cuh:9-14; "C can work with either bf16 or fp32",
 // swiglu.cu:470-471): H is float and receives the gated fp32 value without a rounding. From 2^21 gated weight pairs on
 // (a layer of 1024 x 2816 has 2.9 million) it runs the kernel that the 16-bit output would run, whose tiles fit
-// the rows and the compute units (the persistent decode kernel has no float store: skinny_kernel there); smaller layers
-// run the weight-streaming kernel up to 64 rows and the 256 x 256 kernel above, so that rounding their result gives the
-// 16-bit output of those kernels bit for bit. Measured against those two kernels, us: 4096 x 11008:
+// the rows and the compute units (the persistent decode kernel has no float store: skinny_kernel there). Measured against
+// the weight-streaming kernel (up to 64 rows) and the 256 x 256 kernel (above), us: 4096 x 11008:
 // 40 rows 38.4 -> 31.6, 65 rows 64.6 -> 41.0, 130 rows 66.0 -> 50.1, 200 rows 66.6 -> 55.7; 1024 x 2816: 16 rows level,
 // 65 rows 21.0 -> 10.1, 300 rows 23.5 -> 10.9, 1000 rows 25.3 -> 18.5; 8192 x 28672: 40 rows 189 -> 150.
+// Smaller layers keep those two kernels. Up to 64 rows weight streaming is the faster one there (512 x 1408, 64 rows 6.5 us against
+// 7.1 on 128 x 64; 768 x 2048 6.4 against 9.3). Above, the small tiles would be (512 x 1408: 100 rows 14.7 against 8.5, 300 rows 15.8
+// against 7.5; 768 x 2048: 300 rows 19.0 against 9.2), but they add the products in another order: the results of such layers,
+// of which rounding gives the 256 x 256 kernel's 16-bit output bit for bit, would change in their last bits.
 int fsw_gateup_f32out(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* W13,
                       int64_t ldw, float* H, int64_t ldh, void* stream) {
   const int rc = fsw_validate_gateup(dtype, M, N, K, X, ldx, W13, ldw, H, ldh);
