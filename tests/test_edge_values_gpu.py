@@ -9,9 +9,9 @@ from oracle import oracle
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-# gate/up kernels by fsw_set_variant id: automatic, the tiled kernels (1 is 3), the weight-streaming kernel and the
-# persistent streaming kernel (the last two take at most 64 and 16 rows)
-GATEUP_VARIANTS = [-1, 0, 1, 2, 3, 4, 5, 100, 102]
+# gate/up kernels by fsw_set_variant id: automatic, the tiled kernels (1 is 3), the 256-row kernel with 160, 192 and
+# 224 activation rows per tile, the weight-streaming kernel and the persistent streaming kernel (the last two take at most 64 and 16 rows)
+GATEUP_VARIANTS = [-1, 0, 1, 2, 3, 4, 5, 115, 116, 117, 100, 102]
 
 
 def one_hot_problem(dtype, ups, gates, M=16, K=64, ff=72):

@@ -744,6 +744,45 @@ def test_weights_that_are_no_whole_cache_lines(capi, M, off, pad):
     assert_one_rounding(Y, H0.double() @ inp["W2"].double().T, torch.bfloat16, "Y %s" % ((M, off, pad),))
 
 
+def _behind_nan(t, pad):
+    """t on the device as the left columns of a buffer whose rows are `pad` elements longer, NaN behind every row."""
+    wide = torch.full((t.shape[0], t.shape[1] + pad), float("nan"), dtype=t.dtype, device=DEV)
+    wide[:, :t.shape[1]] = t.to(DEV)
+    return wide[:, :t.shape[1]]
+
+
+@pytest.mark.parametrize("variant,M", [(4, 40), (4, 64), (0, 130), (2, 150), (3, 200), (5, 300), (115, 300), (116, 200), (117, 230)])
+@pytest.mark.parametrize("K,pad", [(328, 8), (320, 64)])
+def test_strided_inputs_of_the_tiled_kernels(capi, variant, M, K, pad):
+    """Rows of X, H and the weights longer than K, NaN behind them: neither the K tail nor the copies past the last K tile of the
+    rings take anything from there (NaN would reach every sum). K with and without a tail, both projections."""
+    ff = 8 * 67
+    inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + K + variant, x_scale=0.5)
+    H0 = (torch.randn(M, ff, generator=torch.Generator().manual_seed(M)) * 0.5).to(torch.bfloat16)
+    try:
+        capi.set_variant(0, variant)
+        capi.set_variant(1, variant)
+        H = capi.gateup(_behind_nan(inp["X"], pad), _behind_nan(inp["W13"], pad))
+        Y = capi.down(_behind_nan(H0, pad), _behind_nan(inp["W2"], pad))
+    finally:
+        capi.set_variant(0, -1)
+        capi.set_variant(1, -1)
+    assert_one_rounding(H, oracle.ref_gateup(inp["X"], inp["W13"], torch.float64), torch.bfloat16, "H")
+    assert_one_rounding(Y, H0.double() @ inp["W2"].double().T, torch.bfloat16, "Y")
+
+
+@pytest.mark.parametrize("M,D,FF,name", [(63, 1000, 2056, "splitk_dma_128x64"), (435, 4096, 8192, "splitk_pair16_256x160"),
+                                         (516, 4096, 8200, "splitk_pair16_256x192"), (887, 4096, 6144, "splitk_pair16_256x224")])
+def test_strided_inputs_of_the_split_down_projection(capi, M, D, FF, name):
+    """The same for the parts of a split K: a part ends inside a row, the last one at its NaN."""
+    assert capi.variant_name(1, 0, M, D, FF) == name
+    gen = torch.Generator().manual_seed(M + FF)
+    H = (torch.randn(M, FF, generator=gen) * 0.5).to(torch.bfloat16)
+    W2 = (torch.randn(D, FF, generator=gen) / FF ** 0.5).to(torch.bfloat16)
+    Y = capi.down(_behind_nan(H, 72), _behind_nan(W2, 8))
+    assert_one_rounding(Y, (H.to(DEV).double() @ W2.to(DEV).double().T).cpu(), torch.bfloat16, name)
+
+
 NARROW_SPLITS = [(435, 4096, 8192, 160), (300, 4096, 8200, 160), (768, 4096, 6144, 192), (516, 4096, 8200, 192),
                  (887, 4096, 6144, 224), (672, 4096, 8200, 224)]
 
