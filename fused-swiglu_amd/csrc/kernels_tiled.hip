@@ -557,9 +557,11 @@ static const NarrowTile kNarrow[] = {{256, 1.0}, {224, 0.91}, {192, 0.81}, {160,
 // blocked H, which these tiles do not read. A narrow tile must be ahead by 1 - `need`.
 // 256 -> best, us: gate/up 4096 x 28672: 300 rows 78 -> 57 (160), 333 rows 79 -> 63 (192), 448 rows 85 -> 77 (224),
 // 640 rows 150 -> 112 (160), 1000 rows stay (168, narrow 193 or more); 8192 x 57344, 520 rows 472 -> 412 (192); down
-// 11008 -> 4096: 2500 rows 173 -> 153 (160), 3000 rows 191 -> 177 (192), 4300 rows 379 -> 282 (160).
-// Rounds decide, not only padding, so row counts that 256 divides gain as well: 11008 -> 4096: 2304 rows 210 -> 169 (160), 2560
-// rows 212 -> 180 (160), 3072 rows 217 -> 199 (192), 4352 rows 408 -> 322 (160); 8192 x 28672, forward of 1280 rows 1371 -> 1332.
+// 11008 -> 4096: 2500 rows 173 -> 153 (160), 3000 rows 191 -> 177 (192), 4300 rows 379 -> 282 (160); inputs that repeat from
+// call to call. With inputs that come from memory: 2500 rows 195 -> 175, 4351 rows 408 -> 323.
+// Rounds decide, not only padding, so row counts that 256 divides gain as well (from memory, too): 11008 -> 4096: 2304 rows
+// 210 -> 169 (160), 2560 rows 212 -> 180 (160), 3072 rows 217 -> 199 (192), 4352 rows 408 -> 322 (160); 8192 x 28672, forward of
+// 1280 rows 1328 -> 1293.
 int pair16_tile_rows(bool gated, long long np, long long nq, double need) {
   const long long tp = (np + 255) / 256;
   if (tp * ((nq + 255) / 256) > (gated ? 1024 : 512)) return 256;
@@ -613,7 +615,7 @@ static double split_time(int np, int nq, int k, int tile_q, double tile_cost, in
 // 371 rows 30.7 / 35.0 / 27.3; 2088 -> 736, 1996 rows 26.0 / 34.5 / 22.5; 3408 -> 1352, 910 rows 28.4 / 34.0 / 27.8; 11104 -> 5904,
 // 479 rows 76.5 / 86.8 / 76.5; 11008 -> 4096, 333 rows 61.7 / 51.9 / 48.4, 1536 rows 133 / 133 / 120; 14336 -> 4096, 1024 rows
 // level at 102. On 302 random problems none of these were fitted to: 0.896 of the first on average (95 % of them below 0.99, worst
-// 1.06), 0.931 of the second (worst 1.02).
+// 1.06), 0.931 of the second (worst 1.02); on 260 with d of 64 .. 768 or ff of up to 12 d 0.869 (worst 1.11) and 0.881 (worst 1.09).
 static SplitPlan mid_split_plan(int np, int nq, int k) {
   static const struct {
     int rows;
