@@ -24,6 +24,7 @@ constexpr int VARIANT_DECODE_FUSED_FAIL = 103;  // 101 with a device-wide barrie
 constexpr int VARIANT_STREAM_SPLIT = 104;    // family 1, fsw_mlp only: split-K streaming down projection for M <= 32
 // the 256 x 256 kernel with narrower tiles: VARIANT_NARROW + 5, 6, 7 = 160, 192, 224 activation rows per tile
 constexpr int VARIANT_NARROW = 110;
+constexpr int VARIANT_MID = 200;             // VARIANT_MID + i: tile i of the producer / consumer kernel, whole tiles, unsplit
 constexpr int64_t MAX_DIM = 1LL << 30;       // every size is cast to int inside the kernels
 constexpr int64_t MAX_LD = 1LL << 21;        // keeps tile-relative byte offsets below 2^31
 
@@ -56,37 +57,15 @@ int check_device() {
 // indices of the tiled kernels (tiled_variant() of kernels_tiled.hip)
 constexpr int V_128x128 = 0, V_128x192 = 2, V_8W_128x256 = 3, V_128x64 = 4, V_256x256 = 5;
 
-// Variant choice for the tiled kernels: the widest tile whose activation-row extent is not mostly padding,
-// stepping down to 128x128 when a 256-wide grid would leave most of the 256 CUs idle.
+// Range of rows of a tiled launch. The 128-row names stand for the producer / consumer kernel (kernels_mid.hip), which chooses its
+// tile by an estimate of its own; they tell the rows that one of its launches shares the weights between (128 x 64: up to 64, 128 x
+// 128 and so on) and are what fsw_set_variant forces. The others are the 256-row kernel.
 // `narrow_need`: a narrower large tile is taken only if its estimated time is below this share of 256 x 256's
 int pick_tiled(int family, int64_t m, int64_t np, int64_t k, double narrow_need = 0.95) {
   const int64_t tiles256 = ((np + 255) / 256) * ((m + 255) / 256);
-  // 256 x 256 tiles down to half-filled compute units. Below that the down product splits K (see
-  // tiled_split_plan); between 129 and 191 tiles one large tile per compute unit beats 128 x 128 tiles in
-  // 1.1 .. 1.4 rounds (down, 4096 x 14336, M = 2304 .. 2816: 250-260 us against 355-365 us; gate/up, 4096 x 22016,
-  // M = 257 .. 512: 79-81 us against 95-102 us).
-  // Up to 128 activation rows are one weight stream whatever the tile count (8192 x 57344, M = 65 .. 128: 173 us on
-  // 128 x 128 tiles, 201-203 us on half-empty large ones).
+  // 256 x 256 tiles down to half-filled compute units (129 tiles); up to 128 activation rows are one weight stream whatever the
+  // tile count.
   if (tiles256 < 129 || m <= 128) {
-    // 128 x 128, direct-to-LDS (with split-K for the down product, see fsw_down). The gate/up product of 129 .. 256
-    // activation rows takes them in ONE 128 x 256 tile, so that every weight byte is still read exactly once
-    // (4096 x 28672: M = 160: 85 -> 64 us, M = 256: 86 -> 68 us; at M = 128 the 128 x 128 tile is faster, 50 vs 66),
-    // provided those tiles still cover half the compute units (1024 x 5632 at M = 256: 44 of them, 18.5 us against
-    // 10.5 us for 88 tiles of 128 x 128).
-    // Up to 192 rows the tile is 128 x 192: the single-tile kernels are bound by their MFMA and LDS work as much as
-    // by the weight stream (4096 x 28672, M = 160: 65 -> 54 us; 5120 x 27648: 89 -> 68 us).
-    // 193 .. 256 rows: 128 x 256 on 8 waves, two per SIMD (4096 x 28672: 72 -> 64 us, 5120 x 27648: 94 -> 79-87 us
-    // against 4 waves).
-    // All that only where two 128-row tiles are more workgroups than compute units: up to 256 workgroups 128 x 128 tiles
-    // have three stages each and a compute unit to themselves (4096 x 16384: M = 129 47.6 -> 41.8 us, M = 256 54.9 -> 45.9;
-    // 2048 x 16384: M = 200 29.3 -> 23.2).
-    // The same limit above 256 rows: 257 .. 512 workgroups of 128 x 128 share compute units two by two and keep two stages,
-    // so the wider tile whose launch fills one round (224 .. 256 workgroups) is taken (4096 x 16384: M = 257 66.6 -> 50.6 us
-    // and M = 384 72.7 -> 58.7 on 128 x 192, M = 450 75.3 -> 61.5 and M = 512 79.0 -> 64.6 on 128 x 256; 2048 x 16384: M =
-    // 384 37.9 -> 31.3), whatever the number of rows (narrower layers: 8192 x 8192, M = 600 121.8 -> 94.0; 2048 x 10240, M = 700
-    // 39.1 -> 33.8; 4096 x 8192, M = 900 69.9 -> 60.3; 2048 x 4096, M = 1179 34.0 -> 28.0, M = 2030 40.4 -> 34.9). Not with fewer
-    // workgroups (2048 x 11264, M = 512, 176 wide ones: 29.5 -> 31.7) and not with a short K (1024 x 16384, M = 384:
-    // 17.1 -> 18.5).
     const int64_t tp = (np + 127) / 128;
     if (family == 0 && m > 128 && tp * ((m + 127) / 128) > 256) {
       if (m <= 256) return m <= 192 ? V_128x192 : V_8W_128x256;
@@ -94,48 +73,25 @@ int pick_tiled(int family, int64_t m, int64_t np, int64_t k, double narrow_need 
       if (k >= 2048 && w192 >= 224 && w192 <= 256) return V_128x192;
       if (k >= 2048 && w256 >= 224 && w256 <= 256) return V_8W_128x256;
     }
-    // up to 64 rows the gate/up tile is 128 x 64 (4096 x 28672, M = 48: 39.4 -> 37.2 us)
     return (family == 0 && m <= 64) ? V_128x64 : V_128x128;
   }
   const int rows = fsw::pair16_tile_rows(family == 0, np, m, narrow_need);
   if (rows != 256) return VARIANT_NARROW + rows / 32;
   if (family == 0 && tiles256 > 256 && tiles256 <= 512) {
-    // A few large tiles more than compute units: the second round is nearly empty, while 128 x 128 tiles (two per
-    // compute unit, ~1.3-1.7 x the time per output element) come in rounds a quarter as long. Per round of 256
-    // workgroups: ~33 us against ~75-100 us at K = 4096; the small tile must win by 20 % to be taken. 4096 x 36864,
-    // M = 300 (288 tiles): 151 -> 130 us; 4096 x 22016, M = 640 (258 tiles): 148 -> 119 us.
+    // A few large tiles more than compute units: the second round is nearly empty, while smaller tiles come in shorter rounds.
     const int64_t tiles128 = ((np + 127) / 128) * ((m + 127) / 128);
     if (((tiles128 + 255) / 256) * 44 < ((tiles256 + 255) / 256) * 100) return V_128x128;
   }
   return V_256x256;
 }
 
-// Most activation rows that still run the weight-streaming kernels (which take up to 64). Their time grows with
-// the rows (each workgroup re-reads every activation row from the L2), the tiled kernels' hardly does, and the
-// larger the weight matrices the earlier the tiled kernels win. Whole forwards, weight-streaming vs tiled, us:
-// 2048 x 8192: M = 32 32.5 / 37.1, 48 39.4 / 39.7, 64 46.0 / 41.7; 4096 x 11008: M = 32 57.7 / 60.4, 40 65.5 / 62.7,
-// 64 77.6 / 64.9; 4096 x 14336: M = 24 72.5 / 75.2, 32 75.3 / 70.4, 64 99.6 / 70.6; 8192 x 28672: M = 17 252.8 /
-// 228.3, 64 370.5 / 242.5. K == 0 stays with the weight-streaming kernels, which write the all-zero result.
+// Most activation rows of the decode range, whose launches are weight streaming by skinny_kernel or, where that is faster
+// (mid_wanted), by the producer / consumer kernel: fewer the larger the weights. K == 0 stays with the weight-streaming kernels,
+// which write the all-zero result.
 int64_t decode_rows(int family, int64_t np, int64_t k) {
   if (k <= 0) return 64;
   const int64_t d_ff = family == 0 ? (np / 2) * k : np * k;
   return d_ff < ((int64_t)1 << 25) ? 48 : d_ff < ((int64_t)1 << 27) ? 32 : 16;
-}
-
-// Weight rows per workgroup of the 128-row tiled kernels when ONE tile of activation rows streams the whole weight
-// matrix (gate/up): cut into 128-row tiles a matrix of fewer than 256 x 128 rows leaves compute units idle, and one
-// compute unit fetches at most ~29 GB/s, so the stream is cut into one piece per compute unit instead (a multiple of 8
-// rows; the kernel's copies of the rows past its piece are out of range and cost no traffic). Gate/up alone, 128-row
-// tiles -> pieces, us: 16384 rows (128 tiles -> 256 x 64) M = 64 33.8 -> 31.0, M = 128 41.1 -> 39.3; 22016 rows (172 ->
-// 251 x 88) 36.1 -> 34.2, 43.4 -> 41.9; 27648 rows (216 -> 247 x 112) M = 16 47.0 -> 45.3, M = 64 52.0 -> 49.4, M = 128
-// 62.6 -> 60.0. Not with 224 tiles or more (28672 rows: 35.2 -> 35.8, the pieces' wasted MFMA and LDS work costs more
-// than the 32 idle compute units) and not above 128 activation rows, where the matrix cores are the limit (16384 rows,
-// M = 256: 53.5 -> 56.2). 0 = the kernel's own tile height.
-int stream_tile_rows(int variant, int64_t m, int64_t np) {
-  if (!(variant == V_128x64 && m <= 64) && !(variant == V_128x128 && m <= 128)) return 0;
-  if ((np + 127) / 128 > 216) return 0;
-  const int64_t rows = ((np + 255) / 256 + 7) / 8 * 8;
-  return (rows >= 64 && rows < 128) ? (int)rows : 0;
 }
 
 int resolve_variant(int family, int64_t m, int64_t np, int64_t k) {
@@ -145,10 +101,7 @@ int resolve_variant(int family, int64_t m, int64_t np, int64_t k) {
     return m <= 64 ? VARIANT_SKINNY : pick_tiled(family, m, np, k);
   if (forced >= 0 && !(forced == VARIANT_SKINNY && m > 64)) return forced;
   if (m <= decode_rows(family, np, k)) {  // decode and small batches: weight streaming, HBM bound
-    // The gate/up product streams its weights faster through the four-stage 128 x 64 tiled kernel (direct-to-LDS
-    // copies) than through the weight-streaming kernel when its tiles of 128 weight rows fill one round of compute
-    // units and there are a dozen rows or more (gate/up, us: 4096 x 28672: M = 16 37.9 -> 35.6, 32 43.3 -> 36.0, M = 1
-    // level; 5120 x 27648: M = 16 49.3 -> 47.3, M = 4 45.3 -> 47.2; 172 tiles of 4096 x 22016: 28.8 -> 33.7, no).
+    // from a dozen rows on a gate/up matrix of 200 .. 256 pieces of 128 rows is past that range
     const int64_t tiles = (np + 127) / 128;
     if (family == 0 && m >= 12 && k > 0 && tiles >= 200 && tiles <= 256) return V_128x64;
     return VARIANT_SKINNY;
@@ -182,10 +135,58 @@ int finish(hipError_t e) {
 
 bool narrow_variant(int v) { return v >= VARIANT_NARROW + 5 && v <= VARIANT_NARROW + 7; }
 
-hipError_t launch_tiled_variant(int v, int dtype, bool gated, fsw::GemmArgs& a, hipStream_t stream) {
-  if (!narrow_variant(v)) return fsw::launch_tiled(v, dtype, gated, a, stream);
-  a.tile_q = 32 * (v - VARIANT_NARROW);
-  return fsw::launch_tiled(V_256x256, dtype, gated, a, stream);
+bool mid_variant(int v) { return v >= VARIANT_MID && v < VARIANT_MID + fsw::mid_tile_count(); }
+bool dma_variant(int v) { return (v >= 0 && v < V_256x256) || mid_variant(v); }
+
+// Rows of a dense operand of `k` columns that are no whole 128-byte lines.
+bool ragged(int64_t k) { return k % 64 != 0; }
+
+// Whether a launch that the rules above give to the kernels for few rows (`v`: VARIANT_SKINNY or a 128-row tile) runs the
+// producer / consumer kernel. skinny_kernel (one launch, one workgroup per 32 weight rows, 16 in the down projection) stays
+// where its workgroups fit the compute units at once and the call is short. Gate/up, us, skinny -> mid: 5632 x 1024 (176
+// workgroups) 16 rows 5.1 -> 6.4; 8192 x 1536 (256) 24 rows 7.4 -> 8.1; 11264 x 2048 (352) 4 rows 10.5 -> 10.8, 16 rows 11.7 ->
+// 10.9, 24 rows 15.4 -> 11.0; 7808 x 1320 (244, ragged) 4 rows 6.7 -> 7.2, 24 rows 8.0 -> 7.3; 16016 x 3000 (ragged) 1 row 22.0 ->
+// 19.4. Down, where K is split and a summing launch follows: 2816 -> 1024 16 rows 6.1 -> 6.4; 8192 -> 3072 16 rows 12.4 -> 13.1,
+// 24 rows 15.2 -> 13.4; 8192 -> 2048 1 row level, 16 rows 12.1 -> 10.7; 13824 -> 5120 (320 workgroups, two rounds) 1 row 31.3 ->
+// 25.2; ragged 3640 -> 1096 4 rows 6.6 -> 6.8, 16 rows 8.0 -> 7.3; 5360 -> 1344 1 row 8.1 -> 7.8, 16 rows 10.7 -> 8.4; 16416 ->
+// 4880 1 row 40.5 -> 28.7. Matrices of the persistent streaming kernel (decode_stream_wanted): gate/up 57344 x 8192 1 row 144.1 ->
+// 142.4, 16 rows 147.4 -> 136.5; 46336 x 7000 (ragged) 1 row 124.0 -> 98.8; down 28672 -> 8192 1 and 4 rows level, 16 rows
+// 84.1 -> 72.1; 23168 -> 7000 1 row 55.5 -> 52.1.
+// The 256-row kernel fetches rows that are no whole lines by K tiles, every line twice; the gate/up product of such rows takes the
+// kernel whose estimated time is less (47 problems of 130 .. 700 rows: it chose the slower one four times, by 7 % at most; 38880 x
+// 5800 130 rows 150.4 -> 119.0, 256 rows 189.6 -> 138.1; 43680 x 7592 279 rows 348 -> 241; 24160 x 3448 409 rows stays, 93.6 and 105).
+bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
+  if (g_forced_variant[family] >= 0) return dma_variant(g_forced_variant[family]);
+  if (k <= 0) return false;
+  if (family == 0 && rag && (v == V_256x256 || narrow_variant(v)) && m <= 1024) {
+    const int rows = narrow_variant(v) ? 32 * (v - VARIANT_NARROW) : 256;
+    return fsw::mid_plan(true, (int)np, (int)m, (int)k, true, 1, 1).us < fsw::pair16_ragged_time((int)np, (int)m, (int)k, rows);
+  }
+  if (!(v == VARIANT_SKINNY || dma_variant(v))) return false;
+  if (v != VARIANT_SKINNY) return true;
+  const int64_t bytes = 2 * np * k;
+  if (family == 0) {
+    const int64_t tiles = (np + 31) / 32;
+    return m > 16 ? tiles > 256 || rag : tiles > 256 && (m > 8 || bytes >= (int64_t)56 << 20);
+  }
+  const int64_t tiles = (np + 15) / 16;
+  if (m > 16) return rag || bytes >= (int64_t)8 << 20;
+  if (rag) return bytes >= (int64_t)14 << 20 || (m >= 8 && bytes >= (int64_t)7 << 20);
+  if (bytes >= (int64_t)1 << 28) return m > 4;
+  return tiles > 256 || (tiles <= 128 && k >= 8192);
+}
+
+// tile of a forced variant
+fsw::MidPlan forced_mid_plan(int v) {
+  if (mid_variant(v)) return {v - VARIANT_MID, fsw::mid_tile_rows(v - VARIANT_MID), 1, 0.0};
+  const int bq = v == V_128x64 ? 64 : v == V_128x192 ? 192 : v == V_128x128 ? 128 : 256;
+  return {fsw::mid_tile_index(128, bq), 128, 1, 0.0};
+}
+
+// the 256-row kernel, row-major operands (GemmArgs::layout 0)
+hipError_t launch_large(int v, int dtype, bool gated, fsw::GemmArgs& a, hipStream_t stream) {
+  if (narrow_variant(v)) a.tile_q = 32 * (v - VARIANT_NARROW);
+  return fsw::launch_pair16(dtype, gated, a, stream);
 }
 
 }  // namespace
@@ -232,18 +233,20 @@ int fsw_set_variant(int family, int variant) {
   if (variant >= 0 && variant != VARIANT_SKINNY && variant != VARIANT_DECODE_STREAM &&
       !(family == 0 && (variant == VARIANT_DECODE_FUSED || variant == VARIANT_DECODE_FUSED_FAIL)) &&
       !(family == 1 && variant == VARIANT_STREAM_SPLIT) &&
-      !narrow_variant(variant) && variant >= fsw::tiled_variant_count())
+      !narrow_variant(variant) && !mid_variant(variant) && variant >= fsw::tiled_variant_count())
     return FSW_E_VARIANT;
   g_forced_variant[family] = variant < 0 ? -1 : variant;
   return FSW_OK;
 }
 
 static fsw::StreamPlan mlp_stream_plan(int64_t M, int64_t D, int64_t FF);
+static const char* running_name(int family, int64_t M, int64_t N_or_D, int64_t K_or_FF);
 static bool blocked_regime(int64_t M, int64_t D, int64_t FF, size_t scratch);
 
 const char* fsw_variant_name(int family, int dtype, int64_t M, int64_t N_or_D, int64_t K_or_FF) {
   (void)dtype;
-  if (family == 2) {  // the down projection as fsw_mlp runs it
+  if (family >= 3 && family <= 5) return running_name(family, M, N_or_D, K_or_FF);
+  if (family == 2) {  // the down projection inside fsw_mlp
     if (mlp_stream_plan(M, N_or_D, K_or_FF).splits > 1) return "stream_split";
     if (blocked_regime(M, N_or_D, K_or_FF, SIZE_MAX)) return fsw::tiled_variant(V_256x256).name;
     family = 1;
@@ -268,6 +271,7 @@ const char* fsw_variant_name(int family, int dtype, int64_t M, int64_t N_or_D, i
     static const char* const names[3] = {"pair16_256x160", "pair16_256x192", "pair16_256x224"};
     return names[v - VARIANT_NARROW - 5];
   }
+  if (mid_variant(v)) return fsw::mid_name(forced_mid_plan(v));
   return fsw::tiled_variant(v).name;
 }
 
@@ -303,6 +307,12 @@ int fsw_validate_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H
   return FSW_OK;
 }
 
+static hipError_t launch_gateup_mid(int v, int dtype, const fsw::GemmArgs& a, hipStream_t stream) {
+  const fsw::MidPlan p = g_forced_variant[0] >= 0 ? forced_mid_plan(v)
+                                                  : fsw::mid_plan(true, a.np, a.nq, a.k, fsw::mid_ragged(a), 1, 1);
+  return fsw::launch_mid(dtype, true, p, a, stream);
+}
+
 // zero_words / n_zero_words: see GemmArgs (only the decode-regime kernels honour them; the caller checks that)
 static int gateup_impl(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* W13,
                        int64_t ldw, void* H, int64_t ldh, void* stream, unsigned* zero_words, int n_zero_words) {
@@ -324,7 +334,7 @@ static int gateup_impl(int dtype, int64_t M, int64_t N, int64_t K, const void* X
   a.zero_words = zero_words;
   a.n_zero_words = n_zero_words;
   const int v = resolve_variant(0, M, N, K);
-  a.tile_p = stream_tile_rows(v, M, N);
+  if (mid_wanted(0, v, M, N, K, fsw::mid_ragged(a))) return finish(launch_gateup_mid(v, dtype, a, (hipStream_t)stream));
   if (v == VARIANT_SKINNY) {
     if (decode_stream_wanted(0, M, N, K)) {  // at most 16 rows: one 8-wave workgroup per CU, X held in registers
       fsw::DecodeArgs da = {};
@@ -341,7 +351,7 @@ static int gateup_impl(int dtype, int64_t M, int64_t N, int64_t K, const void* X
     }
     return finish(fsw::launch_skinny(dtype, true, a, nullptr, (hipStream_t)stream));
   }
-  return finish(launch_tiled_variant(v, dtype, true, a, (hipStream_t)stream));
+  return finish(launch_large(v, dtype, true, a, (hipStream_t)stream));
 }
 
 int fsw_gateup(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* W13, int64_t ldw,
@@ -380,16 +390,19 @@ int fsw_gateup_f32out(int dtype, int64_t M, int64_t N, int64_t K, const void* X,
   a.k = (int)K;
   a.out_f32 = 1;
   int v = M <= 64 ? VARIANT_SKINNY : V_256x256;
-  if ((N / 2) * K >= (int64_t)1 << 21) v = resolve_variant(0, M, N, K);
-  a.tile_p = stream_tile_rows(v, M, N);
+  if ((N / 2) * K >= (int64_t)1 << 21) {
+    v = resolve_variant(0, M, N, K);
+    if (mid_wanted(0, v, M, N, K, fsw::mid_ragged(a))) return finish(launch_gateup_mid(v, dtype, a, (hipStream_t)stream));
+  }
   if (v == VARIANT_SKINNY) return finish(fsw::launch_skinny(dtype, true, a, nullptr, (hipStream_t)stream));
-  return finish(launch_tiled_variant(v, dtype, true, a, (hipStream_t)stream));
+  return finish(launch_large(v, dtype, true, a, (hipStream_t)stream));
 }
 
-// Inside fsw_mlp the down projection of up to 32 activation rows runs the split-K streaming kernel when (i) the
-// gate/up product before it runs a kernel that zeroes the ticket counters (skinny_kernel or the 128 x 64 tiled
-// kernel), (ii) the down projection is in the weight-streaming regime and (iii) the shape is large enough for the
-// saved H traffic to matter (stream_split_plan) -- or when variant 104 forces it (then any shape it supports).
+// Rows of fsw_mlp (17 .. 32, large layers) that have the name "stream_split", and the plan of the split-K streaming kernel for them.
+// That kernel runs only when variant 104 asks for it (then any shape it supports), and where the gate/up product before it runs a
+// kernel that zeroes the ticket counters (skinny_kernel or mid_kernel): K parts of mid_kernel and a summing launch are faster
+// everywhere (whole forwards, us, stream_split -> mid: 4096 x 11008 24 rows 52.1 -> 48.9; 4096 x 14336 17 rows 60.3 -> 59.2, 32 rows
+// 63.5 -> 61.3; 5120 x 13824 24 rows 83.7 -> 72.4; 2048 x 8192 32 rows 28.3 -> 24.6; 4880 x 16416 24 rows 102 -> 83).
 static fsw::StreamPlan mlp_stream_plan(int64_t M, int64_t D, int64_t FF) {
   const fsw::StreamPlan none = {0, 0, 0, 0};
   if (M < 1 || M > 32 || D <= 0 || FF <= 0 || D > MAX_DIM || FF > MAX_DIM / 2) return none;
@@ -404,24 +417,57 @@ static fsw::StreamPlan mlp_stream_plan(int64_t M, int64_t D, int64_t FF) {
   if (!streams_weights(1, M, D, FF) || decode_stream_wanted(1, M, D, FF)) return none;
   return fsw::stream_split_plan((int)D, (int)M, (int)FF, false);
 }
+static bool stream_split_runs(int64_t M, int64_t D, int64_t FF) {
+  return g_forced_variant[1] == VARIANT_STREAM_SPLIT && mlp_stream_plan(M, D, FF).splits > 1;
+}
 static size_t stream_scratch_bytes(const fsw::StreamPlan& p) {
   return (p.partial_bytes + (size_t)p.ticket_words * 4 + 255) & ~(size_t)255;
 }
 
-// Bytes of the split-K down projection's partial sums, 0 if it runs unsplit. `limit`: most bytes they may take; a plan that
-// wants more splits K less often (fsw_mlp_static, whose scratch is fixed, keeps the shapes that any plan fits).
-static size_t down_split(int64_t M, int64_t D, int64_t FF, size_t limit, fsw::SplitPlan* plan) {
-  if (M <= 0 || M > MAX_DIM || D <= 0 || D > MAX_DIM || FF <= 0 || FF > MAX_DIM || streams_weights(1, M, D, FF)) return 0;
-  if (g_forced_variant[1] >= 0) return 0;  // a forced kernel runs unsplit
-  *plan = fsw::tiled_split_plan((int)D, (int)M, (int)FF);
+// How the down projection runs. Parts of K: fp32 partial sums of parts * M * D floats in the workspace.
+//   mid:  the producer / consumer kernel (any number of parts)
+//   else: parts > 1: launch_tiled_splitk on `plan.tile`; 1: the unsplit kernel of resolve_variant()
+// `limit`: most bytes the partial sums may take; a plan that wants more splits K less often (fsw_mlp_static, whose scratch is
+// fixed, keeps the shapes that any plan fits).
+struct DownPlan {
+  bool mid;
+  fsw::SplitPlan plan;
+};
+static DownPlan down_plan(int64_t M, int64_t D, int64_t FF, size_t limit, bool rag) {
+  DownPlan r = {false, {128, 1}};
+  if (M <= 0 || M > MAX_DIM || D <= 0 || D > MAX_DIM || FF <= 0 || FF > MAX_DIM) return r;
+  const int v = resolve_variant(1, M, D, FF);
   const size_t part = (size_t)M * (size_t)D * sizeof(float);
-  if (plan->splits > 1 && limit / part < (size_t)plan->splits) plan->splits = (int)(limit / part);
-  return plan->splits > 1 ? plan->splits * part : 0;
+  const int64_t most = (int64_t)(limit / part < 16 ? limit / part : 16);
+  if (g_forced_variant[1] >= 0) {  // a forced kernel runs unsplit
+    r.mid = dma_variant(v);
+    return r;
+  }
+  if (v == VARIANT_SKINNY || M <= 256) {
+    r.mid = mid_wanted(1, v, M, D, FF, rag);
+    if (r.mid) r.plan.splits = fsw::mid_plan(false, (int)D, (int)M, (int)FF, rag, 0, most < 1 ? 1 : (int)most).splits;
+    if (r.mid || v == VARIANT_SKINNY) return r;
+  }
+  r.plan = fsw::tiled_split_plan((int)D, (int)M, (int)FF);
+  if (r.plan.splits > most) r.plan.splits = most < 1 ? 1 : (int)most;
+  r.mid = r.plan.splits > 1 ? r.plan.tile <= 130 : dma_variant(v);
+  // rows that are no whole lines: the same parts on whichever kernel takes them faster by the estimates (8008 -> 3000 300 rows
+  // 39.6 -> 28.8 us, 900 rows 62.9 -> 58.8; 23568 -> 6168 499 rows stays, 152 and 189)
+  if (!r.mid && rag && r.plan.splits > 1 && M <= 1024)
+    r.mid = fsw::mid_plan(false, (int)D, (int)M, (int)FF, true, r.plan.splits, r.plan.splits).us <
+            0.95 * fsw::pair16_split_time((int)D, (int)M, (int)FF, r.plan);
+  return r;
+}
+
+// bytes of the partial sums; planned for dense operands (FF columns to a row)
+static size_t down_split(int64_t M, int64_t D, int64_t FF, size_t limit, DownPlan* plan) {
+  *plan = down_plan(M, D, FF, limit, ragged(FF));
+  return plan->plan.splits > 1 ? plan->plan.splits * (size_t)M * (size_t)D * sizeof(float) : 0;
 }
 
 size_t fsw_down_workspace_bytes(int dtype, int64_t M, int64_t D, int64_t FF) {
   (void)dtype;
-  fsw::SplitPlan plan;
+  DownPlan plan;
   return down_split(M, D, FF, SIZE_MAX, &plan);
 }
 
@@ -430,9 +476,14 @@ static int down_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* H,
   const int rc = fsw_validate_down(dtype, M, D, FF, H, ldh, W2, ldw2, Y, ldy);
   if (rc != FSW_OK) return rc;
   if (M == 0 || D == 0) return FSW_OK;
-  fsw::SplitPlan plan;
-  const size_t need = down_split(M, D, FF, limit, &plan);
-  if (need > 0 && (!workspace || workspace_bytes < need)) return FSW_E_WORKSPACE;
+  DownPlan plan;
+  size_t need = down_split(M, D, FF, limit, &plan);
+  const int v = resolve_variant(1, M, D, FF);
+  if (need > 0 && (!workspace || workspace_bytes < need)) {
+    if (v != VARIANT_SKINNY) return FSW_E_WORKSPACE;
+    plan.mid = false;  // few rows: the weight-streaming kernel needs no scratch
+    need = 0;
+  }
   const int drc = check_device();
   if (drc != FSW_OK) return drc;
   fsw::GemmArgs a;
@@ -445,7 +496,15 @@ static int down_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* H,
   a.np = (int)D;
   a.nq = (int)M;
   a.k = (int)FF;
-  const int v = resolve_variant(1, M, D, FF);
+  if (need > 0 && !aligned16(workspace)) return FSW_E_ALIGN;
+  if (plan.mid) {
+    a.splits = need > 0 ? plan.plan.splits : 1;
+    a.partial = (float*)workspace;
+    const fsw::MidPlan p = g_forced_variant[1] >= 0
+                               ? forced_mid_plan(v)
+                               : fsw::mid_plan(false, (int)D, (int)M, (int)FF, fsw::mid_ragged(a), a.splits, a.splits);
+    return finish(fsw::launch_mid(dtype, false, p, a, (hipStream_t)stream));
+  }
   if (v == VARIANT_SKINNY) {
     if (decode_stream_wanted(1, M, D, FF)) {
       fsw::DecodeArgs da = {};
@@ -463,12 +522,11 @@ static int down_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* H,
     return finish(fsw::launch_skinny(dtype, false, a, workspace, (hipStream_t)stream));
   }
   if (need > 0) {  // few output tiles, deep K: split K across workgroups
-    if (!aligned16(workspace)) return FSW_E_ALIGN;
-    a.splits = plan.splits;
+    a.splits = plan.plan.splits;
     a.partial = (float*)workspace;
-    return finish(fsw::launch_tiled_splitk(dtype, plan.tile, a, (hipStream_t)stream));
+    return finish(fsw::launch_tiled_splitk(dtype, plan.plan.tile, a, (hipStream_t)stream));
   }
-  return finish(launch_tiled_variant(v, dtype, false, a, (hipStream_t)stream));
+  return finish(launch_large(v, dtype, false, a, (hipStream_t)stream));
 }
 
 int fsw_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H, int64_t ldh, const void* W2, int64_t ldw2,
@@ -495,9 +553,25 @@ static bool blocked_regime(int64_t M, int64_t D, int64_t FF, size_t scratch) {
   if (M > MAX_DIM || D > MAX_DIM || FF > MAX_DIM / 2) return false;
   // a down projection on narrower tiles reads row-major H; it has to gain more than H blocked does (3000 rows of 4096 x
   // 11008: 7 % of the down kernel, a third of the forward, is not enough; 2500 rows: 11 %)
-  fsw::SplitPlan plan;  // a split-K down projection reads row-major H
+  DownPlan plan;  // a split-K down projection reads row-major H
   return pick_tiled(0, M, 2 * FF, D) == V_256x256 && pick_tiled(1, M, D, FF, 0.9) == V_256x256 &&
          (size_t)fsw::blocked_bytes(M, FF) <= scratch && down_split(M, D, FF, beside_h(M, FF, scratch), &plan) == 0;
+}
+
+// fsw_variant_name families 3 .. 5: the kernel that runs, for dense operands on whole lines where the rows are
+static const char* running_name(int family, int64_t M, int64_t N_or_D, int64_t K_or_FF) {
+  if (M <= 0 || M > MAX_DIM || N_or_D <= 0 || N_or_D > MAX_DIM || K_or_FF <= 0 || K_or_FF > MAX_DIM) return "none";
+  if (family == 5) {
+    if (stream_split_runs(M, N_or_D, K_or_FF)) return "stream_split";
+    if (blocked_regime(M, N_or_D, K_or_FF, SIZE_MAX)) return fsw::tiled_variant(V_256x256).name;
+  }
+  const bool gated = family == 3, rag = ragged(K_or_FF);
+  const int f = gated ? 0 : 1, v = resolve_variant(f, M, N_or_D, K_or_FF);
+  const DownPlan d = gated ? DownPlan{false, {0, 1}} : down_plan(M, N_or_D, K_or_FF, SIZE_MAX, rag);
+  if (gated ? mid_wanted(0, v, M, N_or_D, K_or_FF, rag) : d.mid)
+    return fsw::mid_name(g_forced_variant[f] >= 0 ? forced_mid_plan(v)
+                                                  : fsw::mid_plan(gated, (int)N_or_D, (int)M, (int)K_or_FF, rag, d.plan.splits, 1));
+  return fsw_variant_name(f, FSW_BF16, M, N_or_D, K_or_FF);
 }
 
 size_t fsw_blocked_bytes(int64_t rows, int64_t k) {
@@ -635,10 +709,10 @@ int fsw_gateup_ws(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int
 static size_t mlp_workspace(int64_t M, int64_t D, int64_t FF, size_t scratch) {
   if (M <= 0 || D <= 0 || FF <= 0) return 0;
   if (blocked_regime(M, D, FF, scratch)) return (size_t)fsw::blocked_bytes(M, FF);  // H, panel-blocked
-  const fsw::StreamPlan sp = mlp_stream_plan(M, D, FF);
-  if (sp.splits > 1) return h_bytes(M, FF) + stream_scratch_bytes(sp);  // [H row-major][partials][ticket counters]
+  if (stream_split_runs(M, D, FF))
+    return h_bytes(M, FF) + stream_scratch_bytes(mlp_stream_plan(M, D, FF));  // [H row-major][partials][ticket counters]
   // otherwise [H row-major][split-K scratch of the down projection]
-  fsw::SplitPlan plan;
+  DownPlan plan;
   return h_bytes(M, FF) + ((down_split(M, D, FF, beside_h(M, FF, scratch), &plan) + 255) & ~(size_t)255);
 }
 
@@ -699,8 +773,9 @@ static int mlp_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* X, 
     return fsw_down_blocked(dtype, M, D, FF, workspace, W2, ldw2, 0, Y, ldy, stream);
   }
   unsigned char* ws2 = (unsigned char*)workspace + h_bytes(M, FF);
-  const fsw::StreamPlan sp = mlp_stream_plan(M, D, FF);
-  if (sp.splits > 1) {  // decode: the gate/up kernel zeroes the ticket counters of the split-K streaming down projection
+  if (stream_split_runs(M, D, FF)) {
+    const fsw::StreamPlan sp = mlp_stream_plan(M, D, FF);
+    // the gate/up kernel zeroes the ticket counters of the split-K streaming down projection
     unsigned* tickets = (unsigned*)(ws2 + sp.partial_bytes);
     rc = gateup_impl(dtype, M, 2 * FF, D, X, ldx, W13, ldw13, Hbuf, FF, stream, tickets, sp.ticket_words);
     if (rc != FSW_OK) return rc;

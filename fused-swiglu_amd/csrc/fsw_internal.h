@@ -24,17 +24,16 @@ struct GemmArgs {
   // (gated kernel), bit 2 = P. A blocked [rows, k] matrix is ceil(rows / 256) panels of ceil(k / 32) blocks of
   // [256 rows][64 bytes], zero padded (blocked_bytes()).
   int layout = 0;
-  // words the FIRST workgroup of a gate/up launch sets to zero before anything else (tiled_dma_kernel and
+  // words the FIRST workgroup of a gate/up launch sets to zero before anything else (mid_kernel and
   // skinny_kernel honour it): the ticket counters of the split-K streaming down projection that follows in fsw_mlp
   unsigned* zero_words = nullptr;
   int n_zero_words = 0;
-  // gated kernels on row-major operands (skinny_kernel, tiled_dma_kernel, the 256 x 256 kernel with layout 0): O is float [nq, np/2]
+  // gated kernels on row-major operands (skinny_kernel, mid_kernel, the 256 x 256 kernel with layout 0): O is float [nq, np/2]
   // and receives the gated fp32 value unrounded (the reference's build with C_TYPE float, constants.cuh:9)
   int out_f32 = 0;
-  // tiled_dma_kernel with one tile of activation rows: weight rows a workgroup owns when that is fewer than the
-  // kernel's tile height (0 = the tile height). The tile then starts every tile_p rows, rows past tile_p are out
-  // of range for its copies (zeros, no traffic) and are not stored: lets a weight stream be cut into exactly as
-  // many pieces as there are compute units. A multiple of 8 (whole 8-byte stores of the gated output).
+  // mid_kernel: weight rows a workgroup owns when that is fewer than the kernel's tile height (0 = the tile height). The tile
+  // then starts every tile_p rows, rows past tile_p are out of range for its copies (zeros, no traffic) and are not stored: lets a
+  // weight stream be cut into exactly as many pieces as there are compute units. A multiple of 8.
   int tile_p = 0;
   // launch_pair16 with layout 0 and launch_pair16_splitk: activation rows per tile, 256 or one of 224, 192, 160
   int tile_q = 256;
@@ -43,7 +42,7 @@ inline long long blocked_bytes(long long rows, long long k) {
   return ((rows + 255) / 256) * ((k + 31) / 32) * (256 * 64);
 }
 
-// Tiled LDS/MFMA kernels (kernels_tiled.hip). `variant` indexes tiled_variant_table().
+// Names of the tiled kernels (kernels_tiled.hip). `variant` indexes tiled_variant_table().
 struct TiledVariant {
   const char* name;
   int bp, bq;        // workgroup tile: weight rows x activation rows
@@ -52,8 +51,6 @@ struct TiledVariant {
 int tiled_variant_count();
 int pair16_variant();  // index of the 256 x 256 kernel in the table
 const TiledVariant& tiled_variant(int variant);
-// row-major operands (GemmArgs::layout 0)
-hipError_t launch_tiled(int variant, int dtype, bool gated, const GemmArgs& a, hipStream_t stream);
 int raster_group(bool gated, int tiles_q);  // activation-row tiles per raster band of the tiled kernels
 // The 256 x 256 kernel on v_mfma_f32_16x16x32 (kernels_pair16.hip) for GemmArgs::layout 0, 1, 3, 5, 7.
 // gated: X blocked in (bit 0), H blocked out (bit 1) or row-major, W13 blocked (bit 2) or row-major: layouts 1, 3, 5, 7;
@@ -75,7 +72,33 @@ SplitPlan tiled_split_plan(int np, int nq, int k);
 // activation rows per tile (256, 224, 192, 160) of the 256-weight-row kernel on row-major operands; a narrow one is
 // returned only if its estimated time is below `need` times that of 256
 int pair16_tile_rows(bool gated, long long np, long long nq, double need);
-hipError_t launch_tiled_splitk(int dtype, int tile, const GemmArgs& a, hipStream_t stream);  // a.splits, a.partial set
+hipError_t launch_tiled_splitk(int dtype, int tile, const GemmArgs& a, hipStream_t stream);  // tile 160 .. 256; a.splits, a.partial set
+// estimated time, us, of the 256-row gate/up kernel on rows that are no whole lines (`rows` activation rows a tile)
+double pair16_ragged_time(int np, int nq, int k, int rows);
+// the same for the plan of a split down projection (SplitPlan::tile 160 .. 256)
+double pair16_split_time(int np, int nq, int k, const SplitPlan& plan);
+
+hipError_t launch_splitk_reduce(int dtype, const GemmArgs& a, hipStream_t stream);  // sums a.partial's a.splits parts into a.O
+
+// Producer / consumer kernel (kernels_mid.hip): tiles of 64 .. 256 weight rows x 32 .. 256 activation rows.
+struct MidPlan {
+  int tile;    // index of the tile, -1: none
+  int step;    // weight rows a workgroup owns (<= the tile's, a multiple of 8)
+  int splits;  // K parts
+  double us;   // estimated time
+};
+// The plan of least estimated time. ragged: rows that are not whole 128-byte lines. splits: K parts, 0 = as many as pay, at most
+// max_splits (the gated product is never split: pass 1).
+MidPlan mid_plan(bool gated, int np, int nq, int k, bool ragged, int splits, int max_splits);
+int mid_tile_count();
+int mid_tile_rows(int tile);  // weight rows of a whole tile
+int mid_tile_index(int bp, int bq);
+const char* mid_name(const MidPlan& p);
+inline bool mid_ragged(const GemmArgs& a) {
+  return a.ldp % 64 != 0 || a.ldq % 64 != 0 || (((uintptr_t)a.P | (uintptr_t)a.Q) & 127) != 0;
+}
+// a.splits > 1: partial sums to a.partial, then their sum to a.O
+hipError_t launch_mid(int dtype, bool gated, const MidPlan& p, const GemmArgs& a, hipStream_t stream);
 
 // Weight-streaming kernels for M <= 16 activation rows (kernels_skinny.hip).
 struct SkinnyPlan {

@@ -201,7 +201,8 @@ FSW_API int fsw_version(void);
  * variants 115, 116, 117 = the 256-row kernel with 160, 192, 224 activation rows per tile (row-major operands);
  * family 1 variant 104 makes fsw_mlp run the down projection of M <= 32 rows on the split-K streaming kernel
  * (32-row tiles, two K ranges whose partial tiles meet through ticket counters that the gate/up kernel zeroes)
- * whatever the shape; the dispatcher picks it for 17 .. 32 rows of large weight matrices.
+ * whatever the shape (nothing selects it by itself: K parts on the producer / consumer kernel are faster);
+ * variants 200 + i = tile i of the producer / consumer kernel, whole tiles.
  * Returns FSW_E_VARIANT for unknown ids.
  */
 FSW_API int fsw_set_variant(int family, int variant);
@@ -218,10 +219,13 @@ FSW_API int fsw_set_variant(int family, int variant);
  */
 FSW_API int fsw_decode_barrier_failures(void);
 
-/* Name of the kernel variant the dispatcher picks for this shape (static storage); "splitk_<kernel>" when the
- * down projection splits K (family 1; K_or_FF decides). family 2: the down projection as fsw_mlp runs it (differs
- * from family 1, which is fsw_down on its own, for 17 .. 32 rows: "stream_split", and where H stays panel-blocked:
- * "pair16_256x256" also for row counts that fsw_down runs on narrower tiles). */
+/* Families 0 (gate/up), 1 (fsw_down) and 2 (the down projection inside fsw_mlp): name of the dispatcher's range that this
+ * shape falls in (static storage): "skinny", "decode_stream" (up to 48 rows, weight streaming), "stream_split" (17 .. 32 rows of
+ * large layers inside fsw_mlp), "dma_*" (up to 64, 128, 192, 256 rows to share the weights, and small problems), "pair16_*"
+ * (tiles of 256 weight rows); "splitk_<name>" when the down projection splits K. What fsw_set_variant forces has these names.
+ * Families 3, 4 and 5 (of 0, 1 and 2): the kernel that runs there, for operands whose rows are as long as K_or_FF: "mid_<rows of
+ * weights>x<rows of activations>" for the producer / consumer kernel, which serves most of the first four ranges, else the name
+ * above. */
 FSW_API const char* fsw_variant_name(int family, int dtype, int64_t M, int64_t N_or_D, int64_t K_or_FF);
 
 #ifdef __cplusplus

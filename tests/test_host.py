@@ -378,3 +378,31 @@ def test_static_forward_refuses_what_cannot_fit(capi):
     L = capi.lib()
     assert L.fsw_mlp_static(0, 2341, 4096, 14336, None, 4096, None, 4096, None, 14336, None, 4096,
                             None) == capi.E_STATIC_LIMIT
+
+
+def test_kernels_that_run_in_the_ranges_of_few_rows(capi):
+    """Families 3 .. 5 name the kernel: the producer / consumer kernel with its tile where it is the faster one, the
+    weight-streaming kernel for short calls, the 256-row kernel above; a forced tile keeps its own."""
+    runs = lambda fam, M, n, k: capi.variant_name(fam, 0, M, n, k)
+    assert runs(3, 1, 5632, 1024) == "skinny" and runs(4, 16, 1024, 2816) == "skinny" and runs(4, 16, 4096, 14336) == "skinny"
+    assert runs(3, 1, 28672, 4096).startswith("mid_") and runs(4, 1, 5120, 13824).startswith("mid_")
+    assert runs(3, 130, 22016, 4096) == "mid_96x160" and runs(3, 40, 38880, 5800) == "mid_160x64"
+    assert runs(5, 24, 4096, 11008).startswith("mid_") and runs(4, 200, 4096, 14336) == "mid_128x224"
+    assert runs(3, 333, 28672, 4096) == "pair16_256x192" and runs(5, 8192, 4096, 14336) == "pair16_256x256"
+    assert runs(3, 256, 38880, 5800).startswith("mid_") and runs(3, 256, 57344, 8192) == "pair16_256x256"
+    assert runs(3, 0, 64, 64) == "none" and capi.variant_name(6, 0, 1, 64, 64) == "invalid"
+    L = capi.lib()
+    try:
+        assert L.fsw_set_variant(0, 200) == capi.OK and runs(3, 100, 5632, 1024) == "mid_32x32" == runs(0, 100, 5632, 1024)
+        assert L.fsw_set_variant(0, 236) == capi.E_VARIANT and L.fsw_set_variant(0, 199) == capi.E_VARIANT
+    finally:
+        L.fsw_set_variant(0, -1)
+
+
+def test_static_forward_keeps_its_parts_within_its_array(capi):
+    """Few-row down projections split K as far as scratch allows; the workspace query and the plan agree on it."""
+    L = capi.lib()
+    for M, D, FF in ((20, 4096, 11008), (40, 5120, 13824), (200, 3000, 8008), (256, 8192, 28672)):
+        nbytes = L.fsw_down_workspace_bytes(0, M, D, FF)
+        assert nbytes > 0 and nbytes % (4 * M * D) == 0 and 2 <= nbytes // (4 * M * D) <= 16
+        assert L.fsw_mlp_workspace_bytes(0, M, D, FF) == (M * FF * 2 + 255) // 256 * 256 + (nbytes + 255) // 256 * 256

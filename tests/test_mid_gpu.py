@@ -1,0 +1,117 @@
+"""The producer / consumer kernel (kernels_mid.hip): every tile at its edges, rows that start anywhere in a 128-byte line, K
+tails, K parts, pieces lower than the tile. Against the fp64 oracle under "one rounding of the exact value" (half an ulp of the
+result, twice, plus 1e-3 for fp32 sums in another order), and bit for bit between equal problems that lie differently in memory:
+where a row starts moves its bytes in LDS, not the order of the sums."""
+import pytest
+import torch
+
+from oracle import oracle
+import fsw_weights
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+N_TILES = 36
+
+
+def assert_one_rounding(out, ref64, dtype, what):
+    err = (out.detach().cpu().double() - ref64).abs()
+    bound = ref64.abs() * (2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10) + 1e-3
+    assert not (err > bound).any(), "%s: worst excess %g" % (what, (err - bound).max().item())
+
+
+def lay(t, pad, offset):
+    """The same matrix inside a NaN-filled buffer, rows `pad` elements longer, its start `offset` elements past a 256-byte line."""
+    rows, cols = t.shape
+    buf = torch.full((rows * (cols + pad) + offset + 128,), float("nan"), dtype=t.dtype, device=DEV)
+    view = buf[offset:offset + rows * (cols + pad)].view(rows, cols + pad)[:, :cols]
+    view.copy_(t)
+    return view
+
+
+def tile_rows(capi, index):
+    """(weight rows, activation rows) of a forced tile, from its name."""
+    try:
+        assert capi.lib().fsw_set_variant(0, 200 + index) == capi.OK
+        name = capi.variant_name(0, 0, 64, 512, 64)
+    finally:
+        capi.set_variant(0, -1)
+    assert name.startswith("mid_")
+    return tuple(int(x) for x in name[4:].split("x"))
+
+
+@pytest.mark.parametrize("index", range(N_TILES))
+def test_every_tile_at_its_edges(capi, index):
+    """Rows one past the tile in both directions (the second tiles hold one row each), K of less than a line, of whole lines, with a
+    tail; gate/up and the plain product; dense rows and rows at every sixteenth of a line beside NaN."""
+    bp, bq = tile_rows(capi, index)
+    for n, (M, ff, K) in enumerate([(bq + 1, bp // 2 + 4, 200), (bq, bp // 2, 8), (bq - 1, bp // 2 + 3, 328), (bq + 1, bp // 2 - 1, 256)]):
+        dtype = torch.float16 if n % 2 else torch.bfloat16
+        inp = fsw_weights.make_inputs(M, K, ff, dtype, seed=97 * index + n, x_scale=0.5)
+        want = oracle.ref_gateup(inp["X"], inp["W13"], torch.float64)
+        plain = inp["X"].double() @ inp["W13"].double().t()
+        first = None
+        for pad, xo, wo in ((0, 0, 0), (8 * (1 + index % 7), 8 * (1 + n), 8 * (index % 16)), (64 - K % 64, 0, 0)):
+            X, W = lay(inp["X"], pad, xo), lay(inp["W13"], pad, wo)
+            wide = torch.full((M, ff + 8), float("nan"), dtype=dtype, device=DEV)
+            try:
+                capi.set_variant(0, 200 + index)
+                capi.set_variant(1, 200 + index)
+                capi.gateup(X, W, out=wide[:, :ff])
+                P = capi.down(X, W)
+            finally:
+                capi.set_variant(0, -1)
+                capi.set_variant(1, -1)
+            what = "tile %d (%d x %d) %s pad %d" % (index, bp, bq, (M, ff, K), pad)
+            assert torch.isnan(wide[:, ff:]).all(), what
+            assert_one_rounding(wide[:, :ff], want, dtype, what)
+            assert_one_rounding(P, plain, dtype, what + " plain")
+            if M > bq:  # two tiles of rows: no workgroup starts its K walk elsewhere
+                first = first if first is not None else (wide.clone(), P)
+                assert torch.equal(wide[:, :ff], first[0][:, :ff]) and torch.equal(P, first[1]), what
+
+
+@pytest.mark.parametrize("M", [1, 8, 17, 33, 100, 200, 300])
+@pytest.mark.parametrize("D,FF", [(1096, 8008), (1024, 16384), (3000, 4872)])
+def test_down_projection_in_parts_of_k(capi, M, D, FF):
+    """K parts whose bounds fall inside lines: the parts of one line go to two workgroups and are summed once. H beside NaN, and the
+    same numbers from a padded layout."""
+    inp = fsw_weights.make_inputs(M, D, FF, torch.bfloat16, seed=M + FF, x_scale=0.5)
+    H = torch.randn(M, FF, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16) * 0.3
+    ref = oracle.ref_down(H, inp["W2"], torch.float64)
+    Y = capi.down(lay(H, 0, 0), lay(inp["W2"], 0, 0))
+    assert_one_rounding(Y, ref, torch.bfloat16, "parts %s" % ((M, D, FF),))
+    for pad, ho, wo in ((8, 8, 24), (64 - FF % 64, 0, 64)):
+        assert_one_rounding(capi.down(lay(H, pad, ho), lay(inp["W2"], pad, wo)), ref, torch.bfloat16, "pad %d" % pad)
+    assert torch.equal(capi.mlp(*(inp[k].to(DEV) for k in ("X", "W13", "W2"))), capi.down(
+        capi.gateup(inp["X"].to(DEV), inp["W13"].to(DEV)), inp["W2"].to(DEV)))
+
+
+def test_down_projection_of_few_rows_runs_without_scratch(capi):
+    """Up to 48 rows the weight-streaming kernel needs none: a caller that brings no workspace gets that kernel, not an error."""
+    M, D, FF = 20, 2048, 8192
+    L = capi.lib()
+    assert L.fsw_down_workspace_bytes(0, M, D, FF) > 0 and capi.variant_name(4, 0, M, D, FF).startswith("mid_")
+    H = (torch.randn(M, FF, device=DEV) * 0.3).to(torch.bfloat16)
+    W2 = (torch.randn(D, FF, device=DEV) / FF ** 0.5).to(torch.bfloat16)
+    Y = torch.empty(M, D, dtype=torch.bfloat16, device=DEV)
+    assert L.fsw_down(0, M, D, FF, H.data_ptr(), FF, W2.data_ptr(), FF, Y.data_ptr(), D, None, 0,
+                      torch.cuda.current_stream().cuda_stream) == capi.OK
+    assert_one_rounding(Y, oracle.ref_down(H.cpu(), W2.cpu(), torch.float64), torch.bfloat16, "no scratch")
+
+
+@pytest.mark.parametrize("M,d,ff", [(1, 4096, 14336), (16, 3000, 8008), (40, 2048, 8192), (130, 4096, 11008), (200, 3000, 8008),
+                                    (300, 3960, 8040), (512, 1024, 2816), (700, 1320, 3000)])
+def test_chosen_tiles_against_the_256_row_kernel(capi, M, d, ff):
+    """What the dispatcher chooses (pieces lower than the tile included) against the 256-row kernel, which takes any problem: every
+    feature, both sums rounded once; and repeated calls bit for bit."""
+    assert capi.variant_name(3, 0, M, 2 * ff, d).startswith("mid_")
+    inp = fsw_weights.make_inputs(M, d, ff, torch.bfloat16, seed=d, x_scale=1.0)
+    X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
+    H = capi.gateup(X, W)
+    try:
+        capi.set_variant(0, 5)
+        big = capi.gateup(X, W)
+    finally:
+        capi.set_variant(0, -1)
+    assert ((H.float() - big.float()).abs() <= 2.0 ** -7 * big.float().abs() + 1e-3).all()
+    assert all(torch.equal(capi.gateup(X, W), H) for _ in range(3))
