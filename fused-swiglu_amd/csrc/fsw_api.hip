@@ -534,9 +534,18 @@ int fsw_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H, int64_t
   return down_impl(dtype, M, D, FF, H, ldh, W2, ldw2, Y, ldy, workspace, workspace_bytes, SIZE_MAX, stream);
 }
 
-static size_t h_bytes(int64_t M, int64_t FF) {
-  const size_t raw = (size_t)M * (size_t)FF * 2;
+static size_t h_bytes(int64_t M, int64_t ldh) {
+  const size_t raw = (size_t)M * (size_t)ldh * 2;
   return (raw + 255) & ~(size_t)255;
+}
+
+// Row stride of row-major H between the two kernels of fsw_mlp: whole 128-byte lines above 256 rows, where the caller's scratch has
+// room for them beside the `need` bytes of dense H and the partial sums. The 256-row kernel fetches a row that starts inside a line by
+// K tiles that lie in two lines. Forward, us, dense -> whole lines: 4096 x 14344 5000 rows 1480 -> 1394, 1200 rows 400 -> 383; 3488 x
+// 11656 2500 rows 554 -> 532; 3000 x 8008 600 rows 120.1 -> 117.3. Up to 256 rows, where mid_kernel copies whole lines anyway, level.
+static int64_t h_stride(int64_t M, int64_t FF, size_t need, size_t workspace_bytes) {
+  const int64_t lines = (FF + 63) / 64 * 64;
+  return M > 256 && need - h_bytes(M, FF) + h_bytes(M, lines) <= workspace_bytes ? lines : FF;
 }
 
 // what row-major H leaves of `scratch` bytes (SIZE_MAX: no limit) for the down projection's partial sums
@@ -772,29 +781,30 @@ static int mlp_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* X, 
     if (rc != FSW_OK) return rc;
     return fsw_down_blocked(dtype, M, D, FF, workspace, W2, ldw2, 0, Y, ldy, stream);
   }
-  unsigned char* ws2 = (unsigned char*)workspace + h_bytes(M, FF);
+  const int64_t ldh = FF > 0 ? h_stride(M, FF, need, workspace_bytes) : 0;
+  unsigned char* ws2 = (unsigned char*)workspace + h_bytes(M, ldh);
   if (stream_split_runs(M, D, FF)) {
     const fsw::StreamPlan sp = mlp_stream_plan(M, D, FF);
     // the gate/up kernel zeroes the ticket counters of the split-K streaming down projection
     unsigned* tickets = (unsigned*)(ws2 + sp.partial_bytes);
-    rc = gateup_impl(dtype, M, 2 * FF, D, X, ldx, W13, ldw13, Hbuf, FF, stream, tickets, sp.ticket_words);
+    rc = gateup_impl(dtype, M, 2 * FF, D, X, ldx, W13, ldw13, Hbuf, ldh, stream, tickets, sp.ticket_words);
     if (rc != FSW_OK) return rc;
     fsw::GemmArgs a;
     a.P = W2;
     a.Q = Hbuf;
     a.O = Y;
     a.ldp = ldw2;
-    a.ldq = FF;
+    a.ldq = ldh;
     a.ldo = ldy;
     a.np = (int)D;
     a.nq = (int)M;
     a.k = (int)FF;
     return finish(fsw::launch_stream_split(dtype, a, sp, ws2, (hipStream_t)stream));
   }
-  const size_t down_ws = workspace_bytes > h_bytes(M, FF) ? workspace_bytes - h_bytes(M, FF) : 0;
-  rc = fsw_gateup(dtype, M, 2 * FF, D, X, ldx, W13, ldw13, Hbuf, FF, stream);
+  const size_t hb = h_bytes(M, ldh), down_ws = workspace_bytes > hb ? workspace_bytes - hb : 0;
+  rc = fsw_gateup(dtype, M, 2 * FF, D, X, ldx, W13, ldw13, Hbuf, ldh, stream);
   if (rc != FSW_OK) return rc;
-  return down_impl(dtype, M, D, FF, Hbuf, FF, W2, ldw2, Y, ldy, ws2, down_ws, beside_h(M, FF, scratch), stream);
+  return down_impl(dtype, M, D, FF, Hbuf, ldh, W2, ldw2, Y, ldy, ws2, down_ws, beside_h(M, FF, scratch), stream);
 }
 
 int fsw_mlp(int dtype, int64_t M, int64_t D, int64_t FF, const void* X, int64_t ldx, const void* W13, int64_t ldw13,

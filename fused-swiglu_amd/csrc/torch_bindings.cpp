@@ -141,7 +141,8 @@ Tensor fused_swiglu_mlp_typed(at::ScalarType want, Tensor const& X, Tensor const
   const at::hip::OptionalHIPGuardMasqueradingAsCUDA device_guard(device_of(X));
   const int code = dtype_code(want);
   // one call: H (panel-blocked for large problems) and the split-K partials live in this scratch, never as a tensor
-  const size_t ws_bytes = fsw_mlp_workspace_bytes(code, M, D, FF);
+  // (with room for whole 128-byte lines where H's rows are none: fsw.h)
+  const size_t ws_bytes = fsw_mlp_workspace_bytes(code, M, D, FF) + (M > 256 && FF % 64 != 0 ? (size_t)M * 128 : 0);
   Tensor ws = at::empty({(int64_t)std::max<size_t>(ws_bytes, 16)}, X.options().dtype(at::kByte));
   const int rc = fsw_mlp(code, M, D, FF, X.data_ptr(), M > 1 ? X.stride(0) : D, W1W3.data_ptr(),
                          N > 1 ? W1W3.stride(0) : D, W2.data_ptr(), D > 1 ? W2.stride(0) : FF, Y.data_ptr(), D,

@@ -108,7 +108,8 @@ FSW_API int fsw_down(int dtype, int64_t M, int64_t D, int64_t FF,
              void* workspace, size_t workspace_bytes, void* stream);
 
 /* Bytes of device scratch fsw_mlp needs: the H[M, FF] intermediate (panel-blocked in the large-tile regime) plus the
- * scratch of its down projection. */
+ * scratch of its down projection. With 128 * M bytes more, rows of H are whole 128-byte lines where FF % 64 != 0 and M > 256: the
+ * same result, 1 .. 6 % sooner (the torch module allocates that). */
 FSW_API size_t fsw_mlp_workspace_bytes(int dtype, int64_t M, int64_t D, int64_t FF);
 
 /*

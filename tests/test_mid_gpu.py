@@ -115,3 +115,23 @@ def test_chosen_tiles_against_the_256_row_kernel(capi, M, d, ff):
         capi.set_variant(0, -1)
     assert ((H.float() - big.float()).abs() <= 2.0 ** -7 * big.float().abs() + 1e-3).all()
     assert all(torch.equal(capi.gateup(X, W), H) for _ in range(3))
+
+
+@pytest.mark.parametrize("M,d,ff", [(20, 1024, 4104), (257, 520, 2056), (700, 520, 2120), (2049, 264, 1000), (2700, 4096, 3592)])
+def test_forward_with_h_in_whole_lines(capi, M, d, ff):
+    """With 128 bytes a row more scratch than the query asks for, rows of H are whole lines above 256 rows; what lies between them is
+    never read. Scratch full of NaN; against float64, and against the forward on the queried scratch (dense H): the same bits, as no
+    sum changes its order."""
+    gen = torch.Generator(device=DEV).manual_seed(M + ff)
+    X = torch.randn(M, d, generator=gen, device=DEV).to(torch.bfloat16)
+    W13 = (torch.randn(2 * ff, d, generator=gen, device=DEV) / d ** 0.5).to(torch.bfloat16)
+    W2 = (torch.randn(d, ff, generator=gen, device=DEV) / ff ** 0.5).to(torch.bfloat16)
+    queried = capi.mlp_workspace(X, ff)
+    ys = []
+    for extra in (0, 128 * M - 2, 128 * M):
+        ws = torch.full((queried.numel() + extra,), 255, dtype=torch.uint8, device=DEV)
+        ys.append(capi.mlp(X, W13, W2, workspace=ws))
+    pre = X.double() @ W13.double().T
+    H = (pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2]))
+    oracle.assert_parity(ys[2], (H @ W2.double().T).cpu(), "H in whole lines %s" % ((M, d, ff),))
+    assert torch.equal(ys[0], ys[2]) and torch.equal(ys[0], ys[1])
