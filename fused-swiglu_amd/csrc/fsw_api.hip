@@ -146,10 +146,10 @@ bool ragged(int64_t k) { return k % 64 != 0; }
 // where its workgroups fit the compute units at once and the call is short. Gate/up, us, skinny -> mid: 5632 x 1024 (176
 // workgroups) 16 rows 5.1 -> 6.4; 8192 x 1536 (256) 24 rows 7.4 -> 8.1; 11264 x 2048 (352) 4 rows 10.5 -> 10.8, 16 rows 11.7 ->
 // 10.9, 24 rows 15.4 -> 11.0; 7808 x 1320 (244, ragged) 4 rows 6.7 -> 7.2, 24 rows 8.0 -> 7.3; 16016 x 3000 (ragged) 1 row 22.0 ->
-// 19.4. Down, where K is split and a summing launch follows: 2816 -> 1024 16 rows 6.1 -> 6.4; 8192 -> 3072 16 rows 12.4 -> 13.1,
-// 24 rows 15.2 -> 13.4; 8192 -> 2048 1 row level, 16 rows 12.1 -> 10.7; 13824 -> 5120 (320 workgroups, two rounds) 1 row 31.3 ->
-// 25.2; ragged 3640 -> 1096 4 rows 6.6 -> 6.8, 16 rows 8.0 -> 7.3; 5360 -> 1344 1 row 8.1 -> 7.8, 16 rows 10.7 -> 8.4; 16416 ->
-// 4880 1 row 40.5 -> 28.7. Matrices of the persistent streaming kernel (decode_stream_wanted): gate/up 57344 x 8192 1 row 144.1 ->
+// 19.4. Down, where K is split and a summing launch follows: 8192 -> 3072 16 rows 12.4 -> 13.1, 24 rows 15.2 -> 13.4; 13824 ->
+// 5120 (320 workgroups, two rounds) 1 row 31.3 -> 25.2; 16416 -> 4880 (ragged) 1 row 40.5 -> 28.7; up to 2048 features, where
+// skinny_kernel has 4 or 8 a workgroup, 2816 -> 1024 16 rows 4.7 -> 6.4, 8192 -> 2048 16 rows 10.1 -> 10.7, 16384 -> 2048 1 row
+// 16.2 -> 14.2, 16 rows 19.6 -> 15.2; ragged 5360 -> 1344 1 row 6.3 -> 8.1, 12 rows 8.2 -> 8.4, 16 rows 9.0 -> 8.4. Matrices of the persistent streaming kernel (decode_stream_wanted): gate/up 57344 x 8192 1 row 144.1 ->
 // 142.4, 16 rows 147.4 -> 136.5; 46336 x 7000 (ragged) 1 row 124.0 -> 98.8; down 28672 -> 8192 1 and 4 rows level, 16 rows
 // 84.1 -> 72.1; 23168 -> 7000 1 row 55.5 -> 52.1.
 // The 256-row kernel fetches rows that are no whole lines by K tiles, every line twice; the gate/up product of such rows takes the
@@ -171,9 +171,10 @@ bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
   }
   const int64_t tiles = (np + 15) / 16;
   if (m > 16) return rag || bytes >= (int64_t)8 << 20;
+  if (tiles <= 128) return k > 12288 ? m > 4 || np > 1024 : rag && m > 12 && bytes >= (int64_t)12 << 20;
   if (rag) return bytes >= (int64_t)14 << 20 || (m >= 8 && bytes >= (int64_t)7 << 20);
   if (bytes >= (int64_t)1 << 28) return m > 4;
-  return tiles > 256 || (tiles <= 128 && k >= 8192);
+  return tiles > 256;
 }
 
 // tile of a forced variant

@@ -3,7 +3,7 @@
 // With so few activation rows every weight byte is used once: the kernels are bound by HBM bandwidth, and the
 // job is to keep ~100 KB of 16-byte loads in flight per CU with perfectly coalesced addresses.
 //
-// A workgroup owns one tile of 16 output features (16 weight rows; for the gated kernel the 16 "up" rows
+// A workgroup owns one tile of 16 output features (8 or 4 where the plain product is narrow; 16 weight rows; for the gated kernel the 16 "up" rows
 // 2j and the 16 "gate" rows 2j+1, j in the tile) and its NW waves split K between them. Per step a wave
 //   1. loads 128 K-elements (256 contiguous bytes) of each of its rows, 16 lanes per row, 16 bytes per lane
 //      (each load instruction covers 4 rows x 256 B); the data of step s+1 is in flight while step s computes;
@@ -22,11 +22,14 @@
 
 namespace fsw {
 
-template <class E, bool GATED, int MQ, int NW, bool XSLAB>
+// RS: weight rows (features) of a set, 16, or 8 or 4 where 16 would leave compute units idle (skinny_plan). The MFMA always takes 16
+// rows: the others repeat and are not stored.
+// U: steps whose loads are in flight at once; fewer rows a workgroup need more of them.
+template <class E, bool GATED, int MQ, int NW, bool XSLAB, int RS = 16, int U = 1>
 __global__ void __launch_bounds__(NW * 64)
 skinny_kernel(const GemmArgs a) {
   constexpr int T = GATED ? 2 : 1;   // accumulator sets (up, gate)
-  constexpr int R = 16 * T;          // weight rows per tile
+  constexpr int R = RS * T;          // weight rows per tile
   constexpr int NL = R / 4;          // weight loads per lane per step
   constexpr int KS = 128;            // K elements per step
   // Activations pass through the slab too: fetched like weights, 16 lanes per row, every 16-lane pass of a load
@@ -35,7 +38,7 @@ skinny_kernel(const GemmArgs a) {
   // reuse the same bytes: LDS serves a wave's accesses in order. Measured on whole forwards at 4096 x 14336:
   // M = 16: 63.7 -> 61.0 us, M = 32: 85.8 -> 73.0, M = 64: 134.5 -> 98.1; with few activation rows the direct fetch
   // touches few lines per pass anyway (M = 3: 1.3 % faster, M = 8: level), so XSLAB is off for nq <= 8.
-  constexpr int SLAB = R * 256;      // bytes of one wave's transpose buffer
+  constexpr int SLAB = R * 256 > 4096 ? R * 256 : 4096;  // bytes of one wave's transpose buffer (16 activation rows: 4 KB)
   static_assert(MQ * T * 1024 <= SLAB, "the reduction reuses the slabs");
   __shared__ __align__(16) unsigned char lds[NW * SLAB];
 
@@ -64,7 +67,7 @@ skinny_kernel(const GemmArgs a) {
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int row = 4 * i + (lane >> 4);
-    const int grow = GATED ? (row < 16 ? 2 * row : 2 * (row - 16) + 1) : row;
+    const int grow = GATED ? (row < RS ? 2 * row : 2 * (row - RS) + 1) : row;
     const int lc = pc ^ (row & 7);
     woff[i] = (unsigned)grow * (unsigned)a.ldp * 2u + (unsigned)lc * 16u;
   }
@@ -75,6 +78,12 @@ skinny_kernel(const GemmArgs a) {
   unsigned rd[4];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) rd[kk] = (unsigned)r16 * 256u + (unsigned)(((4 * kk + q) ^ (r16 & 7)) * 16);
+
+  // (weights, fewer rows than 16: row r16 modulo RS)
+  unsigned rdw[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    rdw[kk] = (unsigned)(r16 & (RS - 1)) * 256u + (unsigned)(((4 * kk + q) ^ (r16 & (RS - 1) & 7)) * 16);
 
   // activation fragments straight from global memory (L2 resident): lane -> row 16 mq + r16, K chunk q
   unsigned xoff[MQ];
@@ -96,9 +105,11 @@ skinny_kernel(const GemmArgs a) {
   }
   const unsigned xblock = 16u * (unsigned)a.ldq * 2u;  // bytes between 16-row activation blocks
 
-  u32x4 wreg[NL];
-  u32x4 xreg[MQ][4];
-  auto g_load = [&](int step) {
+  u32x4 wregs[U][NL];
+  u32x4 xregs[U][MQ][4];
+  auto g_load = [&](int step, int set) {
+    u32x4(&wreg)[NL] = wregs[set];
+    u32x4(&xreg)[MQ][4] = xregs[set];
     const int k0 = step * KS;
     const unsigned kb = (unsigned)k0 * 2u;
 #pragma unroll
@@ -129,8 +140,9 @@ skinny_kernel(const GemmArgs a) {
     }
   };
 
-  if (s_begin < s_end) g_load(s_begin);
-  for (int step = s_begin; step < s_end; ++step) {
+  auto one_step = [&](int step, int set) {
+    u32x4(&wreg)[NL] = wregs[set];
+    u32x4(&xreg)[MQ][4] = xregs[set];
     // registers -> slab (waits for this step's loads), then free the registers for the next step's loads
     u32x4 xcur[MQ][4];
     if constexpr (XSLAB) {
@@ -150,16 +162,24 @@ skinny_kernel(const GemmArgs a) {
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) xcur[mq][kk] = xreg[mq][kk];
     }
-    if (step + 1 < s_end) g_load(step + 1);
+    if (step + U < s_end) g_load(step + U, set);
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
 #pragma unroll
       for (int s = 0; s < T; ++s) {
-        const u32x4 wf = *(const u32x4*)(slab + s * 4096 + rd[kk]);
+        const u32x4 wf = *(const u32x4*)(slab + s * RS * 256 + rdw[kk]);
 #pragma unroll
         for (int mq = 0; mq < MQ; ++mq) acc[s][mq] = E::mfma16(wf, xcur[mq][kk], acc[s][mq]);
       }
     }
+  };
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (s_begin + u < s_end) g_load(s_begin + u, u);
+  for (int step = s_begin; step < s_end; step += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (step + u < s_end) one_step(step + u, u);
   }
 
   // ---- cross-wave reduction through LDS, then epilogue by the first MQ waves
@@ -188,7 +208,7 @@ skinny_kernel(const GemmArgs a) {
     const int m = 16 * mq + r16;
     const int nout = GATED ? a.np / 2 : a.np;
     const int n = (GATED ? p0 / 2 : p0) + 4 * q;
-    if (m < a.nq) {
+    if (m < a.nq && 4 * q < RS) {
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = GATED ? sum[0][e] * silu_f32(sum[T - 1][e]) : sum[0][e];
@@ -219,18 +239,18 @@ skinny_kernel(const GemmArgs a) {
 
 namespace {
 
-template <class E, bool GATED, int MQ, int NW>
+template <class E, bool GATED, int MQ, int NW, int RS = 16, int U = 1>
 hipError_t launch_skinny_one(const GemmArgs& a, hipStream_t stream) {
-  constexpr int R = GATED ? 32 : 16;
+  constexpr int R = GATED ? 2 * RS : RS;
   const int tiles = (a.np + R - 1) / R;
   if (tiles <= 0) return hipSuccess;
   if constexpr (MQ == 1) {
     if (a.nq <= 8) {
-      hipLaunchKernelGGL((skinny_kernel<E, GATED, MQ, NW, false>), dim3((unsigned)tiles), dim3(NW * 64), 0, stream, a);
+      hipLaunchKernelGGL((skinny_kernel<E, GATED, MQ, NW, false, RS, U>), dim3((unsigned)tiles), dim3(NW * 64), 0, stream, a);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((skinny_kernel<E, GATED, MQ, NW, true>), dim3((unsigned)tiles), dim3(NW * 64), 0, stream, a);
+  hipLaunchKernelGGL((skinny_kernel<E, GATED, MQ, NW, true, RS, U>), dim3((unsigned)tiles), dim3(NW * 64), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -278,6 +298,18 @@ hipError_t launch_skinny(int dtype, bool gated, const GemmArgs& a, void* workspa
   (void)workspace;
   if (a.nq > 64) return hipErrorInvalidValue;
   const int mq = (a.nq + 15) / 16;
+  // Narrow outputs of the plain product: 16 features a workgroup are 64 .. 128 workgroups, each bound by what one compute unit
+  // fetches; 8 (4) features are twice (four times) as many, and their waves need two steps (or twice the waves) in flight. us: 2816 ->
+  // 1024 1 row 4.7 -> 4.2, 16 rows 5.9 -> 4.7; 4096 -> 1536 6.1 -> 5.2, 7.2 -> 6.3; 5632 -> 2048 8.0 -> 6.5, 9.7 -> 8.1; 8192 -> 2048 9.9
+  // -> 8.0. Not with a second round of workgroups (8192 -> 3072 10.0 -> 12.9), not
+  // for a handful of features (1024 -> 256 2.5 -> 2.7), and the gated product has two rows a feature as it is
+  // (5632 x 1024 4.4 -> 4.9). Eight waves of two steps against sixteen of one and of two, eight of four: 2 .. 8 % less.
+  if (!gated && mq == 1 && a.np >= 512 && a.np <= 2048) {
+    if (a.np <= 1024) {
+      return dtype == 0 ? launch_skinny_one<Bf16, false, 1, 16, 4, 1>(a, stream) : launch_skinny_one<Fp16, false, 1, 16, 4, 1>(a, stream);
+    }
+    return dtype == 0 ? launch_skinny_one<Bf16, false, 1, 8, 8, 2>(a, stream) : launch_skinny_one<Fp16, false, 1, 8, 8, 2>(a, stream);
+  }
   const int nw = skinny_plan(gated, a.np, a.nq, a.k).splits;
   if (dtype == 0) {
     return gated ? launch_skinny_mq<Bf16, true>(mq, nw, a, stream) : launch_skinny_mq<Bf16, false>(mq, nw, a, stream);
