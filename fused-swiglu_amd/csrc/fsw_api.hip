@@ -455,7 +455,7 @@ static DownPlan down_plan(int64_t M, int64_t D, int64_t FF, size_t limit, bool r
   // rows that are no whole lines: the same parts on whichever kernel takes them faster by the estimates (8008 -> 3000 300 rows
   // 39.6 -> 28.8 us, 900 rows 62.9 -> 58.8; 23568 -> 6168 499 rows stays, 152 and 189)
   if (!r.mid && rag && r.plan.splits > 1 && M <= 1024)
-    r.mid = fsw::mid_plan(false, (int)D, (int)M, (int)FF, true, r.plan.splits, r.plan.splits).us <
+    r.mid = fsw::mid_plan(false, (int)D, (int)M, (int)FF, true, 0, r.plan.splits).us <
             0.95 * fsw::pair16_split_time((int)D, (int)M, (int)FF, r.plan);
   return r;
 }
@@ -501,9 +501,13 @@ static int down_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* H,
   if (plan.mid) {
     a.splits = need > 0 ? plan.plan.splits : 1;
     a.partial = (float*)workspace;
+    // Above 256 rows the plan's parts are the most there is scratch for: fewer, or none, where smaller tiles fill the chip without
+    // them. us: 2088 -> 736 1996 rows 17.8 -> 14.1; 2816 -> 1024 512 rows 14.8 -> 13.4, 900 rows 17.6 -> 15.3; 8192 -> 2048 371 rows
+    // 27.0 -> 25.7; 12680 -> 3304 (ragged) 368 rows 60.3 -> 48.3; 50 problems 0.940 on average, worst 1.012.
     const fsw::MidPlan p = g_forced_variant[1] >= 0
                                ? forced_mid_plan(v)
-                               : fsw::mid_plan(false, (int)D, (int)M, (int)FF, fsw::mid_ragged(a), a.splits, a.splits);
+                               : fsw::mid_plan(false, (int)D, (int)M, (int)FF, fsw::mid_ragged(a), M > 256 ? 0 : a.splits, a.splits);
+    a.splits = p.splits;
     return finish(fsw::launch_mid(dtype, false, p, a, (hipStream_t)stream));
   }
   if (v == VARIANT_SKINNY) {
@@ -580,7 +584,8 @@ static const char* running_name(int family, int64_t M, int64_t N_or_D, int64_t K
   const DownPlan d = gated ? DownPlan{false, {0, 1}} : down_plan(M, N_or_D, K_or_FF, SIZE_MAX, rag);
   if (gated ? mid_wanted(0, v, M, N_or_D, K_or_FF, rag) : d.mid)
     return fsw::mid_name(g_forced_variant[f] >= 0 ? forced_mid_plan(v)
-                                                  : fsw::mid_plan(gated, (int)N_or_D, (int)M, (int)K_or_FF, rag, d.plan.splits, 1));
+                                                  : fsw::mid_plan(gated, (int)N_or_D, (int)M, (int)K_or_FF, rag,
+                                                                !gated && M > 256 ? 0 : d.plan.splits, d.plan.splits));
   return fsw_variant_name(f, FSW_BF16, M, N_or_D, K_or_FF);
 }
 

@@ -135,3 +135,22 @@ def test_forward_with_h_in_whole_lines(capi, M, d, ff):
     H = (pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2]))
     oracle.assert_parity(ys[2], (H @ W2.double().T).cpu(), "H in whole lines %s" % ((M, d, ff),))
     assert torch.equal(ys[0], ys[2]) and torch.equal(ys[0], ys[1])
+
+
+@pytest.mark.parametrize("M,D,FF", [(257, 264, 1032), (371, 2048, 8192), (300, 3000, 8008), (512, 1024, 2816), (700, 2048, 2056),
+                                    (1996, 736, 2088)])
+def test_fewer_parts_than_there_is_scratch_for(capi, M, D, FF):
+    """Above 256 rows the workspace query gives the most parts; the launch may take fewer. Scratch full of NaN, exactly as large as
+    the query says, a guard behind it."""
+    L = capi.lib()
+    H = (torch.randn(M, FF, device=DEV) * 0.3).to(torch.bfloat16)
+    W2 = (torch.randn(D, FF, device=DEV) / FF ** 0.5).to(torch.bfloat16)
+    nbytes = L.fsw_down_workspace_bytes(0, M, D, FF)
+    ws = torch.full((nbytes + 256,), 255, dtype=torch.uint8, device=DEV)
+    Y = torch.empty(M, D, dtype=torch.bfloat16, device=DEV)
+    assert nbytes > 0 and capi.variant_name(4, 0, M, D, FF).startswith("mid_")
+    for _ in range(2):
+        assert L.fsw_down(0, M, D, FF, H.data_ptr(), FF, W2.data_ptr(), FF, Y.data_ptr(), D, ws.data_ptr(), nbytes,
+                          torch.cuda.current_stream().cuda_stream) == capi.OK
+        assert (ws[nbytes:] == 255).all()
+        assert_one_rounding(Y, (H.double() @ W2.double().T).cpu(), torch.bfloat16, "parts %s" % ((M, D, FF),))
