@@ -466,6 +466,16 @@ static size_t down_split(int64_t M, int64_t D, int64_t FF, size_t limit, DownPla
   return plan->plan.splits > 1 ? plan->plan.splits * (size_t)M * (size_t)D * sizeof(float) : 0;
 }
 
+// Least scratch that the down projection accepts: more than that only buys K parts on the producer / consumer kernel, which runs with
+// as many of them as there is room for.
+static size_t down_least(int64_t M, int64_t D, int64_t FF, size_t limit) {
+  if (M <= 0 || D <= 0 || FF <= 0 || g_forced_variant[1] >= 0 || streams_weights(1, M, D, FF)) return 0;
+  const size_t part = (size_t)M * (size_t)D * sizeof(float);
+  size_t parts = (size_t)fsw::tiled_split_plan((int)D, (int)M, (int)FF).splits;
+  if (parts > limit / part) parts = limit / part;
+  return parts > 1 ? parts * part : 0;
+}
+
 size_t fsw_down_workspace_bytes(int dtype, int64_t M, int64_t D, int64_t FF) {
   (void)dtype;
   DownPlan plan;
@@ -480,10 +490,13 @@ static int down_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* H,
   DownPlan plan;
   size_t need = down_split(M, D, FF, limit, &plan);
   const int v = resolve_variant(1, M, D, FF);
-  if (need > 0 && (!workspace || workspace_bytes < need)) {
-    if (v != VARIANT_SKINNY) return FSW_E_WORKSPACE;
-    plan.mid = false;  // few rows: the weight-streaming kernel needs no scratch
-    need = 0;
+  const size_t room = workspace && aligned16(workspace) ? workspace_bytes : 0;
+  if (need > room) {
+    const size_t least = down_least(M, D, FF, limit);
+    if (least > 0 && (!workspace || workspace_bytes < least)) return FSW_E_WORKSPACE;
+    if (least > 0 && !aligned16(workspace)) return FSW_E_ALIGN;
+    need = down_split(M, D, FF, room < limit ? room : limit, &plan);
+    if (need == 0 && v == VARIANT_SKINNY) plan.mid = false;  // few rows: the weight-streaming kernel needs no scratch
   }
   const int drc = check_device();
   if (drc != FSW_OK) return drc;
@@ -497,7 +510,6 @@ static int down_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* H,
   a.np = (int)D;
   a.nq = (int)M;
   a.k = (int)FF;
-  if (need > 0 && !aligned16(workspace)) return FSW_E_ALIGN;
   if (plan.mid) {
     a.splits = need > 0 ? plan.plan.splits : 1;
     a.partial = (float*)workspace;
@@ -731,6 +743,15 @@ static size_t mlp_workspace(int64_t M, int64_t D, int64_t FF, size_t scratch) {
   return h_bytes(M, FF) + ((down_split(M, D, FF, beside_h(M, FF, scratch), &plan) + 255) & ~(size_t)255);
 }
 
+// The least scratch the forward accepts, `need` bytes being what its plan asks for: see down_least().
+static size_t mlp_least(int64_t M, int64_t D, int64_t FF, size_t scratch, size_t need) {
+  if (blocked_regime(M, D, FF, scratch) || stream_split_runs(M, D, FF)) return need;
+  const fsw::StreamPlan sp = mlp_stream_plan(M, D, FF);
+  const size_t least = h_bytes(M, FF) + (sp.splits > 1 ? stream_scratch_bytes(sp)
+                                                       : (down_least(M, D, FF, beside_h(M, FF, scratch)) + 255) & ~(size_t)255);
+  return least < need ? least : need;
+}
+
 size_t fsw_mlp_workspace_bytes(int dtype, int64_t M, int64_t D, int64_t FF) {
   (void)dtype;
   return mlp_workspace(M, D, FF, SIZE_MAX);
@@ -744,7 +765,8 @@ static int mlp_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* X, 
   if (dtype != FSW_BF16 && dtype != FSW_FP16) return FSW_E_DTYPE;
   if (M < 0 || D < 0 || FF < 0 || M > MAX_DIM || D > MAX_DIM || FF > MAX_DIM / 2) return FSW_E_SHAPE;
   if (M == 0 || D == 0) return FSW_OK;  // Y is empty: nothing to read or write
-  const size_t need = mlp_workspace(M, D, FF, scratch);
+  size_t need = mlp_workspace(M, D, FF, scratch);
+  if (workspace_bytes < need) need = mlp_least(M, D, FF, scratch, need);
   if (need > 0 && (!workspace || workspace_bytes < need)) return FSW_E_WORKSPACE;
   if (need > 0 && !aligned16(workspace)) return FSW_E_ALIGN;
   // FF == 0 needs no H: any non-NULL pointer satisfies the validators and is never dereferenced

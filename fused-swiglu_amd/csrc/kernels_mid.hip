@@ -336,7 +336,7 @@ hipError_t launch_mid_tile(const MidPlan& p, const GemmArgs& a, int ph, hipStrea
   const int tiles_q = (a.nq + 32 * FQ - 1) / (32 * FQ);
   GemmArgs b = a;
   b.tile_p = p.step;
-  // whole lines are non-temporal when at most two tiles of activation rows share them (see launch_dma_kernel)
+  // whole lines are non-temporal when at most two tiles of activation rows share them
   hipLaunchKernelGGL((mid_kernel<E, GATED, 2, 2, FP, FQ, NS>), dim3((unsigned)(tiles_p * tiles_q), (unsigned)a.splits), dim3(512),
                      0, stream, b, tiles_p, tiles_q, GATED ? 4 : 2, ph, tiles_q <= 2 ? 1 : 0);
   return hipGetLastError();

@@ -93,7 +93,8 @@ FSW_API int fsw_validate_down(int dtype, int64_t M, int64_t D, int64_t FF,
                       const void* Y, int64_t ldy);
 
 /* Bytes of device scratch fsw_down needs for this shape: fp32 split-K partials where few output tiles meet a deep K
- * (FSW_E_WORKSPACE without them), 0 otherwise. 4 * M * D bytes per part, at most 256 MB above 256 rows; the number of parts
+ * (FSW_E_WORKSPACE without them), 0 otherwise. Up to 256 rows less is accepted where K parts are only an option (few rows, a short K):
+ * fsw_down and fsw_mlp then make as many parts as there is room for, which is slower. 4 * M * D bytes per part, at most 256 MB above 256 rows; the number of parts
  * follows the shape's fastest plan and may differ from one version to the next. No counterpart in the reference, which has no down projection. */
 FSW_API size_t fsw_down_workspace_bytes(int dtype, int64_t M, int64_t D, int64_t FF);
 

@@ -406,3 +406,16 @@ def test_static_forward_keeps_its_parts_within_its_array(capi):
         nbytes = L.fsw_down_workspace_bytes(0, M, D, FF)
         assert nbytes > 0 and nbytes % (4 * M * D) == 0 and 2 <= nbytes // (4 * M * D) <= 16
         assert L.fsw_mlp_workspace_bytes(0, M, D, FF) == (M * FF * 2 + 255) // 256 * 256 + (nbytes + 255) // 256 * 256
+
+
+@pytest.mark.parametrize("M,d,ff", [(40, 2048, 4096), (121, 336, 904), (4, 5120, 13824)])
+def test_forward_takes_scratch_for_h_alone_where_k_parts_are_optional(capi, M, d, ff):
+    """The producer / consumer kernel splits K as far as there is room; a workspace of H's own size is enough where the kernels
+    before it needed no more. (The NULL operands are what the call then reports.)"""
+    L = capi.lib()
+    h = (2 * M * ff + 255) // 256 * 256
+    assert L.fsw_mlp_workspace_bytes(0, M, d, ff) > h
+    call = lambda nbytes: L.fsw_mlp(0, M, d, ff, None, d, None, d, None, ff, None, d, 0x1000, nbytes, None)
+    assert call(h) == capi.E_NULL and call(h - 1) == capi.E_WORKSPACE
+    M, d, ff = 200, 512, 4096  # K parts without which this range has no kernel
+    assert call(2 * M * ff) == capi.E_WORKSPACE

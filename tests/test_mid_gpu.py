@@ -99,6 +99,27 @@ def test_down_projection_of_few_rows_runs_without_scratch(capi):
     assert_one_rounding(Y, oracle.ref_down(H.cpu(), W2.cpu(), torch.float64), torch.bfloat16, "no scratch")
 
 
+@pytest.mark.parametrize("M,D,FF", [(121, 336, 904), (90, 488, 1000), (20, 2048, 8192), (16, 5120, 13824)])
+def test_down_projection_with_less_scratch_than_its_parts_want(capi, M, D, FF):
+    """K parts on the producer / consumer kernel are as many as there is room for: none without a workspace, or with one that is not
+    16-byte aligned; fewer in less room. A guard behind the scratch stays as it is."""
+    L = capi.lib()
+    nbytes = L.fsw_down_workspace_bytes(0, M, D, FF)
+    part = 4 * M * D
+    assert nbytes >= 2 * part
+    H = (torch.randn(M, FF, device=DEV) * 0.3).to(torch.bfloat16)
+    W2 = (torch.randn(D, FF, device=DEV) / FF ** 0.5).to(torch.bfloat16)
+    ref = (H.double() @ W2.double().T).cpu()
+    ws = torch.full((nbytes + 512,), 255, dtype=torch.uint8, device=DEV)
+    for offset, size in ((None, 0), (0, part), (8, nbytes), (0, 2 * part), (0, nbytes)):
+        Y = torch.empty(M, D, dtype=torch.bfloat16, device=DEV)
+        assert L.fsw_down(0, M, D, FF, H.data_ptr(), FF, W2.data_ptr(), FF, Y.data_ptr(), D,
+                          None if offset is None else ws.data_ptr() + offset, size,
+                          torch.cuda.current_stream().cuda_stream) == capi.OK
+        assert (ws[size + 16:] == 255).all()
+        assert_one_rounding(Y, ref, torch.bfloat16, "scratch of %d bytes %s" % (size, (M, D, FF)))
+
+
 @pytest.mark.parametrize("M,d,ff", [(1, 4096, 14336), (16, 3000, 8008), (40, 2048, 8192), (130, 4096, 11008), (200, 3000, 8008),
                                     (300, 3960, 8040), (512, 1024, 2816), (700, 1320, 3000)])
 def test_chosen_tiles_against_the_256_row_kernel(capi, M, d, ff):
