@@ -175,3 +175,22 @@ def test_fewer_parts_than_there_is_scratch_for(capi, M, D, FF):
                           torch.cuda.current_stream().cuda_stream) == capi.OK
         assert (ws[nbytes:] == 255).all()
         assert_one_rounding(Y, (H.double() @ W2.double().T).cpu(), torch.bfloat16, "parts %s" % ((M, D, FF),))
+
+
+@pytest.mark.parametrize("M,ff,K", [(1, 4096, 3000), (4, 11008, 4096), (20, 5504, 4096), (33, 3000, 2048)])
+def test_float32_output_of_few_rows_keeps_its_short_sums(capi, M, ff, K):
+    """skinny_kernel splits K between its waves; the result as it stands in float32 shows the length of the chains. Bit for bit what that
+    kernel gives when forced, and within its error of float64: a wave's chain has at most K / (32 * 4) sums of relative error 2^-24
+    each, a random walk of sqrt(n) of them; SiLU and the product add about two more roundings. Twice that."""
+    inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + ff, x_scale=1.0)
+    X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
+    H = capi.gateup_f32out(X, W)
+    try:
+        capi.set_variant(0, 100)
+        few = capi.gateup_f32out(X, W)
+    finally:
+        capi.set_variant(0, -1)
+    assert torch.equal(H, few)
+    pre = X.double() @ W.double().T
+    ref = pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2])
+    assert ((H.double() - ref).norm() / ref.norm()).item() <= 2 * 2.0 ** -24 * ((K / 128) ** 0.5 + 2)
