@@ -167,7 +167,17 @@ bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
   const int64_t bytes = 2 * np * k;
   if (family == 0) {
     const int64_t tiles = (np + 31) / 32;
-    return m > 16 ? tiles > 256 || rag : tiles > 256 && (m > 8 || bytes >= (int64_t)56 << 20);
+    if (m > 16) return tiles > 256 || rag;
+    if (tiles <= 256 || (m <= 8 && bytes < (int64_t)56 << 20)) return false;
+    // Up to 8 rows skinny_kernel is as fast where its workgroups leave less than an eighth of the last round of compute units idle. Us,
+    // 1 / 8 rows, skinny -> mid: 28672 x 4096 (896 workgroups) 37.6 -> 36.9 / 38.0 -> 36.6; 32768 x 4096 (1024) 41.5 -> 41.5 / 40.9 ->
+    // 41.4; 24576 x 4608 (768) 35.9 -> 35.4 / level; 40960 x 5120 (1280) 62.5 -> 63.4 / level; 22016 x 4096 (688) 29.8 -> 29.2 / 29.7 ->
+    // 29.1; 16128 x 2880 (504) 16.3 -> 16.9. With more of them idle: 27648 x 5120 (864) 46.2 -> 43.4 / 48.2 -> 43.6; 20480 x 2560 (640)
+    // 18.9 -> 18.3. Rows a multiple of 2 KB apart are the exception: its eight-wave workgroups walk K in step and meet on the same memory
+    // channels (16384 x 4096 25.9 -> 21.9, 16384 x 2048 13.4 -> 12.4, 16384 x 3072 18.2 -> 17.5).
+    const int64_t rounds = (tiles + 255) / 256;
+    if (m <= 8 && !rag && !decode_stream_wanted(0, m, np, k) && 8 * tiles >= 7 * 256 * rounds) return tiles <= 640 && k % 1024 == 0;
+    return true;
   }
   const int64_t tiles = (np + 15) / 16;
   if (m > 16) return rag || bytes >= (int64_t)8 << 20;

@@ -385,7 +385,12 @@ def test_kernels_that_run_in_the_ranges_of_few_rows(capi):
     weight-streaming kernel for short calls, the 256-row kernel above; a forced tile keeps its own."""
     runs = lambda fam, M, n, k: capi.variant_name(fam, 0, M, n, k)
     assert runs(3, 1, 5632, 1024) == "skinny" and runs(4, 16, 1024, 2816) == "skinny" and runs(4, 16, 4096, 14336) == "skinny"
-    assert runs(3, 1, 28672, 4096).startswith("mid_") and runs(4, 1, 5120, 13824).startswith("mid_")
+    assert runs(3, 1, 27648, 5120).startswith("mid_") and runs(4, 1, 5120, 13824).startswith("mid_")
+    # up to 8 rows: weight streaming where its workgroups fill their last round of compute units to seven eighths ...
+    assert runs(3, 1, 28672, 4096) == "skinny" == runs(3, 8, 40960, 5120) and runs(3, 9, 28672, 4096).startswith("mid_")
+    assert runs(3, 1, 28640, 4096).startswith("mid_") and runs(3, 1, 28672, 4104).startswith("mid_")
+    # ... unless its rows lie a multiple of 2 KB apart and its workgroups have eight waves
+    assert runs(3, 1, 16384, 4096).startswith("mid_") and runs(3, 1, 16384, 4160) == "skinny"
     assert runs(3, 130, 22016, 4096) == "mid_96x160" and runs(3, 40, 38880, 5800) == "mid_160x64"
     assert runs(5, 24, 4096, 11008).startswith("mid_") and runs(4, 200, 4096, 14336) == "mid_128x224"
     assert runs(3, 333, 28672, 4096) == "pair16_256x192" and runs(5, 8192, 4096, 14336) == "pair16_256x256"

@@ -120,7 +120,7 @@ def test_down_projection_with_less_scratch_than_its_parts_want(capi, M, D, FF):
         assert_one_rounding(Y, ref, torch.bfloat16, "scratch of %d bytes %s" % (size, (M, D, FF)))
 
 
-@pytest.mark.parametrize("M,d,ff", [(1, 4096, 14336), (16, 3000, 8008), (40, 2048, 8192), (130, 4096, 11008), (200, 3000, 8008),
+@pytest.mark.parametrize("M,d,ff", [(1, 5120, 13824), (16, 3000, 8008), (40, 2048, 8192), (130, 4096, 11008), (200, 3000, 8008),
                                     (300, 3960, 8040), (512, 1024, 2816), (700, 1320, 3000)])
 def test_chosen_tiles_against_the_256_row_kernel(capi, M, d, ff):
     """What the dispatcher chooses (pieces lower than the tile included) against the 256-row kernel, which takes any problem: every
@@ -194,3 +194,18 @@ def test_float32_output_of_few_rows_keeps_its_short_sums(capi, M, ff, K):
     pre = X.double() @ W.double().T
     ref = pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2])
     assert ((H.double() - ref).norm() / ref.norm()).item() <= 2 * 2.0 ** -24 * ((K / 128) ** 0.5 + 2)
+
+
+@pytest.mark.parametrize("M,ff,K", [(1, 14336, 4096), (4, 14336, 4096), (8, 14336, 4096), (1, 11008, 4096)])
+def test_few_rows_of_full_rounds_keep_the_weight_streaming_kernel(capi, M, ff, K):
+    """Gate/up of up to 8 rows where the producer / consumer kernel is no faster: the bits of the weight-streaming kernel, whose waves
+    sum K in several short chains."""
+    inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + ff, x_scale=1.0)
+    X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
+    H = capi.gateup(X, W)
+    try:
+        capi.set_variant(0, 100)
+        few = capi.gateup(X, W)
+    finally:
+        capi.set_variant(0, -1)
+    assert torch.equal(H, few)
