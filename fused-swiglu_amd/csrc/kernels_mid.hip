@@ -367,8 +367,15 @@ static MidPlan find_plan(bool gated, int np, int nq, int k, bool ragged, int spl
     const int full = 32 * t.fp;
     const long long tp = (np + full - 1) / full;
     int steps[2] = {full, 0};
-    if (gated && tp * tq <= 1024) {  // as many pieces as whole rounds hold
-      const long long rounds = (tp * tq + 255) / 256, pieces = rounds * 256 / tq;
+    const long long rounds = (tp * tq + 255) / 256;
+    // As many pieces as whole rounds hold. Aligned 128-row tiles of up to 64 activation rows stay whole where they leave less than an
+    // eighth of a round empty: the pieces' wasted MFMA and LDS work costs what those compute units give, and K is then walked from the same
+    // start (mid_kernel's `rot`) for all these row counts. us, pieces -> whole: 28672 x 4096 (224 tiles) 16 rows 37.1 -> 36.5, 48 rows 38.4
+    // -> 37.9; 28928 x 5568 (226) 11 rows 53.3 -> 51.2; 29056 x 5760 (227) 40 rows 53.7 -> 55.0. With fewer tiles, 27648 x 5120 (216), 16
+    // rows 45.2 whole, 43.9 in pieces, 48 rows 51.4 and 49.7.
+    const bool whole = !ragged && t.fp == 4 && t.fq <= 2 && 8 * tp * tq >= 7 * 256 * rounds;
+    if (gated && tp * tq <= 1024 && !whole) {
+      const long long pieces = rounds * 256 / tq;
       const int step = (int)(((np + pieces - 1) / pieces + 7) / 8 * 8);
       if (step < full && step > full - 32) steps[1] = step;
     }

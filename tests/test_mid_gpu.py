@@ -209,3 +209,19 @@ def test_few_rows_of_full_rounds_keep_the_weight_streaming_kernel(capi, M, ff, K
     finally:
         capi.set_variant(0, -1)
     assert torch.equal(H, few)
+
+
+@pytest.mark.parametrize("M", [12, 16, 24, 32, 48, 64])
+@pytest.mark.parametrize("ff,K", [(14336, 4096), (14464, 1024)])
+def test_whole_tiles_where_they_fill_a_round(capi, M, ff, K):
+    """224 and 226 tiles of 128 weight rows: no pieces, so each feature's sum starts at the K tile it starts at on the forced 128 x 64
+    tile (id 4), bit for bit."""
+    inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + ff, x_scale=1.0)
+    X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
+    H = capi.gateup(X, W)
+    try:
+        capi.set_variant(0, 4)
+        whole = capi.gateup(X, W)
+    finally:
+        capi.set_variant(0, -1)
+    assert torch.equal(H, whole)
