@@ -94,18 +94,21 @@ int64_t decode_rows(int family, int64_t np, int64_t k) {
   return d_ff < ((int64_t)1 << 25) ? 48 : d_ff < ((int64_t)1 << 27) ? 32 : 16;
 }
 
+// whether these rows are in the decode range
+bool few_rows(int family, int64_t m, int64_t np, int64_t k) {
+  if (m > decode_rows(family, np, k)) return false;
+  // from a dozen rows on a gate/up matrix of 200 .. 256 pieces of 128 rows is past that range
+  const int64_t tiles = (np + 127) / 128;
+  return !(family == 0 && m >= 12 && k > 0 && tiles >= 200 && tiles <= 256);
+}
+
 int resolve_variant(int family, int64_t m, int64_t np, int64_t k) {
   const int forced = g_forced_variant[family];
   if (forced == VARIANT_DECODE_FUSED || forced == VARIANT_DECODE_FUSED_FAIL || forced == VARIANT_DECODE_STREAM ||
       forced == VARIANT_STREAM_SPLIT)
     return m <= 64 ? VARIANT_SKINNY : pick_tiled(family, m, np, k);
   if (forced >= 0 && !(forced == VARIANT_SKINNY && m > 64)) return forced;
-  if (m <= decode_rows(family, np, k)) {  // decode and small batches: weight streaming, HBM bound
-    // from a dozen rows on a gate/up matrix of 200 .. 256 pieces of 128 rows is past that range
-    const int64_t tiles = (np + 127) / 128;
-    if (family == 0 && m >= 12 && k > 0 && tiles >= 200 && tiles <= 256) return V_128x64;
-    return VARIANT_SKINNY;
-  }
+  if (few_rows(family, m, np, k)) return VARIANT_SKINNY;  // decode and small batches: weight streaming, HBM bound
   return pick_tiled(family, m, np, k);
 }
 
@@ -321,7 +324,9 @@ int fsw_validate_down(int dtype, int64_t M, int64_t D, int64_t FF, const void* H
 static hipError_t launch_gateup_mid(int v, int dtype, const fsw::GemmArgs& a, hipStream_t stream) {
   const fsw::MidPlan p = g_forced_variant[0] >= 0 ? forced_mid_plan(v)
                                                   : fsw::mid_plan(true, a.np, a.nq, a.k, fsw::mid_ragged(a), 1, 1);
-  return fsw::launch_mid(dtype, true, p, a, stream);
+  fsw::GemmArgs b = a;
+  b.short_sums = few_rows(0, a.nq, a.np, a.k) ? 1 : 0;
+  return fsw::launch_mid(dtype, true, p, b, stream);
 }
 
 // zero_words / n_zero_words: see GemmArgs (only the decode-regime kernels honour them; the caller checks that)
@@ -533,6 +538,7 @@ static int down_impl(int dtype, int64_t M, int64_t D, int64_t FF, const void* H,
                                ? forced_mid_plan(v)
                                : fsw::mid_plan(false, (int)D, (int)M, (int)FF, fsw::mid_ragged(a), M > 256 ? 0 : a.splits, a.splits);
     a.splits = p.splits;
+    a.short_sums = few_rows(1, M, D, FF) ? 1 : 0;
     return finish(fsw::launch_mid(dtype, false, p, a, (hipStream_t)stream));
   }
   if (v == VARIANT_SKINNY) {

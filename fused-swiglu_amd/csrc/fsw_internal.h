@@ -24,6 +24,10 @@ struct GemmArgs {
   // (gated kernel), bit 2 = P. A blocked [rows, k] matrix is ceil(rows / 256) panels of ceil(k / 32) blocks of
   // [256 rows][64 bytes], zero padded (blocked_bytes()).
   int layout = 0;
+  // mid_kernel on tiles of up to 64 activation rows: K is summed in chains of 256 elements, whose sums are added. Set for the rows that
+  // the weight-streaming kernels take otherwise, whose waves sum an eighth or a quarter of K each. (Here, between a 4- and an 8-byte field, it costs no space: with 8 bytes
+  // more mid_kernel's arguments reach a third cache line, 0.2 us a launch.)
+  int short_sums = 0;
   // words the FIRST workgroup of a gate/up launch sets to zero before anything else (mid_kernel and
   // skinny_kernel honour it): the ticket counters of the split-K streaming down projection that follows in fsw_mlp
   unsigned* zero_words = nullptr;

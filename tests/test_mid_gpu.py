@@ -225,3 +225,23 @@ def test_whole_tiles_where_they_fill_a_round(capi, M, ff, K):
     finally:
         capi.set_variant(0, -1)
     assert torch.equal(H, whole)
+
+
+@pytest.mark.parametrize("M,ff,K", [(1, 13824, 5120), (4, 5504, 4096), (16, 8192, 3000), (20, 4096, 2048), (40, 3904, 1320)])
+def test_few_rows_are_summed_as_finely_as_by_the_weight_streaming_kernel(capi, M, ff, K):
+    """The unrounded gate/up product of few rows, on tiles of 32 and 64 activation rows: no further from float64 than the
+    weight-streaming kernel, which sums an eighth or a quarter of K in a chain. Both errors are root mean squares over thousands of sums;
+    a tenth covers their spread."""
+    inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + ff, x_scale=1.0)
+    X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
+    pre = X.double() @ W.double().T
+    ref = pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2])
+    error = {}
+    for v in (100, 202, 204, 210):  # weight streaming; 64 x 32, 128 x 32, 128 x 64
+        try:
+            capi.set_variant(0, v)
+            H = capi.gateup_f32out(X, W)
+        finally:
+            capi.set_variant(0, -1)
+        error[v] = ((H.double() - ref).norm() / ref.norm()).item()
+    assert max(error[v] for v in (202, 204, 210)) <= 1.1 * error[100], error
