@@ -172,14 +172,16 @@ bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
     const int64_t tiles = (np + 31) / 32;
     if (m > 16) return tiles > 256 || rag;
     if (tiles <= 256 || (m <= 8 && bytes < (int64_t)56 << 20)) return false;
-    // Up to 8 rows skinny_kernel is as fast where its workgroups leave less than an eighth of the last round of compute units idle. Us,
-    // 1 / 8 rows, skinny -> mid: 28672 x 4096 (896 workgroups) 37.6 -> 36.9 / 38.0 -> 36.6; 32768 x 4096 (1024) 41.5 -> 41.5 / 40.9 ->
-    // 41.4; 24576 x 4608 (768) 35.9 -> 35.4 / level; 40960 x 5120 (1280) 62.5 -> 63.4 / level; 22016 x 4096 (688) 29.8 -> 29.2 / 29.7 ->
-    // 29.1; 16128 x 2880 (504) 16.3 -> 16.9. With more of them idle: 27648 x 5120 (864) 46.2 -> 43.4 / 48.2 -> 43.6; 20480 x 2560 (640)
-    // 18.9 -> 18.3. Rows a multiple of 2 KB apart are the exception: its eight-wave workgroups walk K in step and meet on the same memory
-    // channels (16384 x 4096 25.9 -> 21.9, 16384 x 2048 13.4 -> 12.4, 16384 x 3072 18.2 -> 17.5).
-    const int64_t rounds = (tiles + 255) / 256;
-    if (m <= 8 && !rag && !decode_stream_wanted(0, m, np, k) && 8 * tiles >= 7 * 256 * rounds) return tiles <= 640 && k % 1024 == 0;
+    // Up to 8 rows skinny_kernel is as fast where its workgroups leave less than an eighth of their rounds of compute units empty (less than a
+    // sixteenth above four rounds). us, 1 / 8 rows, skinny -> mid: 28672 x 4096 (896 workgroups) 37.6 -> 36.9 / 38.0 -> 36.6; 32768 x 4096
+    // (1024) 41.5 -> 41.5 / 40.9 -> 41.4; 24576 x 4608 (768) 35.9 -> 35.4 / level; 40960 x 5120 (1280) 62.5 -> 63.4 / level; 22016 x 4096
+    // (688) 29.8 -> 29.2 / 29.7 -> 29.1; 16128 x 2880 (504) 16.3 -> 16.9; 39424 x 5568 (1232) 65.1 -> 65.6. With more of them empty:
+    // 27648 x 5120 (864) 46.2 -> 43.4 / 48.2 -> 43.6; 20480 x 2560 (640) 18.9 -> 18.3; 37760 x 6336 (1180) 73.9 -> 71.3. Rows a multiple
+    // of 2 KB apart are the exception: its eight-wave workgroups walk K in step and meet on the same memory channels (16384 x 4096 25.9 ->
+    // 21.9, 16384 x 2048 13.4 -> 12.4, 16384 x 3072 18.2 -> 17.5).
+    const int64_t rounds = (tiles + 255) / 256, empty = 256 * rounds - tiles;
+    if (m <= 8 && !rag && !decode_stream_wanted(0, m, np, k) && empty <= (rounds <= 4 ? 32 : 16) * rounds)
+      return tiles <= 640 && k % 1024 == 0;
     return true;
   }
   const int64_t tiles = (np + 15) / 16;

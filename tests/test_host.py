@@ -389,6 +389,7 @@ def test_kernels_that_run_in_the_ranges_of_few_rows(capi):
     # up to 8 rows: weight streaming where its workgroups fill their last round of compute units to seven eighths ...
     assert runs(3, 1, 28672, 4096) == "skinny" == runs(3, 8, 40960, 5120) and runs(3, 9, 28672, 4096).startswith("mid_")
     assert runs(3, 1, 28640, 4096).startswith("mid_") and runs(3, 1, 28672, 4104).startswith("mid_")
+    assert runs(3, 1, 37760, 6336).startswith("mid_") and runs(3, 1, 39424, 5568) == "skinny"  # fifteen sixteenths above four rounds
     # ... unless its rows lie a multiple of 2 KB apart and its workgroups have eight waves
     assert runs(3, 1, 16384, 4096).startswith("mid_") and runs(3, 1, 16384, 4160) == "skinny"
     assert runs(3, 130, 22016, 4096) == "mid_96x160" and runs(3, 40, 38880, 5800) == "mid_160x64"
