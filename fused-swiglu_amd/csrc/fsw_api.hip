@@ -159,7 +159,8 @@ bool ragged(int64_t k) { return k % 64 != 0; }
 // kernel whose estimated time is less (47 problems of 130 .. 700 rows: it chose the slower one four times, by 7 % at most; 38880 x
 // 5800 130 rows 150.4 -> 119.0, 256 rows 189.6 -> 138.1; 43680 x 7592 279 rows 348 -> 241; 24160 x 3448 409 rows stays, 93.6 and 105).
 bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
-  if (g_forced_variant[family] >= 0) return dma_variant(g_forced_variant[family]);
+  // what resolve_variant() makes of the forced id: a weight-streaming id takes up to 64 rows, more run the range's own kernel
+  if (g_forced_variant[family] >= 0) return dma_variant(v);
   if (k <= 0) return false;
   if (family == 0 && rag && (v == V_256x256 || narrow_variant(v)) && m <= 1024) {
     const int rows = narrow_variant(v) ? 32 * (v - VARIANT_NARROW) : 256;

@@ -401,8 +401,14 @@ def test_kernels_that_run_in_the_ranges_of_few_rows(capi):
     try:
         assert L.fsw_set_variant(0, 200) == capi.OK and runs(3, 100, 5632, 1024) == "mid_32x32" == runs(0, 100, 5632, 1024)
         assert L.fsw_set_variant(0, 236) == capi.E_VARIANT and L.fsw_set_variant(0, 199) == capi.E_VARIANT
+        for forced in (100, 102):  # weight streaming takes up to 64 rows: above, both products run their range's kernel
+            assert L.fsw_set_variant(0, forced) == capi.OK and L.fsw_set_variant(1, forced) == capi.OK
+            assert runs(3, 100, 28672, 4096) == "mid_128x128" == runs(4, 100, 4096, 14336)
+            assert runs(3, 64, 28672, 4096) == ("skinny" if forced == 100 else runs(0, 64, 28672, 4096))
+            assert runs(3, 8192, 28672, 4096) == "pair16_256x256"
     finally:
         L.fsw_set_variant(0, -1)
+        L.fsw_set_variant(1, -1)
 
 
 def test_static_forward_keeps_its_parts_within_its_array(capi):
