@@ -78,6 +78,12 @@ def traffic_from_profile(workload):
     return (int(m.group(1)), rel) if m else (None, None)
 
 
+def kernel_names(capi, M, d, ff):
+    """The kernels that a forward of this size runs: gate/up, and the down projection inside fsw_mlp. (Families 0 .. 2 of
+    fsw_variant_name name the range that a size falls in, which another kernel may serve.)"""
+    return capi.variant_name(3, 0, M, 2 * ff, d), capi.variant_name(5, 0, M, d, ff)
+
+
 def run_steps(capi, torch, g, cfg, steps, warmup, fused_entry=False, prepacked=False, weight_sets=None, settle_ms=0.0):
     """Times exactly `steps` forwards between two device synchronisations.
     fused_entry=False: a step is the launch sequence fsw_mlp enqueues for this shape, issued through the
@@ -230,7 +236,7 @@ def configs_leg(capi, torch, fsw_weights):
         rec = {"M": M, "d": d, "ff": ff, "dtype": "bf16" if dtype == torch.bfloat16 else "fp16", "calls": n,
                "ms_median": round(med, 5), "ms_p20": round(p20, 5), "ms_p80": round(p80, 5),
                "tflops": round(flops / med / 1e9, 2), "gbs": round(nbytes / med / 1e6, 2),
-               "kernels": "%s + %s" % (capi.variant_name(0, 0, M, 2 * ff, d), capi.variant_name(2, 0, M, d, ff))}
+               "kernels": "%s + %s" % kernel_names(capi, M, d, ff)}
         net = max(med - overhead, 1e-6)
         rec["ms_net"] = round(net, 5)
         if name == "C4":
@@ -415,14 +421,14 @@ def main():
     traffic, traffic_src = traffic_from_profile(args.workload)
     if hbm_bound:
         all_bytes = fsw_weights.hbm_bytes(M, d, ff)
-        roofline = {"bound": "hbm", "kernel": "%s gate/up + %s down (whole forward, two launches)" % (
-                        capi.variant_name(0, 0, M, 2 * ff, d), capi.variant_name(2, 0, M, d, ff)),
+        roofline = {"bound": "hbm",
+                    "kernel": "%s gate/up + %s down (whole forward, two launches)" % kernel_names(capi, M, d, ff),
                     "achieved": round(all_bytes / (gu_ms * 1e-3) / 1e9, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(all_bytes / (gu_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                     "traffic": traffic, "traffic_source": traffic_src, "algorithmic_bytes": all_bytes,
                     "avg_kernel_ms": round(gu_ms, 5)}
     else:
-        kname = capi.variant_name(0, 0, M, 2 * ff, d) + (" (v_mfma_f32_16x16x32), X row-major, H panel-blocked" if blocked else "")
+        kname = kernel_names(capi, M, d, ff)[0] + (" (v_mfma_f32_16x16x32), X row-major, H panel-blocked" if blocked else "")
         roofline = {"bound": "mfma", "kernel": kname + " (gate/up)",
                     "achieved": round(gu_tflops, 2), "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                     "frac": round(gu_tflops / MFMA_PEAK_TFLOPS, 4),
@@ -470,8 +476,7 @@ def main():
         ms4, msc = wall4 / 200 * 1e3, wallc / 201 * 1e3
         k4_ms, kc_ms = sum(k4) / len(k4), sum(kc) / len(kc)
         traffic4, traffic4_src = traffic_from_profile("C4")
-        kern4 = "%s gate/up + %s down" % (capi.variant_name(0, 0, c4["M"], 2 * c4["ff"], c4["d"]),
-                                          capi.variant_name(2, 0, c4["M"], c4["d"], c4["ff"]))
+        kern4 = "%s gate/up + %s down" % kernel_names(capi, c4["M"], c4["d"], c4["ff"])
         out["decode"] = {
             "workload": "C4: M=16 d=4096 ff=14336 bf16", "entry": "fsw_mlp (one call, two launches)",
             "warmup_steps": DECODE_WARMUP, "steps": 200,

@@ -411,6 +411,17 @@ def test_kernels_that_run_in_the_ranges_of_few_rows(capi):
         L.fsw_set_variant(1, -1)
 
 
+def test_benchmark_names_the_kernels_that_run(capi):
+    """The record's kernel names are those of the kernels, not of the ranges that fsw_set_variant forces."""
+    import bench
+    assert bench.kernel_names(capi, 16, 4096, 14336) == ("mid_128x32", "skinny")
+    assert bench.kernel_names(capi, 32, 4096, 14336)[1].startswith("mid_")
+    assert bench.kernel_names(capi, 8192, 4096, 14336) == ("pair16_256x256", "pair16_256x256")
+    for (M, d, ff) in [(1, 1024, 2816), (17, 4096, 14336), (200, 3000, 8008), (512, 4096, 11008)]:
+        names = bench.kernel_names(capi, M, d, ff)
+        assert not [n for n in names if "dma" in n or n == "stream_split"], names
+
+
 def test_static_forward_keeps_its_parts_within_its_array(capi):
     """Few-row down projections split K as far as scratch allows; the workspace query and the plan agree on it."""
     L = capi.lib()
