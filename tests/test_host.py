@@ -191,6 +191,8 @@ def test_variant_choice_by_regime(capi):
 
 @pytest.mark.parametrize("M,want", [(33, "splitk_dma_128x64"), (64, "splitk_dma_128x64"), (65, "splitk_dma_128x128")])
 def test_split_plan_names_the_tile_that_runs(capi, M, want):
+    """The range's name, and a tile of the producer / consumer kernel as the kernel that runs there."""
+    assert capi.variant_name(4, 0, M, 4096, 14336).startswith("mid_") and capi.variant_name(5, 0, M, 4096, 14336).startswith("mid_")
     assert capi.variant_name(1, 0, M, 4096, 14336) == capi.variant_name(2, 0, M, 4096, 14336) == want
 
 
@@ -440,5 +442,5 @@ def test_forward_takes_scratch_for_h_alone_where_k_parts_are_optional(capi, M, d
     assert L.fsw_mlp_workspace_bytes(0, M, d, ff) > h
     call = lambda nbytes: L.fsw_mlp(0, M, d, ff, None, d, None, d, None, ff, None, d, 0x1000, nbytes, None)
     assert call(h) == capi.E_NULL and call(h - 1) == capi.E_WORKSPACE
-    M, d, ff = 200, 512, 4096  # K parts without which this range has no kernel
+    M, d, ff = 200, 512, 4096  # a range that refused less than its K parts when it had no kernel without them, and still does
     assert call(2 * M * ff) == capi.E_WORKSPACE

@@ -346,8 +346,8 @@ def test_single_launch_decode_reports_a_failed_barrier(capi):
 @pytest.mark.parametrize("M", [1, 9, 16, 17, 32])
 def test_split_k_streaming_down_inside_mlp(capi, M, dtype):
     """Inside fsw_mlp the down projection of up to 32 rows runs 32-row tiles with K split over two workgroups whose
-    partial tiles meet through ticket counters (zeroed by the gate/up kernel before it). Forced (variant 104) on small
-    and ragged shapes, automatic at decode size: against the oracle given the GPU's H, against the 16-row kernel, bit
+    partial tiles meet through ticket counters (zeroed by the gate/up kernel before it). Forced (variant 104, nothing selects it by
+    itself) on small and ragged shapes and at decode size: against the oracle given the GPU's H, against the 16-row kernel, bit
     for bit call after call (the summation order does not depend on which workgroup arrives last), and with a
     workspace full of garbage (nothing but the gate/up kernel initialises the counters)."""
     shapes = [(8, 8), (136, 40), (1000, 264), (520, 1032), (256, 2056), (40, 20000), (4096, 1032)]
@@ -375,36 +375,31 @@ def test_split_k_streaming_down_inside_mlp(capi, M, dtype):
         finally:
             capi.set_variant(1, -1)
         assert (Y.float() - Y16.float()).abs().max().item() <= 2e-2
-    # automatic at decode size, and only there
+    # the range of that name, which another kernel serves unless it is forced
     name = lambda m, d_, ff_: capi.variant_name(2, 0, m, d_, ff_)
+    runs = lambda m, d_, ff_: capi.variant_name(5, 0, m, d_, ff_)
+    assert runs(17, 4096, 14336).startswith("mid_") and runs(32, 4096, 14336).startswith("mid_")
     assert name(17, 4096, 14336) == "stream_split" and name(32, 4096, 14336) == "stream_split"
     assert name(16, 4096, 14336) == "skinny" and name(24, 512, 1024) == "skinny" and name(33, 4096, 14336) != "stream_split"
     assert name(16, 8192, 28672) == "decode_stream"
-    # decode size with a ragged last tile (d % 32 != 0: 129 tiles, the last one 8 rows wide) and a K that the two
-    # workgroups of a tile and their waves do not split evenly
-    if M in (17, 32):
-        d, ff = 4104, 14344
-        assert name(M, d, ff) == "stream_split"
-        inp = fsw_weights.make_inputs(M, d, ff, dtype, seed=8, x_scale=0.5)
+    # decode size, with a ragged last tile (d % 32 != 0: 129 tiles, the last one 8 rows wide) and a K that the two
+    # workgroups of a tile and their waves do not split evenly, and without
+    for (d, ff, fill, repeats) in [(4104, 14344, 0xA5, 5), (4096, 14336, 0x5A, 20)] if M in (17, 32) else []:
+        inp = fsw_weights.make_inputs(M, d, ff, dtype, seed=8 if d == 4104 else 7, x_scale=0.5)
         g = to_dev(inp)
-        ws = capi.mlp_workspace(g["X"], ff)
-        ws.fill_(0xA5)
-        Y = capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws)
-        H = ws[: M * ff * 2].view(dtype).view(M, ff).clone()
-        assert_one_rounding(Y, oracle.ref_down(H.cpu(), inp["W2"], torch.float64), dtype, "stream-split ragged decode size")
-        for _ in range(5):
-            assert torch.equal(capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws), Y)
-    if M in (17, 32):
-        d, ff = 4096, 14336
-        inp = fsw_weights.make_inputs(M, d, ff, dtype, seed=7, x_scale=0.5)
-        g = to_dev(inp)
-        ws = capi.mlp_workspace(g["X"], ff)
-        ws.fill_(0x5A)
-        Y = capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws)
-        H = ws[: M * ff * 2].view(dtype).view(M, ff).clone()
+        try:
+            capi.set_variant(1, 104)
+            assert runs(M, d, ff) == "stream_split"
+            ws = capi.mlp_workspace(g["X"], ff)
+            ws.fill_(fill)
+            Y = capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws)
+            H = ws[: M * ff * 2].view(dtype).view(M, ff).clone()
+            reps = [capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws) for _ in range(repeats)]
+        finally:
+            capi.set_variant(1, -1)
         assert_one_rounding(Y, oracle.ref_down(H.cpu(), inp["W2"], torch.float64), dtype, "stream-split decode size")
-        for _ in range(20):
-            assert torch.equal(capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws), Y)
+        for r in reps:
+            assert torch.equal(r, Y)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -577,8 +572,8 @@ def test_swiglu_fwd_bf16_writes_dense_half_width_rows(ext):
 
 @pytest.mark.parametrize("shape", [(16, 520, 8200), (64, 136, 11008), (128, 264, 13824), (100, 72, 8192), (40, 64, 10004)])
 def test_weight_stream_cut_into_one_piece_per_compute_unit(capi, shape):
-    """Gate/up with one tile of activation rows and between 128 and 216 tiles of 128 weight rows: the dispatcher hands
-    every workgroup a piece of 64 .. 120 rows instead (as many pieces as compute units), whose tile reads its missing
+    """Gate/up with one tile of activation rows: the dispatcher hands every workgroup a piece lower than its tile (72, 88, 112 and
+    80 weight rows here, as many pieces as compute units; whole tiles of 64 rows at 8192 features), which reads its missing
     rows as zeros and stores only the features it owns. Against the oracle (every feature, so a piece that stored a
     neighbour's features from its zero rows would show as zeros there) and against the kernel on whole 128-row tiles; H
     inside a wider NaN buffer, so a store past the row's end would show."""
@@ -586,16 +581,10 @@ def test_weight_stream_cut_into_one_piece_per_compute_unit(capi, shape):
     dtype = torch.bfloat16 if ff % 16 == 0 else torch.float16
     inp = fsw_weights.make_inputs(M, d, ff, dtype, seed=M + ff, x_scale=0.5)
     g = to_dev(inp)
-    want = "dma_128x64" if M <= 64 else "dma_128x128"
-    forced = capi.variant_name(0, 0, M, 2 * ff, d) != want  # small K: the weight-streaming kernel would run
     wide = torch.full((M, ff + 8), float("nan"), dtype=dtype, device=DEV)
-    try:
-        if forced:
-            capi.set_variant(0, 4)
-        assert capi.variant_name(0, 0, M, 2 * ff, d) == want
-        H = capi.gateup(g["X"], g["W13"], out=wide[:, :ff])
-    finally:
-        capi.set_variant(0, -1)
+    assert capi.variant_name(3, 0, M, 2 * ff, d) == {8200: "mid_96x32", 11008: "mid_96x64", 13824: "mid_128x128",
+                                                     8192: "mid_64x128", 10004: "mid_96x64"}[ff]
+    H = capi.gateup(g["X"], g["W13"], out=wide[:, :ff])
     assert_one_rounding(H, oracle.ref_gateup(inp["X"], inp["W13"], torch.float64), dtype, "pieces %s" % (shape,))
     assert torch.isnan(wide[:, ff:]).all()
     # the same kernel on whole tiles: a problem of the same rows that the rule leaves alone (more than 128 activation
@@ -613,25 +602,31 @@ def test_weight_stream_cut_into_one_piece_per_compute_unit(capi, shape):
 
 def test_pieces_zero_the_ticket_counters_of_the_down_projection_too(capi):
     """A decode-sized forward whose gate/up stream is cut into pieces (27648 rows: 247 pieces of 112) AND whose down
-    projection is the split-K streaming kernel (24 rows): the first workgroup of the gate/up launch still zeroes the
-    ticket counters, whatever rows it owns. Workspace full of garbage, repeated calls bit for bit."""
+    projection is the split-K streaming kernel (24 rows, variant 104): the first workgroup of the gate/up launch zeroes
+    the ticket counters, whatever rows it owns. Workspace full of garbage, repeated calls bit for bit."""
     M, d, ff = 24, 5120, 13824
     assert capi.variant_name(0, 0, M, 2 * ff, d) == "dma_128x64" and capi.variant_name(2, 0, M, d, ff) == "stream_split"
     inp = fsw_weights.make_inputs(M, d, ff, torch.bfloat16, seed=61, x_scale=0.5)
     g = to_dev(inp)
-    ws = capi.mlp_workspace(g["X"], ff)
-    ws.fill_(0xC3)
-    Y = capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws)
+    try:
+        capi.set_variant(1, 104)
+        assert capi.variant_name(3, 0, M, 2 * ff, d) == "mid_128x32" and capi.variant_name(5, 0, M, d, ff) == "stream_split"
+        ws = capi.mlp_workspace(g["X"], ff)
+        ws.fill_(0xC3)
+        Y = capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws)
+        reps = [capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws) for _ in range(5)]
+    finally:
+        capi.set_variant(1, -1)
     oracle.assert_parity(Y, oracle.ref_mlp(inp["X"], inp["W13"], inp["W2"], torch.float64), "pieces + stream_split")
-    for _ in range(5):
-        assert torch.equal(capi.mlp(g["X"], g["W13"], g["W2"], workspace=ws), Y)
+    for r in reps:
+        assert torch.equal(r, Y)
 
 
 @pytest.mark.parametrize("M", [40, 200, 300])
 @pytest.mark.parametrize("K", [8, 64, 72, 128, 192, 200, 256, 320, 328])
 def test_stage_ring_with_few_k_tiles(capi, M, K):
-    """The three- and four-stage rings of the 128-row tiles (launches of at most 256 workgroups: one, two and three tiles
-    of activation rows) with fewer K tiles than stages, as many, one more, and a K tail: copies issued past the last
+    """The rings of five lines of the 128 x 64 and 128 x 128 tiles (one, two and three tiles of activation rows) and those of the
+    down projection's own choice with fewer K tiles than lines, as many, one more, and a K tail: copies issued past the last
     tile bring nothing in."""
     inp = fsw_weights.make_inputs(M, K, 8 * K, torch.bfloat16, seed=41 * K + M)
     g = to_dev(inp)
@@ -651,17 +646,23 @@ def test_stage_ring_with_few_k_tiles(capi, M, K):
                                          (511, 2048, 7172, "dma8w_128x256"), (576, 2048, 5120, "dma_128x192"),
                                          (1179, 2048, 2048, "dma_128x192"), (2030, 2056, 2044, "dma8w_128x256")])
 def test_gateup_tiles_that_fill_one_round(capi, M, K, ff, name):
-    """129 rows and more on the tile whose launch has at most 256 workgroups: both sides of its rows, two, three and more tiles
-    of activation rows on the wide kernels, ragged features, K tails; output inside a wider NaN buffer."""
-    assert capi.variant_name(0, 0, M, 2 * ff, K) == name
+    """129 rows and more in the ranges whose launches have at most 256 workgroups of the 128-row tile of that name: both sides of
+    their rows, ragged features, K tails, on the tile that runs there and on the named one; output inside a wider NaN buffer."""
+    assert capi.variant_name(0, 0, M, 2 * ff, K) == name and capi.variant_name(3, 0, M, 2 * ff, K).startswith("mid_")
     inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + ff, x_scale=0.5)
     X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
     wide = torch.full((M, ff + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
-    capi.gateup(X, W, out=wide[:, :ff])
-    assert torch.isnan(wide[:, ff:]).all()
     pre = X.double() @ W.double().T
     ref = (pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2])).cpu()
-    assert_one_rounding(wide[:, :ff], ref, torch.bfloat16, "H %s" % ((M, K, ff),))
+    for forced in (-1, {"dma_128x128": 0, "dma_128x192": 2, "dma8w_128x256": 3}[name]):
+        wide.fill_(float("nan"))
+        try:
+            capi.set_variant(0, forced)
+            capi.gateup(X, W, out=wide[:, :ff])
+        finally:
+            capi.set_variant(0, -1)
+        assert torch.isnan(wide[:, ff:]).all()
+        assert_one_rounding(wide[:, :ff], ref, torch.bfloat16, "H %s id %d" % ((M, K, ff), forced))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -709,9 +710,12 @@ def test_narrow_tiles_give_the_bits_of_256_row_tiles(capi, rows, dtype, K):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,D,FF", [(49, 512, 4096), (63, 1000, 2056), (64, 512, 4104), (64, 136, 1032), (33, 4096, 8200)])
 def test_split_k_of_at_most_64_rows(capi, M, D, FF, dtype):
-    """The split-K down projection on 128 x 64 tiles (four stages): full and ragged rows and features, K with and without
-    a tail, parts of a few K tiles. Output inside a wider NaN buffer."""
+    """The split-K down projection of up to 64 rows (tiles of 32 x 32 and 64 x 64 of the producer / consumer kernel, four and
+    eight parts): full and ragged rows and features, K with and without a tail, parts of a few K tiles. Output inside a wider NaN
+    buffer."""
     assert capi.variant_name(1, 0, M, D, FF) == "splitk_dma_128x64"
+    assert capi.variant_name(4, 0, M, D, FF) == ("mid_64x64" if D == 4096 else "mid_32x32")
+    assert capi.lib().fsw_down_workspace_bytes(0, M, D, FF) == (8 if D == 512 else 4) * 4 * M * D
     gen = torch.Generator().manual_seed(M + FF)
     H = (torch.randn(M, FF, generator=gen) * 0.5).to(dtype)
     W2 = (torch.randn(D, FF, generator=gen) / FF ** 0.5).to(dtype)
@@ -776,6 +780,8 @@ def test_strided_inputs_of_the_tiled_kernels(capi, variant, M, K, pad):
 def test_strided_inputs_of_the_split_down_projection(capi, M, D, FF, name):
     """The same for the parts of a split K: a part ends inside a row, the last one at its NaN."""
     assert capi.variant_name(1, 0, M, D, FF) == name
+    assert capi.variant_name(4, 0, M, D, FF) == (name if M > 64 else "mid_32x32")
+    assert capi.lib().fsw_down_workspace_bytes(0, M, D, FF) >= 2 * 4 * M * D
     gen = torch.Generator().manual_seed(M + FF)
     H = (torch.randn(M, FF, generator=gen) * 0.5).to(torch.bfloat16)
     W2 = (torch.randn(D, FF, generator=gen) / FF ** 0.5).to(torch.bfloat16)
@@ -783,7 +789,7 @@ def test_strided_inputs_of_the_split_down_projection(capi, M, D, FF, name):
     assert_one_rounding(Y, (H.to(DEV).double() @ W2.to(DEV).double().T).cpu(), torch.bfloat16, name)
 
 
-NARROW_SPLITS = [(435, 4096, 8192, 160), (300, 4096, 8200, 160), (768, 4096, 6144, 192), (516, 4096, 8200, 192),
+NARROW_SPLITS = [(435, 4096, 8192, 160), (470, 4096, 8200, 160), (768, 4096, 6144, 192), (516, 4096, 8200, 192),
                  (887, 4096, 6144, 224), (672, 4096, 8200, 224)]
 
 
@@ -792,7 +798,7 @@ NARROW_SPLITS = [(435, 4096, 8192, 160), (300, 4096, 8200, 160), (768, 4096, 614
 def test_split_k_on_narrow_tiles(capi, M, D, FF, rows, dtype):
     """The split-K down projection on tiles of 160, 192 and 224 activation rows, K a multiple of 64 and not, last tile full
     and not: against the oracle on a one-rounding bound, output inside a wider NaN buffer."""
-    assert capi.variant_name(1, 0, M, D, FF) == "splitk_pair16_256x%d" % rows
+    assert capi.variant_name(1, 0, M, D, FF) == capi.variant_name(4, 0, M, D, FF) == "splitk_pair16_256x%d" % rows
     gen = torch.Generator().manual_seed(M + FF)
     H = (torch.randn(M, FF, generator=gen) * 0.5).to(dtype)
     W2 = (torch.randn(D, FF, generator=gen) / FF ** 0.5).to(dtype)

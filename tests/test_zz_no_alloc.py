@@ -25,9 +25,7 @@ def test_static_scratch_forward_matches_fsw_mlp_call_after_call(capi):
     L = capi.lib()
     limit = L.fsw_mlp_static_max_bytes()
     assert limit == 64 << 20
-    # (M, d, ff): split-K partials + H; small; a decode shape; the split-K streaming down projection of 17 .. 32 rows
-    # (its ticket counters sit in the array behind another call's leftovers and are zeroed by the gate/up kernel);
-    # ragged everything; tiny; H panel-blocked (both projections on 256 x 256 tiles); ragged mid size
+    # (M, d, ff): split-K partials + H; small; a decode shape; one of 17 .. 32 rows; ragged everything; tiny; H panel-blocked (both projections on 256 x 256 tiles); ragged mid size
     shapes = [(200, 1024, 4096), (48, 512, 1032), (16, 4096, 14336), (24, 4096, 14336), (300, 264, 1032), (4, 136, 40),
               (2304, 4096, 2048), (700, 1024, 2056)]
     assert capi.variant_name(2, 0, 24, 4096, 14336) == "stream_split"
@@ -60,6 +58,19 @@ def test_static_scratch_forward_matches_fsw_mlp_call_after_call(capi):
     torch.cuda.synchronize()
     for (inp, g, want), Y, shape in zip(cases, outs, shapes):
         assert torch.equal(Y, want), "second pass differs at %s" % (shape,)
+    # the split-K streaming down projection (variant 104) behind another call's leftovers: the gate/up kernel zeroes its ticket
+    # counters, which sit in the array as well
+    inp, g, _ = cases[3]
+    try:
+        capi.set_variant(1, 104)
+        assert capi.variant_name(5, 0, 24, 4096, 14336) == "stream_split"
+        want = capi.mlp(g["X"], g["W13"], g["W2"])
+        for _ in range(3):
+            outs[3].fill_(float("nan"))
+            capi.mlp_static(g["X"], g["W13"], g["W2"], out=outs[3])
+            assert torch.equal(outs[3], want)
+    finally:
+        capi.set_variant(1, -1)
 
 
 # plan of the down projection with all the scratch it wants -> within the array: fewer splits, no split, H row-major
