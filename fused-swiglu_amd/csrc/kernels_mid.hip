@@ -84,9 +84,10 @@ mid_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const int gro
   const unsigned char* pbase = (const unsigned char*)a.P + (long long)p0 * a.ldp * 2;
   const unsigned char* qbase = (const unsigned char*)a.Q + (long long)q0 * a.ldq * 2;
 
-  // The copies start the launch: their code goes first, next to the prologue (behind the epilogue it is fetched into the instruction
-  // cache later: gate/up 9216 x 1280, 22 rows 8.1 -> 7.9 us)
-  if (__builtin_expect(wave >= NC, 1)) {
+  // The copies start the launch: where few rows leave little else to do their code goes first, next to the prologue (behind the epilogue it
+  // is fetched into the instruction cache later: gate/up 9216 x 1280, 22 rows 8.1 -> 7.9 us). Not on wider tiles (5632 x 1024, 130 rows 8.8 ->
+  // 9.2, 512 rows 10.1 -> 10.4).
+  if (FQ <= 2 ? __builtin_expect(wave >= NC, 1) : wave >= NC) {
     // ---- producers
     const int u = t - NC * 64;
     const int rb = u >> 3, pos = (u & 7) ^ ((rb >> 1) & 7);
@@ -406,7 +407,7 @@ static MidPlan find_plan(bool gated, int np, int nq, int k, bool ragged, int spl
     // start (mid_kernel's `rot`) for all these row counts. us, pieces -> whole: 28672 x 4096 (224 tiles) 16 rows 37.1 -> 36.5, 48 rows 38.4
     // -> 37.9; 28928 x 5568 (226) 11 rows 53.3 -> 51.2; 29056 x 5760 (227) 40 rows 53.7 -> 55.0. With fewer tiles, 27648 x 5120 (216), 16
     // rows 45.2 whole, 43.9 in pieces, 48 rows 51.4 and 49.7.
-    const bool whole = !ragged && t.fp == 4 && t.fq <= 2 && 8 * tp * tq >= 7 * 256 * rounds;
+    const bool whole = !ragged && nq <= 64 && t.fp == 4 && 8 * tp >= 7 * 256 * rounds;
     if (gated && tp * tq <= 1024 && !whole) {
       const long long pieces = rounds * 256 / tq;
       const int step = (int)(((np + pieces - 1) / pieces + 7) / 8 * 8);
