@@ -25,7 +25,8 @@ namespace fsw {
 // RS: weight rows (features) of a set, 16, or 8 or 4 where 16 would leave compute units idle (skinny_plan). The MFMA always takes 16
 // rows: the others repeat and are not stored.
 // U: steps whose loads are in flight at once; fewer rows a workgroup need more of them.
-template <class E, bool GATED, int MQ, int NW, bool XSLAB, int RS = 16, int U = 1>
+// UNROLLED: see the main loop
+template <class E, bool GATED, int MQ, int NW, bool XSLAB, int RS = 16, int U = 1, bool UNROLLED = (U > 1)>
 __global__ void __launch_bounds__(NW * 64)
 skinny_kernel(const GemmArgs a) {
   constexpr int T = GATED ? 2 : 1;   // accumulator sets (up, gate)
@@ -174,10 +175,10 @@ skinny_kernel(const GemmArgs a) {
     }
   };
   // The same steps written twice: the compiler keeps other registers and places the first loads elsewhere. Gate/up of up to 16 rows on eight
-  // and sixteen waves is 1 .. 5 % faster on the second form (6000 x 4096 1 row 11.8 -> 11.2 us); four waves and more rows are faster on the
-  // first (40960 x 5120 1 row 65.7 -> 62.6, 6912 x 1152 26 rows 6.7 -> 6.3, 16384 x 2048 40 rows 22.2 -> 21.4; not 11264 x 2048 24 rows,
-  // 15.5 -> 16.3).
-  if constexpr (U == 1 && !(GATED && MQ == 1 && NW >= 8)) {
+  // and sixteen waves is 1 .. 5 % faster on the second form (6000 x 4096 1 row 11.8 -> 11.2 us), on four waves of a short K where the activations
+  // pass through the slab (2960 x 800 14 rows 4.9 -> 4.6); the rest is faster on the first (40960 x 5120 1 row 65.7 -> 62.6, 6912 x 1152 26 rows
+  // 6.7 -> 6.3, 16384 x 2048 40 rows 22.2 -> 21.4; not 11264 x 2048 24 rows, 15.5 -> 16.3).
+  if constexpr (!UNROLLED) {
     if (s_begin < s_end) g_load(s_begin, 0);
     for (int step = s_begin; step < s_end; ++step) one_step(step, 0);
   } else {
@@ -251,15 +252,22 @@ namespace {
 template <class E, bool GATED, int MQ, int NW, int RS = 16, int U = 1>
 hipError_t launch_skinny_one(const GemmArgs& a, hipStream_t stream) {
   constexpr int R = GATED ? 2 * RS : RS;
+  constexpr bool UNROLLED = U > 1 || (GATED && MQ == 1 && NW >= 8);
   const int tiles = (a.np + R - 1) / R;
   if (tiles <= 0) return hipSuccess;
   if constexpr (MQ == 1) {
     if (a.nq <= 8) {
-      hipLaunchKernelGGL((skinny_kernel<E, GATED, MQ, NW, false, RS, U>), dim3((unsigned)tiles), dim3(NW * 64), 0, stream, a);
+      hipLaunchKernelGGL((skinny_kernel<E, GATED, MQ, NW, false, RS, U, UNROLLED>), dim3((unsigned)tiles), dim3(NW * 64), 0, stream, a);
       return hipGetLastError();
     }
+    if constexpr (GATED && NW == 4) {
+      if (a.k <= 896) {  // four waves because there are no more steps (skinny_plan)
+        hipLaunchKernelGGL((skinny_kernel<E, GATED, MQ, NW, true, RS, U, true>), dim3((unsigned)tiles), dim3(NW * 64), 0, stream, a);
+        return hipGetLastError();
+      }
+    }
   }
-  hipLaunchKernelGGL((skinny_kernel<E, GATED, MQ, NW, true, RS, U>), dim3((unsigned)tiles), dim3(NW * 64), 0, stream, a);
+  hipLaunchKernelGGL((skinny_kernel<E, GATED, MQ, NW, true, RS, U, UNROLLED>), dim3((unsigned)tiles), dim3(NW * 64), 0, stream, a);
   return hipGetLastError();
 }
 

@@ -245,3 +245,20 @@ def test_few_rows_are_summed_as_finely_as_by_the_weight_streaming_kernel(capi, M
             capi.set_variant(0, -1)
         error[v] = ((H.double() - ref).norm() / ref.norm()).item()
     assert max(error[v] for v in (202, 204, 210)) <= 1.1 * error[100], error
+
+
+@pytest.mark.parametrize("M,ff,K", [(14, 1480, 800), (9, 1500, 8), (16, 1000, 896)])
+def test_gateup_of_a_short_k_gives_the_bits_of_the_weight_streaming_kernel(capi, M, ff, K):
+    """Workgroups of four waves with a K of up to 896: against the kernel forced and the oracle, output inside a wider NaN buffer."""
+    inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + ff, x_scale=1.0)
+    X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
+    wide = torch.full((M, ff + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    capi.gateup(X, W, out=wide[:, :ff])
+    try:
+        capi.set_variant(0, 100)
+        few = capi.gateup(X, W)
+    finally:
+        capi.set_variant(0, -1)
+    assert torch.equal(wide[:, :ff], few) and torch.isnan(wide[:, ff:]).all()
+    pre = inp["X"].double() @ inp["W13"].double().T
+    assert_one_rounding(wide[:, :ff], pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2]), torch.bfloat16, "H %s" % ((M, ff, K),))
