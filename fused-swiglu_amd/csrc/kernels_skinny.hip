@@ -22,7 +22,7 @@
 
 namespace fsw {
 
-// RS: weight rows (features) of a set, 16, or 8 or 4 where 16 would leave compute units idle (skinny_plan). The MFMA always takes 16
+// RS: weight rows (features) of a set, 16, or 8 or 4 where 16 would leave compute units idle (launch_skinny). The MFMA always takes 16
 // rows: the others repeat and are not stored.
 // U: steps whose loads are in flight at once; fewer rows a workgroup need more of them.
 // UNROLLED: see the main loop
@@ -315,13 +315,15 @@ hipError_t launch_skinny(int dtype, bool gated, const GemmArgs& a, void* workspa
   (void)workspace;
   if (a.nq > 64) return hipErrorInvalidValue;
   const int mq = (a.nq + 15) / 16;
-  // Narrow outputs of the plain product: 16 features a workgroup are 64 .. 128 workgroups, each bound by what one compute unit
+  // Narrow outputs of the plain product: 16 features a workgroup are 32 .. 128 workgroups, each bound by what one compute unit
   // fetches; 8 (4) features are twice (four times) as many, and their waves need two steps (or twice the waves) in flight. us: 2816 ->
   // 1024 1 row 4.7 -> 4.2, 16 rows 5.9 -> 4.7; 4096 -> 1536 6.1 -> 5.2, 7.2 -> 6.3; 5632 -> 2048 8.0 -> 6.5, 9.7 -> 8.1; 8192 -> 2048 9.9
   // -> 8.0. Not with a second round of workgroups (8192 -> 3072 10.0 -> 12.9), not
   // for a handful of features (1024 -> 256 2.5 -> 2.7), and the gated product has two rows a feature as it is
   // (5632 x 1024 4.4 -> 4.9). Eight waves of two steps against sixteen of one and of two, eight of four: 2 .. 8 % less.
-  if (!gated && mq == 1 && a.np >= 512 && a.np <= 2048) {
+  // Nor with a short K, which has no steps for as many waves: 512 -> 512 2.3 -> 2.8, 1024 -> 512 2.6 -> 2.9, 1152 -> 512 3.2 -> 3.0; 512 -> 1024
+  // 2.6 -> 3.0, 768 -> 1024 level (16 rows 3.5 -> 3.4); 512 -> 2048 2.7 -> 3.0, 768 -> 2048 3.3 -> 3.1.
+  if (!gated && mq == 1 && a.np >= 512 && a.np <= 2048 && a.k > (a.np < 768 ? 1024 : a.np <= 1024 ? 640 : 512)) {
     if (a.np <= 1024) {
       return dtype == 0 ? launch_skinny_one<Bf16, false, 1, 16, 4, 1>(a, stream) : launch_skinny_one<Fp16, false, 1, 16, 4, 1>(a, stream);
     }
