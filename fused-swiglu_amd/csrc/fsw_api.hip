@@ -171,7 +171,10 @@ bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
   const int64_t bytes = 2 * np * k;
   if (family == 0) {
     const int64_t tiles = (np + 31) / 32;
-    if (m > 16) return tiles > 256 || rag;
+    // Ragged rows of few workgroups, us, skinny -> mid: 17 rows 2048 x 1160 6.1 -> 6.8, 2672 x 1336 6.5 -> 7.1, 4096 x 1640 8.3 -> 8.1, 6016 x
+    // 2008 9.9 -> 9.4; 32 rows 4096 x 1000 5.9 -> 6.4, 7808 x 1320 8.2 -> 7.7; 48 rows 1024 x 392 4.2 -> 4.6, 6000 x 968 6.9 -> 7.2, 4096 x 1000
+    // 6.6 -> 6.4, 2832 x 1096 7.1 -> 6.8.
+    if (m > 16) return tiles > 256 || (rag && (m <= 32 ? bytes >= (int64_t)12 << 20 : k >= 1000));
     if (tiles <= 256 || (m <= 8 && bytes < (int64_t)56 << 20)) return false;
     // Up to 8 rows skinny_kernel is as fast where its workgroups leave less than an eighth of their rounds of compute units empty (less than a
     // sixteenth above four rounds). us, 1 / 8 rows, skinny -> mid: 28672 x 4096 (896 workgroups) 37.6 -> 36.9 / 38.0 -> 36.6; 32768 x 4096
@@ -183,6 +186,10 @@ bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
     const int64_t rounds = (tiles + 255) / 256, empty = 256 * rounds - tiles;
     if (m <= 8 && !rag && !decode_stream_wanted(0, m, np, k) && empty <= (rounds <= 4 ? 32 : 16) * rounds)
       return tiles <= 640 && k % 1024 == 0;
+    // 9 .. 16 rows, 9 / 16 rows, us, skinny -> mid: 8704 x 512 4.5 -> 5.0 / 4.6 -> 5.0, 8704 x 1024 6.5 -> 6.8 / 6.7 -> 6.8, 12800 x 1024 level / 7.4
+    // -> 7.1, 24576 x 512 6.4 -> 6.6 / level; ragged 10000 x 520 5.3 -> 5.6 / 5.4 -> 5.7, 10000 x 1000 7.5 -> 7.7 / 7.9 -> 7.7, 8800 x 1320 9.3 ->
+    // 8.8 / 9.9 -> 8.9.
+    if (m > 8 && !(rag ? k * m >= 11000 : k >= 1024 && bytes >= (int64_t)22 << 20)) return false;
     return true;
   }
   const int64_t tiles = (np + 15) / 16;

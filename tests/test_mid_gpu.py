@@ -247,9 +247,9 @@ def test_few_rows_are_summed_as_finely_as_by_the_weight_streaming_kernel(capi, M
     assert max(error[v] for v in (202, 204, 210)) <= 1.1 * error[100], error
 
 
-@pytest.mark.parametrize("M,ff,K", [(14, 1480, 800), (9, 1500, 8), (16, 1000, 896)])
+@pytest.mark.parametrize("M,ff,K", [(17, 1112, 736), (48, 300, 200), (9, 4352, 256), (16, 4400, 264), (14, 1480, 800), (9, 1500, 8), (16, 1000, 896)])
 def test_gateup_of_a_short_k_gives_the_bits_of_the_weight_streaming_kernel(capi, M, ff, K):
-    """Workgroups of four waves with a K of up to 896: against the kernel forced and the oracle, output inside a wider NaN buffer."""
+    """Workgroups of four waves with a K of up to 896 among them: against the kernel forced and the oracle, output inside a wider NaN buffer."""
     inp = fsw_weights.make_inputs(M, K, ff, torch.bfloat16, seed=M + ff, x_scale=1.0)
     X, W = inp["X"].to(DEV), inp["W13"].to(DEV)
     wide = torch.full((M, ff + 8), float("nan"), dtype=torch.bfloat16, device=DEV)

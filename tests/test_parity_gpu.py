@@ -570,7 +570,7 @@ def test_swiglu_fwd_bf16_writes_dense_half_width_rows(ext):
         ext.swiglu_fwd_bf16(M, N + 1, K, g["X"], K, g["W13"], K, C, N)  # odd N
 
 
-@pytest.mark.parametrize("shape", [(16, 520, 8200), (64, 136, 11008), (128, 264, 13824), (100, 72, 8192), (40, 64, 10004)])
+@pytest.mark.parametrize("shape", [(16, 1032, 8200), (64, 136, 11008), (128, 264, 13824), (100, 72, 8192), (40, 64, 10004)])
 def test_weight_stream_cut_into_one_piece_per_compute_unit(capi, shape):
     """Gate/up with one tile of activation rows: the dispatcher hands every workgroup a piece lower than its tile (72, 88, 112 and
     80 weight rows here, as many pieces as compute units; whole tiles of 64 rows at 8192 features), which reads its missing
