@@ -197,6 +197,9 @@ bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
   if (tiles <= 128) return k > 12288 ? m > 4 || np > 1024 : rag && m > 12 && bytes >= (int64_t)12 << 20;
   if (rag) return bytes >= (int64_t)14 << 20 || (m >= 8 && bytes >= (int64_t)7 << 20);
   if (bytes >= (int64_t)1 << 28) return m > 4;
+    // Up to 4 rows with 257 .. 448 workgroups, which share the compute units unevenly but run at once, us, skinny -> mid: 8448 x 4800 1 row 19.1 ->
+    // 23.3, 10240 x 3776 16.1 -> 16.8, 12288 x 6016 25.1 -> 27.7, 13824 x 4800 21.4 -> 22.8, 15872 x 4800 level; 8 rows 10240 x 3776 17.5 -> 16.6.
+    if (m <= 4 && !rag && tiles <= 448 && k % 1024 != 0) return false;
   return tiles > 256;
 }
 
