@@ -10,17 +10,13 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 
-// bf16: v_mfma_f32_32x32x16_bf16 / v_mfma_f32_16x16x32_bf16, fp32 -> bf16 by v_cvt_pk_bf16_f32 (RNE, the
+// bf16: v_mfma_f32_16x16x32_bf16, fp32 -> bf16 by v_cvt_pk_bf16_f32 (RNE, the
 // rounding of cute::bfloat16_t(float) used at swiglu.cu:73-75).
 struct Bf16 {
-  static __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
   static __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
@@ -42,11 +38,8 @@ struct Bf16 {
   }
 };
 
-// fp16: v_mfma_f32_32x32x16_f16 / v_mfma_f32_16x16x32_f16, fp32 -> fp16 by v_cvt_f16_f32 (RNE).
+// fp16: v_mfma_f32_16x16x32_f16, fp32 -> fp16 by v_cvt_f16_f32 (RNE).
 struct Fp16 {
-  static __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
   static __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }

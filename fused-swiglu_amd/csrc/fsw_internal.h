@@ -46,14 +46,11 @@ inline long long blocked_bytes(long long rows, long long k) {
   return ((rows + 255) / 256) * ((k + 31) / 32) * (256 * 64);
 }
 
-// Names of the tiled kernels (kernels_tiled.hip). `variant` indexes tiled_variant_table().
+// Names of the tiled kernels (kernels_tiled.hip) by their ids in fsw_set_variant.
 struct TiledVariant {
   const char* name;
-  int bp, bq;        // workgroup tile: weight rows x activation rows
-  int threads;
 };
 int tiled_variant_count();
-int pair16_variant();  // index of the 256 x 256 kernel in the table
 const TiledVariant& tiled_variant(int variant);
 int raster_group(bool gated, int tiles_q);  // activation-row tiles per raster band of the tiled kernels
 // The 256 x 256 kernel on v_mfma_f32_16x16x32 (kernels_pair16.hip) for GemmArgs::layout 0, 1, 3, 5, 7.

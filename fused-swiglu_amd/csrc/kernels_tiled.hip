@@ -87,14 +87,13 @@ namespace {
 
 const TiledVariant kVariants[] = {
     // the first five name ranges of rows of the producer / consumer kernel (kernels_mid.hip) and, forced, its tile
-    {"dma_128x128", 128, 128, 512},
-    {"dma8w_128x256", 128, 256, 512},  // id 3 under an older number
-    {"dma_128x192", 128, 192, 512},
-    {"dma8w_128x256", 128, 256, 512},
-    {"dma_128x64", 128, 64, 512},
-    {"pair16_256x256", 256, 256, 256}, // v_mfma_f32_16x16x32 prefill kernel (kernels_pair16.hip), row-major operands
+    {"dma_128x128"},
+    {"dma8w_128x256"},  // id 3 under an older number
+    {"dma_128x192"},
+    {"dma8w_128x256"},
+    {"dma_128x64"},
+    {"pair16_256x256"}, // the prefill kernel (kernels_pair16.hip), row-major operands
 };
-constexpr int kPair16Variant = 5;
 
 }  // namespace
 
@@ -352,7 +351,6 @@ hipError_t launch_block_rows(const void* src, long long ld, int rows, int k, voi
 }
 
 int tiled_variant_count() { return (int)(sizeof(kVariants) / sizeof(kVariants[0])); }
-int pair16_variant() { return kPair16Variant; }
 const TiledVariant& tiled_variant(int variant) { return kVariants[variant]; }
 
 }  // namespace fsw
