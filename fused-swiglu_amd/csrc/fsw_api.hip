@@ -187,6 +187,9 @@ bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
     // 27648 x 5120 (864) 46.2 -> 43.4 / 48.2 -> 43.6; 20480 x 2560 (640) 18.9 -> 18.3; 37760 x 6336 (1180) 73.9 -> 71.3. Rows a multiple
     // of 2 KB apart are the exception: its eight-wave workgroups walk K in step and meet on the same memory channels (16384 x 4096 25.9 ->
     // 21.9, 16384 x 2048 13.4 -> 12.4, 16384 x 3072 18.2 -> 17.5).
+    // Up to 4 rows with 257 .. 448 workgroups, which share the compute units unevenly but run at once, us, skinny -> mid: 8448 x 4800 1 row 19.1 ->
+    // 23.3, 10240 x 3776 16.1 -> 16.8, 12288 x 6016 25.1 -> 27.7, 13824 x 4800 21.4 -> 22.8, 15872 x 4800 level; 8 rows 10240 x 3776 17.5 -> 16.6.
+    if (m <= 4 && !rag && tiles <= 448 && k % 1024 != 0) return false;
     const int64_t rounds = (tiles + 255) / 256, empty = 256 * rounds - tiles;
     if (m <= 8 && !rag && !decode_stream_wanted(0, m, np, k) && empty <= (rounds <= 4 ? 32 : 16) * rounds)
       return tiles <= 640 && k % 1024 == 0;

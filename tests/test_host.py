@@ -414,13 +414,14 @@ def test_kernels_that_run_in_the_ranges_of_few_rows(capi):
 
 
 def test_gateup_of_few_rows_or_a_short_k_stays_with_the_weight_streaming_kernel(capi):
-    """9 .. 48 rows: the producer / consumer kernel only where the weights are enough for it, on both sides of the lines."""
+    """9 .. 48 rows: the producer / consumer kernel only where the weights are enough for it, and not for up to 4 rows with few more
+    workgroups than compute units; both sides of the lines."""
     runs = lambda M, ff, k: capi.variant_name(3, 0, M, 2 * ff, k)
     for M, ff, K in [(17, 1112, 736), (32, 2048, 1000), (32, 1400, 1336), (48, 3000, 968), (9, 4352, 512), (16, 4352, 1024), (16, 8192, 768),
-                     (9, 5000, 1000), (16, 5000, 520)]:
+                     (9, 5000, 1000), (16, 5000, 520), (1, 5120, 3776), (4, 6912, 4800)]:
         assert runs(M, ff, K) == "skinny", (M, ff, K)
     for M, ff, K in [(17, 3904, 1320), (32, 2048, 1640), (48, 2048, 1000), (24, 4352, 512), (16, 4608, 1280), (16, 8192, 1024), (9, 4400, 1320),
-                     (16, 5000, 1000)]:
+                     (16, 5000, 1000), (8, 5120, 3776), (1, 5120, 4096)]:
         assert runs(M, ff, K).startswith("mid_"), (M, ff, K)
 
 
