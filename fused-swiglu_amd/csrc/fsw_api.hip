@@ -144,6 +144,16 @@ bool dma_variant(int v) { return (v >= 0 && v < V_256x256) || mid_variant(v); }
 // Rows of a dense operand of `k` columns that are no whole 128-byte lines.
 bool ragged(int64_t k) { return k % 64 != 0; }
 
+// Estimated time, us, of skinny_kernel's down projection of up to 48 rows and a K of up to 8192: 7 % rms over 448 timings. Rounds of one
+// workgroup of 16 features per compute unit, the activations (in blocks of 16 rows) that they all fetch from the L2, and more of these in
+// pieces of lines with ragged rows.
+double skinny_down_time(int64_t np, int64_t m, int64_t k, bool rag) {
+  const double tiles = (double)((np + 15) / 16), rounds = (double)(((np + 15) / 16 + 255) / 256);
+  const double over = tiles > 256 ? tiles / 256 : 1.0, fill = tiles / (256 * rounds);
+  const double blocks = 0.3 * (double)((m + 15) / 16) + 0.7 * (double)m / 16;
+  return 2.412 + (double)k / 1024 * (1.088 * rounds + blocks * over * (0.487 * fill + (rag ? 0.36 : 0.0)));
+}
+
 // Whether a launch that the rules above give to the kernels for few rows (`v`: VARIANT_SKINNY or a 128-row tile) runs the
 // producer / consumer kernel. skinny_kernel (one launch, one workgroup per 32 weight rows, 16 in the down projection) stays
 // where its workgroups fit the compute units at once and the call is short. Gate/up, us, skinny -> mid: 5632 x 1024 (176
@@ -196,6 +206,16 @@ bool mid_wanted(int family, int v, int64_t m, int64_t np, int64_t k, bool rag) {
     return true;
   }
   const int64_t tiles = (np + 15) / 16;
+  // K of up to 8192, where the second launch weighs most: only where the estimated time is less than skinny_kernel's (448 timings: the pair
+  // of estimates picks a kernel 0.3 % slower than the faster one on average, 12 % at worst; the rules below alone 11 % and 90 %). Not for ragged
+  // rows of more than 256 workgroups, where it flatters skinny_kernel (3800 -> 6000 1 row 12.9 -> 11.8); for up to 4 ragged rows it is too high
+  // (7312 -> 2376 1 row 10.1 -> 11.2). us, skinny -> mid: 17 rows 1000 -> 512
+  // 3.2 -> 6.1, 2048 -> 4096 5.9 -> 8.5, 6144 -> 2048 11.2 -> 10.2; 48 rows 2048 -> 2048 6.7 -> 8.0, 4104 -> 4096 15.1 -> 13.0; 1 row 1024 -> 5120
+  // 4.3 -> 6.2, 4096 -> 8192 12.9 -> 17.1, 6144 -> 5120 15.1 -> 14.0; ragged 1 row 3080 -> 4096 6.8 -> 9.2, 4104 -> 4880 13.0 -> 11.1, 16 rows
+  // 4744 -> 3104 10.9 -> 10.3.
+  if (k <= 8192 && (m > 16 || tiles > 128) && !(rag && tiles > 256 && k >= 3400) &&
+      fsw::mid_plan(false, (int)np, (int)m, (int)k, rag, 0, 16).us >= (rag && m <= 4 ? 0.86 : 0.98) * skinny_down_time(np, m, k, rag))
+    return false;
   if (m > 16) return rag || bytes >= (int64_t)8 << 20;
   if (tiles <= 128) return k > 12288 ? m > 4 || np > 1024 : rag && m > 12 && bytes >= (int64_t)12 << 20;
   if (rag) return bytes >= (int64_t)14 << 20 || (m >= 8 && bytes >= (int64_t)7 << 20);

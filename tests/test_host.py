@@ -413,6 +413,18 @@ def test_kernels_that_run_in_the_ranges_of_few_rows(capi):
         L.fsw_set_variant(1, -1)
 
 
+def test_down_projections_of_a_short_k_keep_one_launch(capi):
+    """Up to 48 rows and a K of up to 8192: K parts and a summing launch only where they are faster than the weight-streaming kernel, on
+    both sides of the lines (the scratch query follows)."""
+    runs = lambda M, d, k: capi.variant_name(4, 0, M, d, k)
+    for M, D, FF in [(17, 512, 1000), (32, 2048, 1000), (17, 4096, 4096), (48, 4096, 2048), (1, 5120, 1024), (16, 4352, 2048), (1, 8192, 4096),
+                     (1, 8192, 8192), (1, 4096, 3080), (10, 3584, 4104), (1, 6000, 2008), (1, 2376, 7312)]:
+        assert runs(M, D, FF) == "skinny" and capi.lib().fsw_down_workspace_bytes(0, M, D, FF) == 0, (M, D, FF)
+    for M, D, FF in [(17, 2048, 6144), (48, 4096, 4104), (48, 2048, 4096), (1, 4352, 6144), (16, 3104, 4744), (16, 3000, 8008), (1, 6000, 3800),
+                     (1, 4880, 4104), (17, 512, 20000), (1, 5120, 13824)]:
+        assert runs(M, D, FF).startswith("mid_") and capi.lib().fsw_down_workspace_bytes(0, M, D, FF) > 0, (M, D, FF)
+
+
 def test_gateup_of_few_rows_or_a_short_k_stays_with_the_weight_streaming_kernel(capi):
     """9 .. 48 rows: the producer / consumer kernel only where the weights are enough for it, and not for up to 4 rows with few more
     workgroups than compute units; both sides of the lines."""

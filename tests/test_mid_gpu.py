@@ -262,3 +262,20 @@ def test_gateup_of_a_short_k_gives_the_bits_of_the_weight_streaming_kernel(capi,
     assert torch.equal(wide[:, :ff], few) and torch.isnan(wide[:, ff:]).all()
     pre = inp["X"].double() @ inp["W13"].double().T
     assert_one_rounding(wide[:, :ff], pre[:, 0::2] * torch.nn.functional.silu(pre[:, 1::2]), torch.bfloat16, "H %s" % ((M, ff, K),))
+
+
+@pytest.mark.parametrize("M,D,FF", [(17, 512, 1000), (48, 264, 2056), (40, 4104, 520), (16, 4352, 512), (1, 5000, 1000), (9, 4200, 1800)])
+def test_down_projection_of_a_short_k_gives_the_bits_of_the_weight_streaming_kernel(capi, M, D, FF):
+    """No scratch, no K parts: against the kernel forced and the oracle, output inside a wider NaN buffer."""
+    gen = torch.Generator().manual_seed(M + FF)
+    H = (torch.randn(M, FF, generator=gen) * 0.5).to(torch.bfloat16)
+    W2 = (torch.randn(D, FF, generator=gen) / FF ** 0.5).to(torch.bfloat16)
+    wide = torch.full((M, D + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    capi.down(H.to(DEV), W2.to(DEV), out=wide[:, :D])
+    try:
+        capi.set_variant(1, 100)
+        few = capi.down(H.to(DEV), W2.to(DEV))
+    finally:
+        capi.set_variant(1, -1)
+    assert torch.equal(wide[:, :D], few) and torch.isnan(wide[:, D:]).all()
+    assert_one_rounding(wide[:, :D], H.double() @ W2.double().T, torch.bfloat16, "Y %s" % ((M, D, FF),))
