@@ -162,9 +162,9 @@ double skinny_down_time(int64_t np, int64_t m, int64_t k, bool rag) {
 // 19.4. Down, where K is split and a summing launch follows: 8192 -> 3072 16 rows 12.4 -> 13.1, 24 rows 15.2 -> 13.4; 13824 ->
 // 5120 (320 workgroups, two rounds) 1 row 31.3 -> 25.2; 16416 -> 4880 (ragged) 1 row 40.5 -> 28.7; up to 2048 features, where
 // skinny_kernel has 4 or 8 a workgroup, 2816 -> 1024 16 rows 4.7 -> 6.4, 8192 -> 2048 16 rows 10.1 -> 10.7, 16384 -> 2048 1 row
-// 16.2 -> 14.2, 16 rows 19.6 -> 15.2; ragged 5360 -> 1344 1 row 6.3 -> 8.1, 12 rows 8.2 -> 8.4, 16 rows 9.0 -> 8.4. Matrices of the persistent streaming kernel (decode_stream_wanted): gate/up 57344 x 8192 1 row 144.1 ->
-// 142.4, 16 rows 147.4 -> 136.5; 46336 x 7000 (ragged) 1 row 124.0 -> 98.8; down 28672 -> 8192 1 and 4 rows level, 16 rows
-// 84.1 -> 72.1; 23168 -> 7000 1 row 55.5 -> 52.1.
+// 16.2 -> 14.2, 16 rows 19.6 -> 15.2; ragged 5360 -> 1344 1 row 6.3 -> 8.1, 12 rows 8.2 -> 8.4, 16 rows 9.0 -> 8.4. Matrices of the
+// persistent streaming kernel (decode_stream_wanted): gate/up 57344 x 8192 1 row 144.1 -> 142.4, 16 rows 147.4 -> 136.5; 46336 x 7000
+// (ragged) 1 row 124.0 -> 98.8; down 28672 -> 8192 1 and 4 rows level, 16 rows 84.1 -> 72.1; 23168 -> 7000 1 row 55.5 -> 52.1.
 // The 256-row kernel fetches rows that are no whole lines by K tiles, every line twice; the gate/up product of such rows takes the
 // kernel whose estimated time is less (47 problems of 130 .. 700 rows: it chose the slower one four times, by 7 % at most; 38880 x
 // 5800 130 rows 150.4 -> 119.0, 256 rows 189.6 -> 138.1; 43680 x 7592 279 rows 348 -> 241; 24160 x 3448 409 rows stays, 93.6 and 105).
@@ -410,15 +410,12 @@ int fsw_gateup(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int64_
 
 // The reference's other build (C_TYPE float, constants.cuh:9-14; "C can work with either bf16 or fp32",
 // swiglu.cu:470-471): H is float and receives the gated fp32 value without a rounding. From 2^21 gated weight pairs on
-// (a layer of 1024 x 2816 has 2.9 million) it runs the kernel that the 16-bit output would run, whose tiles fit
-// the rows and the compute units (the persistent decode kernel has no float store: skinny_kernel there). Measured against
-// the weight-streaming kernel (up to 64 rows) and the 256 x 256 kernel (above), us: 4096 x 11008:
-// 40 rows 38.4 -> 31.6, 65 rows 64.6 -> 41.0, 130 rows 66.0 -> 50.1, 200 rows 66.6 -> 55.7; 1024 x 2816: 16 rows level,
-// 65 rows 21.0 -> 10.1, 300 rows 23.5 -> 10.9, 1000 rows 25.3 -> 18.5; 8192 x 28672: 40 rows 189 -> 150.
-// Smaller layers keep those two kernels. Up to 64 rows weight streaming is the faster one there (512 x 1408, 64 rows 6.5 us against
-// 7.1 on 128 x 64; 768 x 2048 6.4 against 9.3). Above, the small tiles would be (512 x 1408: 100 rows 14.7 against 8.5, 300 rows 15.8
-// against 7.5; 768 x 2048: 300 rows 19.0 against 9.2), but they add the products in another order: the results of such layers,
-// of which rounding gives the 256 x 256 kernel's 16-bit output bit for bit, would change in their last bits.
+// (a layer of 1024 x 2816 has 2.9 million) it runs the kernel that the 16-bit output runs, but for the decode range (few_rows), which
+// skinny_kernel keeps whole (the persistent streaming kernel has no float store). Against the weight-streaming kernel (up to 64 rows) and
+// the 256 x 256 kernel (above), us: 4096 x 11008: 40 rows 38.4 -> 30.0, 130 rows 66.0 -> 42.0; 4608 x 9216: 65 rows 33.5; 1024 x 2816: 65 rows
+// 21.0 -> 10.1, 300 rows 23.5 -> 9.4.
+// Smaller layers keep those two kernels: others add the products in another order, and the results of such layers, of which rounding gives
+// the 16-bit output of these kernels bit for bit, would change in their last bits.
 int fsw_gateup_f32out(int dtype, int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* W13,
                       int64_t ldw, float* H, int64_t ldh, void* stream) {
   const int rc = fsw_validate_gateup(dtype, M, N, K, X, ldx, W13, ldw, H, ldh);
@@ -441,8 +438,8 @@ int fsw_gateup_f32out(int dtype, int64_t M, int64_t N, int64_t K, const void* X,
   int v = M <= 64 ? VARIANT_SKINNY : V_256x256;
   if ((N / 2) * K >= (int64_t)1 << 21) {
     v = resolve_variant(0, M, N, K);
-    // Few rows stay on skinny_kernel, whose waves sum a quarter or less of K each: against float64 its result is 1.6e-7 off, with all of
-    // K in one chain of sums 4.1e-7, which only 16-bit outputs hide (the time it costs: 11.8 -> 12.6 us on one such call).
+    // The decode range stays on skinny_kernel, whose waves sum a quarter or less of K each: 1.6e-7 off float64 at 16384 x 2048. The rows past
+    // it have all of K in one chain of sums, as they had on the 128-row tiles that mid_kernel replaced (6.9e-7 at 27648 x 5120, 16 rows).
     if (v != VARIANT_SKINNY && mid_wanted(0, v, M, N, K, fsw::mid_ragged(a)))
       return finish(launch_gateup_mid(v, dtype, a, (hipStream_t)stream));
   }
@@ -518,7 +515,7 @@ static size_t down_split(int64_t M, int64_t D, int64_t FF, size_t limit, DownPla
 }
 
 // Least scratch that the down projection accepts: more than that only buys K parts on the producer / consumer kernel, which runs with
-// as many of them as there is room for.
+// as many of them as there is room for. What the 128-row tiles asked for is still asked for: a call that was refused stays refused.
 static size_t down_least(int64_t M, int64_t D, int64_t FF, size_t limit) {
   if (M <= 0 || D <= 0 || FF <= 0 || g_forced_variant[1] >= 0 || streams_weights(1, M, D, FF)) return 0;
   const size_t part = (size_t)M * (size_t)D * sizeof(float);

@@ -61,9 +61,8 @@ hipError_t launch_pair16_splitk(int dtype, const GemmArgs& a, hipStream_t stream
 // row-major [rows, k] (row stride ld elements) -> blocked; gated_order: W13's up/gate rows de-interleaved per panel
 hipError_t launch_block_rows(const void* src, long long ld, int rows, int k, void* dst, bool gated_order,
                              hipStream_t stream);
-// Plan for the plain (down-projection) product when the output has few tiles and K is deep: which direct-to-LDS
-// tile (128 or 256 square) and how many K partitions, so that about two workgroups per CU are in flight.
-// splits == 1 means the ordinary launch path.
+// Plan for the plain (down-projection) product when the output has few tiles and K is deep: which tile and how many K partitions.
+// splits == 1 means the ordinary launch path. Tiles 128 .. 130 are mid_kernel's, which then plans its own (mid_plan).
 struct SplitPlan {
   int tile;    // 128 (square), 129 = 128 output features x 256 activation rows, 130 = 128 x 192, else 256 x tile
                // (256, 224, 192 or 160 activation rows)

@@ -5,7 +5,8 @@
 // that an accumulator lane owns two are "up" and two "gate" rows of the same two features, so the gating (swiglu.cu:380-381) is
 // per-lane arithmetic without a de-interleave, and a tile may hold any multiple of 32 weight rows.
 //
-// What bounds it: the copies. A compute unit fetches 45 .. 60 bytes per ns when some of the lines come from HBM, whatever the
+// What bounds it: the copies. A compute unit fetches 45 .. 60 bytes per ns when some of the lines come from HBM (62 .. 76 on the 256-row
+// kernel's larger tiles, where the L2 serves more of them; 30 where all do and half the compute units fetch), whatever the
 // number of lines asked for ahead (copy loops of 2 .. 8 stages of 24 KB measure the same): the loads of a compute unit return in
 // order through its 32 KB L1, so an activation line that the L2 has at once waits behind the weight lines ahead of it. Time is
 // therefore bytes per compute unit, and the tile follows from it: any height of 32 weight rows and any multiple of 32 activation
@@ -316,7 +317,7 @@ mid_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const int gro
 namespace {
 
 struct MidTile {
-  int fp, fq, ns;  // tile of 32 fp weight rows x 32 fq activation rows, ring of ns lines (up to five, what 160 KB hold)
+  int fp, fq, ns;  // tile of 32 fp weight rows x 32 fq activation rows, ring of ns lines (five or what 160 KB hold, eight of the two smallest)
 };
 #define FSW_MID_TILES(X)                                                                                              \
   X(1, 1, 8) X(1, 2, 8) X(2, 1, 5) X(3, 1, 5) X(4, 1, 5) X(5, 1, 5) X(6, 1, 5) X(8, 1, 4) X(2, 2, 5) X(3, 2, 5) X(4, 2, 5) X(5, 2, 5)         \

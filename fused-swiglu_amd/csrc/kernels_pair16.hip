@@ -1,6 +1,5 @@
-// The prefill kernel of the dispatcher: 256 x 256 tiles on v_mfma_f32_16x16x32, weights in a ring of K-pair slots (or
-// 64-byte-row stages when prepacked), activations in a ring of four stages. Own translation unit: it is the largest
-// set of instances of the library and compiles beside kernels_tiled.hip, which keeps the 32x32x16 kernels.
+// The prefill kernel of the dispatcher: tiles of 256 weight rows x 160 .. 256 activation rows on v_mfma_f32_16x16x32, weights in a ring of
+// K-pair slots, activations in pair slots or, panel-blocked, in four stages. Own translation unit: it is a large set of instances and compiles beside the others.
 #include <type_traits>
 
 #include "fsw_internal.h"

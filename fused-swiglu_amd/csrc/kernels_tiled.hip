@@ -167,7 +167,9 @@ double pair16_ragged_time(int np, int nq, int k, int rows) {
 // than the fastest one on average, 12 % at worst.
 //   * a workgroup's K tiles of 64: 1.19 us on 256 x 256 plus 1.9 us to fill and drain the pipeline (what shallow parts pay
 //     for: 1996 rows of 2088 -> 736 in two parts of 17 tiles 34.4 us on 256 x 160, 22.2 on 128 x 128), 0.6 us on 128 x 128
-//     alone on a compute unit (three stages), 1.6 .. 1.83 times that where 257 .. 512 workgroups share them two by two;
+//     alone on a compute unit, 1.6 .. 1.83 times that with 257 .. 512 workgroups. The 128 x 128 terms are those of the kernel that mid_kernel
+//     replaced there; they still draw the line between the 256-row kernel and mid_kernel, which then plans its own tile and parts by
+//     mid_plan() and is faster than they say (down 2816 -> 1024, 512 rows 15.9 -> 13.5; 8192 -> 2048, 371 rows 27.0 -> 25.7);
 //   * a round costs the same whether 100 or 256 compute units are in it, but 256 workgroups of eight parts and more take
 //     a fifth longer (4096 x 11008, 426 rows on 256 x 224: seven parts 53.7 us, eight 65.7);
 //   * K no multiple of 64: rows share cache lines, all tiles take 1.22 times as long;
@@ -195,8 +197,8 @@ static const struct {
   double cost;  // of a K tile against 256 x 256
 } kSplitTiles[] = {{128, 0.0}, {256, 1.0}, {224, 0.926}, {192, 0.863}, {160, 0.797}};
 
-// The fastest plan by split_time() among those that are resident at once (two 128 x 128 workgroups or one large one per
-// compute unit: a second, partly filled round costs a whole one), whose parts are 8 (16) K tiles deep at least and whose
+// The fastest plan by split_time() among those of one round (256 large workgroups, 512 of 128 x 128: a second, partly filled round costs
+// a whole one; mid_kernel's own plan takes these parts as the most it may have), whose parts are 8 (16) K tiles deep at least and whose
 // partial sums stay under 256 MB. Tiles half filled with rows and row counts that are multiples of 256 need no rule of their own.
 // Down projection, us, with 128 x 128 and 256 x 256 tiles only / with an estimate that knew neither the fill of short parts nor
 // the three-stage ring and left half-filled tiles out / with this one: 28672 -> 8192, 264 rows 170 / 239 / 144; 8192 -> 2048,
@@ -279,8 +281,8 @@ SplitPlan tiled_split_plan(int np, int nq, int k) {
     tiles = t256;
     by_k = k / 1024;
   }
-  // One tile of activation rows: three-stage workgroups, one per compute unit, beat two two-stage ones (less
-  // partial-sum traffic as well); 129..256 rows take one 128 x 256 tile per workgroup for the same reason.
+  // Up to 256 rows mid_plan() plans what runs; these parts name the range and are the least scratch that a call of 49 .. 256 rows has to
+  // bring (down_least). One tile of activation rows: one workgroup per compute unit.
   int target = 512;
   if (nq <= 128) {
     target = 256;
