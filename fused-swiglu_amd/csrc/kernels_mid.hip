@@ -203,7 +203,8 @@ mid_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const int gro
   if constexpr (FQ <= 2) {
     // GemmArgs::short_sums (few rows, where a second set of accumulators fits): every four K tiles the sums so far go to the totals and
     // start again, so that no value is the end of one chain of K / 32 sums. Off float64, gate/up unrounded, one chain -> this (skinny_kernel):
-    // 27648 x 5120 6.6e-7 -> 2.0e-7 (3.1e-7), 16384 x 2048 4.2e-7 -> 1.6e-7 (1.6e-7).
+    // 27648 x 5120 6.6e-7 -> 2.0e-7 (3.1e-7), 16384 x 2048 4.2e-7 -> 1.6e-7 (1.6e-7). The four is a constant: with chains of an eighth of K the
+    // compiler (ROCm 7.2) let the 32 x 32 tile add the sums two wait states behind the last MFMA, which needs seven, and they were wrong.
     f32x4 total[FP][FQ];
 #pragma unroll
     for (int f = 0; f < FP; ++f)
