@@ -57,7 +57,7 @@ int check_device() {
 // indices of the tiled kernels (tiled_variant() of kernels_tiled.hip)
 constexpr int V_128x128 = 0, V_128x192 = 2, V_8W_128x256 = 3, V_128x64 = 4, V_256x256 = 5;
 
-// Range of rows of a tiled launch. The 128-row names stand for the producer / consumer kernel (kernels_mid.hip), which chooses its
+// Range of rows of a tiled launch. The 128-row names stand for the producer / consumer kernel (mid_kernel.h), which chooses its
 // tile by an estimate of its own; they tell the rows that one of its launches shares the weights between (128 x 64: up to 64, 128 x
 // 128 and so on) and are what fsw_set_variant forces. The others are the 256-row kernel.
 // `narrow_need`: a narrower large tile is taken only if its estimated time is below this share of 256 x 256's

@@ -80,7 +80,7 @@ double pair16_split_time(int np, int nq, int k, const SplitPlan& plan);
 
 hipError_t launch_splitk_reduce(int dtype, const GemmArgs& a, hipStream_t stream);  // sums a.partial's a.splits parts into a.O
 
-// Producer / consumer kernel (kernels_mid.hip): tiles of 32 .. 256 weight rows x 32 .. 256 activation rows.
+// Producer / consumer kernel (mid_kernel.h): tiles of 32 .. 256 weight rows x 32 .. 256 activation rows.
 struct MidPlan {
   int tile;    // index of the tile, -1: none
   int step;    // weight rows a workgroup owns (<= the tile's, a multiple of 8)

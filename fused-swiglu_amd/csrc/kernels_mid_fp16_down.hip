@@ -1,0 +1,10 @@
+// The producer / consumer kernel (mid_kernel.h), fp16, plain product.
+#include "mid_kernel.h"
+
+namespace fsw {
+
+hipError_t launch_mid_fp16_down(const MidPlan& p, const GemmArgs& a, int ph, hipStream_t stream) {
+  return launch_mid_typed<Fp16, false>(p, a, ph, stream);
+}
+
+}  // namespace fsw

@@ -1,5 +1,5 @@
 // Plans of the tiled kernels (which tile, how many K parts), the split-K reduction and the row-major -> panel-blocked copy. The
-// kernels live in kernels_pair16.hip (256 weight rows a tile, prefill) and kernels_mid.hip (smaller tiles).
+// kernels live in kernels_pair16.hip (256 weight rows a tile, prefill) and mid_kernel.h (smaller tiles).
 //
 // Orientation of both. The MFMA "A" operand (rows of the result block) is fed with WEIGHT rows and the "B" operand (columns of
 // the result) with ACTIVATION rows, so an accumulator lane owns one activation row m and runs of consecutive output features,
@@ -86,7 +86,7 @@ block_rows_kernel(const unsigned short* __restrict__ src, long long ld, int rows
 namespace {
 
 const TiledVariant kVariants[] = {
-    // the first five name ranges of rows of the producer / consumer kernel (kernels_mid.hip) and, forced, its tile
+    // the first five name ranges of rows of the producer / consumer kernel (mid_kernel.h) and, forced, its tile
     {"dma_128x128"},
     {"dma8w_128x256"},  // id 3 under an older number
     {"dma_128x192"},
@@ -97,7 +97,7 @@ const TiledVariant kVariants[] = {
 
 }  // namespace
 
-// Activation-row tiles per raster band of the 256 x 256 kernel (kernels_mid.hip uses 4 for the gate/up and 2 for the down
+// Activation-row tiles per raster band of the 256 x 256 kernel (mid_kernel uses 4 for the gate/up and 2 for the down
 // product): 4, i.e. the 32 tiles an XCD runs at once are 4 activation panels x 8 weight
 // panels (12 operand panels through its L2 per round). The down product of tall problems (32 activation tiles or
 // more, 16 weight panels, 14336-deep K) measures level to 1 % slower that way and keeps bands of 2; with fewer

@@ -21,7 +21,8 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OBJ_DIR = os.path.join(HERE, "build", "hip_obj")
 LIB_NAME = "libfsw_hip.so"
-HIP_SOURCES = ["kernels_pair16.hip", "kernels_mid.hip", "kernels_tiled.hip", "kernels_skinny.hip", "kernels_stream.hip", "kernels_decode.hip", "fsw_api.hip"]
+HIP_SOURCES = ["kernels_pair16.hip", "kernels_mid_bf16_gateup.hip", "kernels_mid_bf16_down.hip",
+               "kernels_mid_fp16_gateup.hip", "kernels_mid_fp16_down.hip", "kernels_mid.hip", "kernels_tiled.hip", "kernels_skinny.hip", "kernels_stream.hip", "kernels_decode.hip", "fsw_api.hip"]
 PROBE_LIB_NAME = "libfsw_probe.so"  # measurement kernels of the benchmark (include/fsw_probe.h): not part of the product
 PROBE_SOURCES = ["probes.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -70,6 +70,33 @@ def test_every_tile_at_its_edges(capi, index):
                 assert torch.equal(wide[:, :ff], first[0][:, :ff]) and torch.equal(P, first[1]), what
 
 
+@pytest.mark.parametrize("index", range(N_TILES))
+def test_rings_and_left_out_copies(capi, index):
+    """K of 3 .. 13 lines (fewer than a ring holds, as many, a few more: the last of them masked), whole and with a tail, dense and in
+    padded rows; weight and activation rows that end 8 rows or more before the tile does, where waves leave copies out."""
+    bp, bq = tile_rows(capi, index)
+    for lines in range(3, 14):
+        M, ff = bq - (8, 9, 17, 31)[lines % 4], bp // 2 - (0, 4, 8, 15)[lines // 4]
+        K = 64 * lines - (0, 8, 40)[lines % 3]
+        g = torch.Generator(device=DEV).manual_seed(100 * index + lines)
+        X = torch.randn(M, K, device=DEV, generator=g).to(torch.bfloat16)
+        W = (torch.randn(2 * ff, K, device=DEV, generator=g) / K ** 0.5).to(torch.bfloat16)
+        plain = X.double() @ W.double().t()
+        want = plain[:, 0::2] * torch.nn.functional.silu(plain[:, 1::2])
+        for pad in (0, (-K) % 64):
+            Xp, Wp = lay(X, pad, 0), lay(W, pad, 0)
+            try:
+                capi.set_variant(0, 200 + index)
+                capi.set_variant(1, 200 + index)
+                H, P = capi.gateup(Xp, Wp), capi.down(Xp, Wp)
+            finally:
+                capi.set_variant(0, -1)
+                capi.set_variant(1, -1)
+            what = "tile %d (%d x %d) %s pad %d" % (index, bp, bq, (M, ff, K), pad)
+            assert_one_rounding(H, want.cpu(), torch.bfloat16, what)
+            assert_one_rounding(P, plain.cpu(), torch.bfloat16, what + " plain")
+
+
 @pytest.mark.parametrize("M", [1, 8, 17, 33, 100, 200, 300])
 @pytest.mark.parametrize("D,FF", [(1096, 8008), (1024, 16384), (3000, 4872)])
 def test_down_projection_in_parts_of_k(capi, M, D, FF):
