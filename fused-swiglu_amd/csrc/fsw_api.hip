@@ -500,11 +500,18 @@ static DownPlan down_plan(int64_t M, int64_t D, int64_t FF, size_t limit, bool r
   r.plan = fsw::tiled_split_plan((int)D, (int)M, (int)FF);
   if (r.plan.splits > most) r.plan.splits = most < 1 ? 1 : (int)most;
   r.mid = r.plan.splits > 1 ? r.plan.tile <= 130 : dma_variant(v);
-  // rows that are no whole lines: the same parts on whichever kernel takes them faster by the estimates (8008 -> 3000 300 rows
-  // 39.6 -> 28.8 us, 900 rows 62.9 -> 58.8; 23568 -> 6168 499 rows stays, 152 and 189)
-  if (!r.mid && rag && r.plan.splits > 1 && M <= 1024)
-    r.mid = fsw::mid_plan(false, (int)D, (int)M, (int)FF, true, 0, r.plan.splits).us <
-            0.95 * fsw::pair16_split_time((int)D, (int)M, (int)FF, r.plan);
+  // The same parts or fewer on whichever kernel takes them faster by the estimates. Outputs of up to 3072 features, whole lines: mid_kernel's
+  // is 8 % high where the 256-row kernel's is right, but for tiles of 224 and 256 activation rows (3 lines in a ring). Down, us, 256-row
+  // kernel -> mid_kernel: 8192 -> 2048 333 rows 30.3 -> 24.3, 656 rows 41.8 -> 35.9, 700 rows 39.3 -> 34.3, 768 rows 45.3 -> 39.2. Wider
+  // ones are level within what one call differs from run to run (11008 -> 4096 359 rows 52 and 57, 384 rows 48.5 and 45.0; 14336 -> 4096 333
+  // rows 55.7 and 52.2, the forward 135 either way). Other rows: 8008 -> 3000 300 rows 39.6 -> 28.8, 900 rows 62.9 -> 58.8; 23568 -> 6168
+  // 499 rows stays, 152 and 189.
+  if (!r.mid && r.plan.splits > 1 && M <= 1024) {
+    const bool narrow = !rag && D <= 3072;
+    const fsw::MidPlan p = fsw::mid_plan(false, (int)D, (int)M, (int)FF, rag, 0, r.plan.splits);
+    r.mid = (rag || (narrow && fsw::mid_tile_cols(p.tile) <= 192)) &&
+            p.us < (narrow ? 1.05 : 0.95) * fsw::pair16_split_time((int)D, (int)M, (int)FF, r.plan);
+  }
   return r;
 }
 

@@ -92,6 +92,7 @@ struct MidPlan {
 MidPlan mid_plan(bool gated, int np, int nq, int k, bool ragged, int splits, int max_splits);
 int mid_tile_count();
 int mid_tile_rows(int tile);  // weight rows of a whole tile
+int mid_tile_cols(int tile);  // activation rows
 int mid_tile_index(int bp, int bq);
 const char* mid_name(const MidPlan& p);
 inline bool mid_ragged(const GemmArgs& a) {

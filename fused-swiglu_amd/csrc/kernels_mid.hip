@@ -130,6 +130,7 @@ const char* mid_name(const MidPlan& p) {
 
 int mid_tile_count() { return kNumTiles; }
 int mid_tile_rows(int tile) { return 32 * kMidTiles[tile].fp; }
+int mid_tile_cols(int tile) { return 32 * kMidTiles[tile].fq; }
 int mid_tile_index(int bp, int bq) {
   for (int i = 0; i < kNumTiles; ++i)
     if (kMidTiles[i].fp * 32 == bp && kMidTiles[i].fq * 32 == bq) return i;

@@ -113,6 +113,35 @@ def test_down_projection_in_parts_of_k(capi, M, D, FF):
         capi.gateup(inp["X"].to(DEV), inp["W13"].to(DEV)), inp["W2"].to(DEV)))
 
 
+@pytest.mark.parametrize("M,D,FF", [(656, 2048, 8192), (999, 1530, 6144), (257, 3072, 12288), (259, 3070, 12288)])
+def test_down_projection_of_more_rows_on_narrow_outputs(capi, M, D, FF):
+    """Rows past 256 whose parts the 256-row kernel took: H and W2 in rows of whole lines beside NaN, output inside a wider NaN buffer, all of
+    the scratch and the least that is accepted with a guard behind it; against float64 and against the 256-row kernel."""
+    L = capi.lib()
+    assert capi.variant_name(1, 0, M, D, FF).startswith("splitk_pair16") and capi.variant_name(4, 0, M, D, FF).startswith("mid_")
+    H = (torch.randn(M, FF, device=DEV) * 0.3).to(torch.bfloat16)
+    W2 = (torch.randn(D, FF, device=DEV) / FF ** 0.5).to(torch.bfloat16)
+    ref = (H.double() @ W2.double().t()).cpu()
+    Hp, Wp = lay(H, 64, 0), lay(W2, 128, 0)
+    nbytes, part = L.fsw_down_workspace_bytes(0, M, D, FF), 4 * M * D
+    assert nbytes >= 2 * part
+    ws = torch.full((nbytes + 256,), 7, dtype=torch.uint8, device=DEV)
+    wide = torch.full((M, D + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    args = (0, M, D, FF, Hp.data_ptr(), Hp.stride(0), Wp.data_ptr(), Wp.stride(0), wide.data_ptr(), D + 8)
+    assert L.fsw_down(*args, ws.data_ptr(), nbytes, stream) == capi.OK
+    assert (ws[nbytes:] == 7).all() and torch.isnan(wide[:, D:]).all()
+    assert_one_rounding(wide[:, :D], ref, torch.bfloat16, "parts")
+    assert L.fsw_down(*args, ws.data_ptr(), nbytes - part, stream) != capi.OK  # refused as before
+    try:
+        capi.set_variant(1, 5)
+        large = capi.down(H, W2)
+    finally:
+        capi.set_variant(1, -1)
+    # either is one rounding of a sum off by fp32 noise: they differ by an ulp where the sum lies next to a tie
+    assert ((wide[:, :D].float() - large.float()).abs() <= large.float().abs() * 2.0 ** -7 + 1e-3).all()
+
+
 def test_down_projection_of_few_rows_runs_without_scratch(capi):
     """Up to 48 rows the weight-streaming kernel needs none: a caller that brings no workspace gets that kernel, not an error."""
     M, D, FF = 20, 2048, 8192
