@@ -90,6 +90,12 @@ static MidPlan find_plan(bool gated, int np, int nq, int k, bool ragged, int spl
       }
       for (int i = 0; i < 3; ++i) {
         if (sps[i] < 1) continue;
+        // Three activation lines and rows that are no whole lines: the shift takes one line of the ring, so every step waits for the activation
+        // line that it asked for, which short parts of K do not make up for. Down, 193 .. 256 rows, against the plans of tiles with four lines
+        // and more: parts of fewer than 24 lines 1.03 of their time (151 problems, 0.93 .. 1.15; 10840 -> 2728 195 rows 27.6 us on 96 x 224 in
+        // 8 parts, 31.8 on 128 x 224 in 11), longer ones 0.93 (189, 0.78 .. 1.03; 24560 -> 6288 193 rows 99 and 77). Whole K is faster, too: 160
+        // gate/up problems of 65 .. 1024 rows 0.86 (0.70 .. 1.09; 25776 x 3664 199 rows 62.5 and 50.3, 57104 x 7176 204 rows 214 and 197).
+        if (ragged && t.na < 4 && sps[i] > 1 && (k + 63) / 64 < 24 * sps[i]) continue;
         double us = mid_time(np, nq, k, ragged, t, steps[s], sps[i]);
         // The estimate flatters fewer parts on lower tiles, which fetch every activation row for fewer weight rows (11008 -> 4096,
         // 200 rows: four parts on 64 x 224 38.4 us, eight on 128 x 224 34.5; 14336 -> 4096, 256 rows 48.8 and 45.6).

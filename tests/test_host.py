@@ -3,6 +3,7 @@ argument validation returns the documented codes before any HIP call, the packer
 row interleave, and the operator surface matches csrc/torch_bindings.cpp:31-50 of the reference."""
 import ctypes
 import os
+import random
 import re
 
 import pytest
@@ -468,3 +469,23 @@ def test_forward_takes_scratch_for_h_alone_where_k_parts_are_optional(capi, M, d
     assert call(h) == capi.E_NULL and call(h - 1) == capi.E_WORKSPACE
     M, d, ff = 200, 512, 4096  # a range that refused less than its K parts when it had no kernel without them, and still does
     assert call(2 * M * ff) == capi.E_WORKSPACE
+
+
+def test_ragged_rows_take_rings_of_three_activation_lines_on_long_parts_only(capi):
+    """Rows that are no whole 128-byte lines leave a ring of three activation lines without a copy under way: not for K parts of fewer than
+    24 lines, both sides of the line."""
+    three = ("mid_128x224", "mid_96x256", "mid_128x256")
+    runs = lambda M, D, FF: capi.variant_name(4, 0, M, D, FF)
+    parts = lambda M, D, FF: capi.lib().fsw_down_workspace_bytes(0, M, D, FF) // (4 * M * D)
+    for M, D, FF in [(195, 2728, 10840), (224, 2752, 10224), (224, 3456, 9368), (196, 2968, 11208), (253, 3040, 14736)]:
+        assert runs(M, D, FF) in ("mid_96x224", "mid_192x128") and parts(M, D, FF) in (7, 8), (M, D, FF)
+    for M, D, FF in [(193, 6288, 24560), (251, 5368, 20168), (242, 3576, 17296)]:
+        assert runs(M, D, FF) in three, (M, D, FF)
+    rng = random.Random(3)
+    for _ in range(400):
+        M, D, FF = rng.randint(193, 256), 8 * rng.randint(90, 800), 8 * rng.randint(300, 2000)
+        if FF % 64 and runs(M, D, FF) in three and parts(M, D, FF) > 1:
+            assert (FF + 63) // 64 >= 24 * parts(M, D, FF), (M, D, FF)
+    # whole K is faster on them, and whole lines have no line to spare for a shift
+    assert capi.variant_name(3, 0, 245, 30784, 4464) == "mid_128x256" and capi.variant_name(3, 0, 206, 56000, 7512) == "mid_128x224"
+    assert runs(195, 2728, 10880) in three and parts(195, 2728, 10880) > 8
