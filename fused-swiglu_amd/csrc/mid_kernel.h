@@ -83,9 +83,13 @@ constexpr int copies_behind(int parity, int ph, int g, int nw, int na, int lp, i
   return behind;
 }
 
+// bits of the kernel's `how`
+constexpr int MID_STREAM = 1;  // weight lines are non-temporal
+constexpr int MID_SPREAD = 2;  // workgroups start their walk over K at different lines
+
 template <class E, bool GATED, int FP, int FQ, int PAIRS, int NW, int NA>
 __global__ void __launch_bounds__(512)
-mid_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const int group, const int ph, const int stream_w) {
+mid_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const int group, const int ph, const int how) {
   constexpr int NC = 4;
   constexpr int WP = 2, WQ = 2, BP = WP * FP * 16, BQ = WQ * FQ * 16;
   constexpr int LP = BP / 32, LQ = BQ / 32;
@@ -109,7 +113,7 @@ mid_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const int gro
   const int kt_per = (nkt_all + a.splits - 1) / a.splits;
   const int kt0 = (int)blockIdx.y * kt_per;
   const int nkt = nkt_all - kt0 < kt_per ? (nkt_all - kt0 > 0 ? nkt_all - kt0 : 0) : kt_per;
-  const int rot = (!ph && tiles_q == 1 && nkt > 1 && (a.k & 63) == 0) ? (int)(((unsigned)blockIdx.x * 2654435761u >> 12) % (unsigned)nkt) : 0;
+  const int rot = (how & MID_SPREAD) && nkt > 1 ? (int)(((unsigned)blockIdx.x * 2654435761u >> 12) % (unsigned)nkt) : 0;
   const unsigned char* pbase = (const unsigned char*)a.P + (long long)p0 * a.ldp * 2;
   const unsigned char* qbase = (const unsigned char*)a.Q + (long long)q0 * a.ldq * 2;
 
@@ -160,7 +164,7 @@ mid_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const int gro
                                              (int)(in ? (OFF) + (unsigned)rel : OOB_OFFSET), 0, 0, AUX);                     \
   else                                                                                                                       \
     __builtin_amdgcn_raw_ptr_buffer_load_lds(RSRC, (lds_void*)(st + (I) * 32 * 128), 16, (int)(OFF), rel, 0, AUX)
-        if (stream_w) {
+        if (how & MID_STREAM) {
 #pragma unroll
           for (int i = 0; i < CP; ++i) { FSW_MID_COPY(prs, poff[i], i, 2); }
         } else {
@@ -211,7 +215,8 @@ mid_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const int gro
           else wait_copies<copies_behind(1, 0, G, LW, NA, CP, CQ)>();
         }
       };
-      const int whole = ph || (a.k & 63) != 0 ? nkt - 1 : nkt;  // lines behind the prologue's and before this one are whole
+      // Lines behind the prologue's and before this one are whole: all, or those before the line that K ends in (ph: before the last, too)
+      const int whole = ph ? nkt - 1 : (a.k & 63) != 0 && kt0 + nkt == nkt_all ? nkt - 1 - rot : nkt;
       constexpr int AHEAD = NA > LW - 1 + (G == 1) ? NA : LW - 1 + (G == 1);
       for (; kt + AHEAD < whole; kt += 2) {
         step(0, std::false_type{});
@@ -430,8 +435,16 @@ hipError_t launch_mid_tile(const MidPlan& p, const GemmArgs& a, int ph, hipStrea
   GemmArgs b = a;
   b.tile_p = p.step;
   // whole lines are non-temporal when at most two tiles of activation rows share them
+  int how = tiles_q <= 2 ? MID_STREAM : 0;
+  // Where one tile holds all activation rows, the walks over K start at different lines, so that workgroups do not meet on the same memory
+  // channels. Padded rows whose K ends inside a line do that only with weight rows a multiple of 4 KB apart, which all start on one channel
+  // (all from line 0 -> spread, us: gate/up 47040 x 6096 in rows of 6144 7 rows 112 -> 84, 31648 x 4080 15 rows 53 -> 41, down 14328 -> 5600 35
+  // rows 38.7 -> 31.3; 92 such problems 0.96, 49 with other strides 1.02), and while the activations fit an XCD's 4 MB L2, for all their lines
+  // are in use at once then (down 20464 -> 7496 174 rows, 7 MB, 74 and 100; 16344 -> 4464 161 rows, 5 MB, 41 and 51).
+  const bool line_tail = (a.k & 63) != 0;
+  if (!ph && tiles_q == 1 && (!line_tail || ((a.ldp & 2047) == 0 && (long long)a.nq * a.k <= 1 << 21))) how |= MID_SPREAD;
   hipLaunchKernelGGL((mid_kernel<E, GATED, FP, FQ, G, NW, NA>), dim3((unsigned)(tiles_p * tiles_q), (unsigned)a.splits), dim3(512),
-                     0, stream, b, tiles_p, tiles_q, GATED ? 4 : 2, ph, tiles_q <= 2 ? 1 : 0);
+                     0, stream, b, tiles_p, tiles_q, GATED ? 4 : 2, ph, how);
   return hipGetLastError();
 }
 

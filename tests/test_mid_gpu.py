@@ -113,6 +113,33 @@ def test_down_projection_in_parts_of_k(capi, M, D, FF):
         capi.gateup(inp["X"].to(DEV), inp["W13"].to(DEV)), inp["W2"].to(DEV)))
 
 
+@pytest.mark.parametrize("tile", [0, 2, 10, 14, 22, 30])
+@pytest.mark.parametrize("M,K,ld,spread", [(20, 2048, 2048, True), (20, 2040, 2048, True), (20, 2040, 2112, False), (20, 4088, 4096, True),
+                                           (31, 6104, 6144, True)])
+def test_workgroups_start_their_walk_over_k_at_different_lines(capi, tile, M, K, ld, spread):
+    """All weight rows are the same two, so every workgroup sums the same products: in one order, and to the same float32 bits, if they all
+    start at line 0, in different orders if the walk is spread. Off float64 at most what fp32 sums of K products in any order are."""
+    gen = torch.Generator(device=DEV).manual_seed(K + M)
+    ff = 4096
+    X = torch.randn(M, ld, generator=gen, device=DEV).to(torch.bfloat16)[:, :K]
+    pair = (torch.randn(2, K, generator=gen, device=DEV) / K ** 0.5).to(torch.bfloat16)
+    W = torch.full((2 * ff, ld), float("nan"), dtype=torch.bfloat16, device=DEV)[:, :K]
+    W[0::2], W[1::2] = pair[0], pair[1]
+    try:
+        capi.set_variant(0, 200 + tile)
+        H = capi.gateup_f32out(X, W)
+    finally:
+        capi.set_variant(0, -1)
+    assert (H != H[:, :1]).any().item() == spread
+    pre = X.double() @ pair.double().t()
+    want = (pre[:, 0] * torch.nn.functional.silu(pre[:, 1]))[:, None]
+    # a sum of K products whose absolute values add up to S is off by at most (K / 32 + 32) rounding errors of 2^-24 S; the two sums enter the
+    # result multiplied by at most 1.1 |up| + |gate| (silu' <= 1.1)
+    S = X.double().abs() @ pair.double().abs().t()
+    bound = (K / 32 + 32) * 2.0 ** -24 * (S[:, 0] * pre[:, 1].abs() + 1.1 * S[:, 1] * pre[:, 0].abs())[:, None] + 1e-6 * want.abs() + 1e-9
+    assert ((H.double() - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("M,D,FF", [(656, 2048, 8192), (999, 1530, 6144), (257, 3072, 12288), (259, 3070, 12288)])
 def test_down_projection_of_more_rows_on_narrow_outputs(capi, M, D, FF):
     """Rows past 256 whose parts the 256-row kernel took: H and W2 in rows of whole lines beside NaN, output inside a wider NaN buffer, all of
