@@ -1,4 +1,4 @@
-"""The producer / consumer kernel (kernels_mid.hip): every tile at its edges, rows that start anywhere in a 128-byte line, K
+"""The producer / consumer kernel (mid_kernel.h): every tile at its edges, rows that start anywhere in a 128-byte line, K
 tails, K parts, pieces lower than the tile. Against the fp64 oracle under "one rounding of the exact value" (half an ulp of the
 result, twice, plus 1e-3 for fp32 sums in another order), and bit for bit between equal problems that lie differently in memory:
 where a row starts moves its bytes in LDS, not the order of the sums."""
@@ -97,6 +97,40 @@ def test_rings_and_left_out_copies(capi, index):
             assert_one_rounding(P, plain.cpu(), torch.bfloat16, what + " plain")
 
 
+@pytest.mark.parametrize("index", range(N_TILES))
+def test_long_walks_over_k(capi, index):
+    """K of 31 .. 38 lines, where tiles of more than 64 activation rows ask for weight lines in pairs (32 and more), rings are refilled several
+    times and whole lines are copied without bounds checks: line counts of both parities around the bound, with and without a tail; dense rows,
+    rows of whole lines, rows a multiple of 4 KB apart (walks from different lines), rows at every sixteenth of a line. Weight and activation
+    rows that end with the tile, and 8 rows and more before it (waves leave copies out). All tiles of one call and of a call with one row more
+    than the tile. One rounding of the exact value, and where no walk starts elsewhere the same bits however the rows lie."""
+    bp, bq = tile_rows(capi, index)
+    for n, (K, M, ff) in enumerate([(64 * 31, bq, bp // 2), (64 * 32, bq + 1, bp + 3), (64 * 33 - 8, bq - 9, bp // 2 - 4), (64 * 34 - 40, bq, bp),
+                                    (64 * 37, bq - 17, bp // 2 - 8), (64 * 37 - 56, bq + 1, bp // 2 + 1), (64 * 38, bq - 31, bp - 15)]):
+        dtype = torch.float16 if n % 2 else torch.bfloat16
+        g = torch.Generator(device=DEV).manual_seed(100 * index + n)
+        X = torch.randn(M, K, device=DEV, generator=g).to(dtype)
+        W = (torch.randn(2 * ff, K, device=DEV, generator=g) / K ** 0.5).to(dtype)
+        plain = X.double() @ W.double().t()
+        want = (plain[:, 0::2] * torch.nn.functional.silu(plain[:, 1::2])).cpu()
+        plain, first = plain.cpu(), None
+        for pad, xo, wo in ((0, 0, 0), ((-K) % 64 + 64, 0, 0), (-K % 2048, 0, 0), (8 * (1 + index % 7), 8 * (1 + n), 8 * (index % 16))):
+            Xp, Wp = lay(X, pad, xo), lay(W, pad, wo)
+            try:
+                capi.set_variant(0, 200 + index)
+                capi.set_variant(1, 200 + index)
+                H, P = capi.gateup(Xp, Wp), capi.down(Xp, Wp)
+            finally:
+                capi.set_variant(0, -1)
+                capi.set_variant(1, -1)
+            what = "tile %d (%d x %d) %s pad %d" % (index, bp, bq, (M, ff, K), pad)
+            assert_one_rounding(H, want, dtype, what)
+            assert_one_rounding(P, plain, dtype, what + " plain")
+            if M > bq:
+                first = first or (H, P)
+                assert torch.equal(H, first[0]) and torch.equal(P, first[1]), what
+
+
 @pytest.mark.parametrize("M", [1, 8, 17, 33, 100, 200, 300])
 @pytest.mark.parametrize("D,FF", [(1096, 8008), (1024, 16384), (3000, 4872)])
 def test_down_projection_in_parts_of_k(capi, M, D, FF):
@@ -143,7 +177,7 @@ def test_workgroups_start_their_walk_over_k_at_different_lines(capi, tile, M, K,
 @pytest.mark.parametrize("M,D,FF", [(656, 2048, 8192), (999, 1530, 6144), (257, 3072, 12288), (259, 3070, 12288)])
 def test_down_projection_of_more_rows_on_narrow_outputs(capi, M, D, FF):
     """Rows past 256 whose parts the 256-row kernel took: H and W2 in rows of whole lines beside NaN, output inside a wider NaN buffer, all of
-    the scratch and the least that is accepted with a guard behind it; against float64 and against the 256-row kernel."""
+    the scratch with a guard behind it, less of it refused; against float64 and against the 256-row kernel."""
     L = capi.lib()
     assert capi.variant_name(1, 0, M, D, FF).startswith("splitk_pair16") and capi.variant_name(4, 0, M, D, FF).startswith("mid_")
     H = (torch.randn(M, FF, device=DEV) * 0.3).to(torch.bfloat16)
@@ -167,6 +201,24 @@ def test_down_projection_of_more_rows_on_narrow_outputs(capi, M, D, FF):
         capi.set_variant(1, -1)
     # either is one rounding of a sum off by fp32 noise: they differ by an ulp where the sum lies next to a tie
     assert ((wide[:, :D].float() - large.float()).abs() <= large.float().abs() * 2.0 ** -7 + 1e-3).all()
+
+
+@pytest.mark.parametrize("M,D,FF", [(656, 2048, 8192), (300, 2048, 4096), (259, 3070, 12288)])
+@pytest.mark.parametrize("h_pad,w_pad,offset", [(8, 24, 0), (64, 64, 8), (0, 40, 24)])
+def test_down_projection_on_narrow_outputs_of_rows_that_are_no_whole_lines(capi, M, D, FF, h_pad, w_pad, offset):
+    """K of whole lines, which the plan of the scratch goes by, in rows that start anywhere in a line, which the launch goes by: beside NaN,
+    exactly the scratch that was asked for with a guard behind it, against float64."""
+    L = capi.lib()
+    H = (torch.randn(M, FF, device=DEV) * 0.3).to(torch.bfloat16)
+    W2 = (torch.randn(D, FF, device=DEV) / FF ** 0.5).to(torch.bfloat16)
+    Hp, Wp = lay(H, h_pad, offset), lay(W2, w_pad, offset)
+    nbytes = L.fsw_down_workspace_bytes(0, M, D, FF)
+    ws = torch.full((nbytes + 256,), 7, dtype=torch.uint8, device=DEV)
+    wide = torch.full((M, D + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert L.fsw_down(0, M, D, FF, Hp.data_ptr(), Hp.stride(0), Wp.data_ptr(), Wp.stride(0), wide.data_ptr(), D + 8, ws.data_ptr(), nbytes,
+                      torch.cuda.current_stream().cuda_stream) == capi.OK
+    assert (ws[nbytes:] == 7).all() and torch.isnan(wide[:, D:]).all()
+    assert_one_rounding(wide[:, :D], (H.double() @ W2.double().t()).cpu(), torch.bfloat16, "parts")
 
 
 def test_down_projection_of_few_rows_runs_without_scratch(capi):
