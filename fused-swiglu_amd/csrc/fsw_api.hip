@@ -501,11 +501,16 @@ static DownPlan down_plan(int64_t M, int64_t D, int64_t FF, size_t limit, bool r
   if (r.plan.splits > most) r.plan.splits = most < 1 ? 1 : (int)most;
   r.mid = r.plan.splits > 1 ? r.plan.tile <= 130 : dma_variant(v);
   // The same parts or fewer on whichever kernel takes them faster by the estimates. Outputs of up to 3072 features, whole lines: mid_kernel's
-  // is 8 % high where the 256-row kernel's is right, but for tiles of 224 and 256 activation rows (3 lines in a ring). Down, us, 256-row
-  // kernel -> mid_kernel: 8192 -> 2048 333 rows 30.3 -> 24.3, 656 rows 41.8 -> 35.9, 700 rows 39.3 -> 34.3, 768 rows 45.3 -> 39.2. Wider
-  // ones are level within what one call differs from run to run (11008 -> 4096 359 rows 52 and 57, 384 rows 48.5 and 45.0; 14336 -> 4096 333
-  // rows 55.7 and 52.2, the forward 135 either way). Other rows: 8008 -> 3000 300 rows 39.6 -> 28.8, 900 rows 62.9 -> 58.8; 23568 -> 6168
-  // 499 rows stays, 152 and 189.
+  // is 8 % high where the 256-row kernel's is right. Down, us, 256-row kernel -> mid_kernel: 8192 -> 2048 656 rows 41.8 -> 35.9, 700 rows
+  // 39.3 -> 34.3, 768 rows 45.3 -> 39.2; 9792 -> 2776 328 rows 34.1 -> 31.0; 12288 -> 3064 295 rows 39.0 -> 34.2; 25 problems of 1024 .. 2304
+  // features 0.91 (worst 1.025), 25 of 2304 .. 3072 0.91 (worst 0.98). Left out are tiles of 224 and 256 activation rows, which the estimate
+  // does not tell apart there: 20 problems that would take 96 x 224 0.94 (0.86 .. 1.03). Wider outputs are level within what one call differs
+  // from run to run (11008 -> 4096 359 rows 52 and 57, 384 rows 48.5 and 45.0; 14336 -> 4096 333 rows 55.7 and 52.2, the forward 135 either
+  // way). The plan is that of dense rows, as the scratch is: K of whole lines in rows that are none gains more, as the 256-row kernel fetches
+  // their lines twice (20 problems, rows 8 elements longer: 0.76, 0.67 .. 0.82). Fewer parts are longer chains of sums in fp32: 6144 -> 1536
+  // 1024 rows in two parts where six were, 3.3e-4 of the bf16 results are not the nearest to the exact one, 2.4e-4 before (fp16 2.2e-3 and
+  // 1.6e-3), and the error of the result is the same to five digits (1.6539e-3, fp16 2.0704e-4).
+  // Other rows: 8008 -> 3000 300 rows 39.6 -> 28.8, 900 rows 62.9 -> 58.8; 23568 -> 6168 499 rows stays, 152 and 189.
   if (!r.mid && r.plan.splits > 1 && M <= 1024) {
     const bool narrow = !rag && D <= 3072;
     const fsw::MidPlan p = fsw::mid_plan(false, (int)D, (int)M, (int)FF, rag, 0, r.plan.splits);

@@ -23,11 +23,14 @@ const TileSet kNarrower = [] {
   return s;
 }();
 
-// Estimated time, us, of one launch (and the summing kernel of a split one): fitted to 2300 timings of 230 problems (gate/up and
-// down, 1 .. 900 rows, d 1024 .. 8192, aligned and ragged rows, weights from memory), 4 % rms; the tile it picks is 1.3 % slower
-// than the best of them on average. A K tile of 64 costs the copies of its weight and activation rows (0.00256 us = 128 bytes at
-// 50 bytes per ns) or the LDS reads and MFMAs, whichever is more, plus a part of the other; a part that fills the chip shares
-// HBM; a second round overlaps with the first where it is partly filled.
+// Estimated time, us, of one launch (and the summing kernel of a split one). The coefficients were fitted to 2300 timings of 230 problems
+// (gate/up and down, 1 .. 900 rows, d 1024 .. 8192, aligned and ragged rows, weights from memory) while weight and activation lines shared a
+// ring and were asked for in turn. For the kernel as it is: 4.9 % rms and no bias over 1039 chosen plans of up to 1100 rows, worst where they
+// hold 129 .. 256 rows of a down projection (aligned 13 % rms, 8 % too low on average) or more than 256 (5 and 8 % too high, aligned and
+// ragged); the gate/up tile it picks is 1.0 % slower than the best whole one on average (110 problems of 20 .. 700 rows; worst 1.155: 7392 x
+// 1472 208 rows 13.5 on 64 x 128, 11.7 on 96 x 96). It knows neither the depth of the rings nor pairs. A K tile of 64 costs the copies of its
+// weight and activation rows (0.00256 us = 128 bytes at 50 bytes per ns, which 0.672 and 0.464 scale) or the LDS reads and MFMAs, whichever
+// is more, plus a part of the other; a part that fills the chip shares HBM; a second round overlaps with the first where it is partly filled.
 double mid_time(int np, int nq, int k, bool ragged, const MidTile& t, int step, int splits) {
   const int tq = (nq + 32 * t.fq - 1) / (32 * t.fq);
   const long long tp = (np + step - 1) / step;

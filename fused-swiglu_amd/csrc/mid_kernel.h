@@ -240,9 +240,11 @@ mid_kernel(const GemmArgs a, const int tiles_p, const int tiles_q, const int gro
       else produce(integral_constant<int, LP - 1>{}, integral_constant<int, LQ - 1>{}, g);
     };
     // Two weight lines at once where the tile says so and there are enough to fill the rings a few times (11008 -> 4096 in parts of 22 lines,
-    // 75 rows 25.4 us with pairs 26.2, 149 rows 30.6 and 31.9; 8008 -> 3000 in parts of 32, 200 rows 26.0 and 24.4). Not on rings of four weight
-    // lines with rows that are no whole lines: the step before needs the second pair's first line then, one step after it was asked for
-    // (40736 x 6928, 349 rows 229 and 271).
+    // 75 rows 25.4 us with pairs 26.2, 149 rows 30.6 and 31.9; 8008 -> 3000 in parts of 32, 200 rows 26.0 and 24.4). 22 .. 31 lines, line by
+    // line -> pairs: tiles of 128 and more activation rows 0.94 (25 problems, 0.87 .. 1.00; gate/up 16336 x 1520 176 rows 19.4 -> 16.9), of 96
+    // 1.01 (19, 0.95 .. 1.04; 31696 x 1976 87 rows 25.5 -> 26.6): one bound for both lies on the safe side. A launch whose last part of K is
+    // the only one below it runs that part line by line. Not on rings of four weight lines with rows that are no whole lines: the step before
+    // needs the second pair's first line then, one step after it was asked for (40736 x 6928, 349 rows 229 and 271).
     if constexpr (PAIRS == 2) {
       if (nkt >= 32 && (NW > 4 || !ph)) rows(integral_constant<int, 2>{});
       else rows(integral_constant<int, 1>{});
